@@ -110,8 +110,11 @@ __device__ void finalize_body(const View &d, const Acc &A, int g, v3 da, v3 dq) 
 // Field of non-point item `row` at partner jl of its system, per unit GM of
 // the item's body (k_np_field; also run by extra workgroups of the deform
 // launches, since it needs only the stage's positions and frames).
-__device__ __forceinline__ void np_field_one(const View &d, const Acc &A, int row, int jl) {
-    const NPItem it = d.items[row];
+// Rows past the thread-pool-order items (row >= nrows) are the models of the
+// single-thread-order systems (View::sitems, written to View::san).
+__device__ __forceinline__ void np_field_one(const View &d, const Acc &A, int row, int jl, int nrows) {
+    const bool serial = row >= nrows;
+    const NPItem it = serial ? d.sitems[row - nrows] : d.items[row];
     const SysMeta sm = d.sys[it.sys];
     if (jl >= sm.n) return;
     const int gj = sm.off + jl;
@@ -120,7 +123,7 @@ __device__ __forceinline__ void np_field_one(const View &d, const Acc &A, int ro
         const v3 r = diff(A.lddv(F_R, gj), A.lddv(F_R, it.body));
         an = nonpoint_field_inl(d, A, it.body, it.kind, it.model, r);
     }
-    double *o = d.an + 3 * ((int64_t)it.an_off + jl);
+    double *o = (serial ? d.san : d.an) + 3 * ((int64_t)it.an_off + jl);
     o[0] = an.x; o[1] = an.y; o[2] = an.z;
 }
 
@@ -128,13 +131,13 @@ __device__ __forceinline__ void np_field_one(const View &d, const Acc &A, int ro
 // deform workgroups covers 64 partners of one item row.  Units are taken
 // chunk-major, so the chunks of one row (a ring's are costly) run in
 // different workgroups and on different CUs.
-struct NpTail { int ndef, nrows, chunks; };           // chunks of 64 partners per row
+struct NpTail { int ndef, nrows, chunks, npool; };    // rows (npool of them thread-pool-order items), chunks of 64 partners per row
 __device__ __forceinline__ bool np_tail(const View &d, const NpTail &np) {
     if ((int)blockIdx.x < np.ndef) return false;
     if (np.nrows <= 0) return true;
     const int u = ((int)blockIdx.x - np.ndef) * ((int)blockDim.x >> 6) + ((int)threadIdx.x >> 6);
     const int c = u / np.nrows, row = u - c * np.nrows;
-    if (c < np.chunks) np_field_one(d, Acc{d.F, d.nbp}, row, c * 64 + ((int)threadIdx.x & 63));
+    if (c < np.chunks) np_field_one(d, Acc{d.F, d.nbp}, row, c * 64 + ((int)threadIdx.x & 63), np.npool);
     return true;
 }
 
@@ -1406,15 +1409,184 @@ __global__ __launch_bounds__(BS) void k_main_serial(View d, const int2 *__restri
     finalize_body(d, A, gi, da, dq);
 }
 
+// The same sums with one workgroup of W wavefronts per body.  The body's
+// partners are walked as a sequence of 64-partner tiles in the order of the
+// sequential loop: the reactions of the partners below i, the own loop over
+// every partner, the reactions of the partners above i (a tile that i splits
+// appears on both sides).  Each wavefront evaluates one tile per round, one
+// partner per lane, and leaves the non-zero terms as six-value entries
+// (daccel, dtorque) in LDS, compacted in partner and slot order as in
+// k_main_wpb; lanes 0-5 of wave 0 then add the entries of the round's tiles
+// and wave 1 the G rows of its own-loop tiles.  A reaction entry holds +0 for
+// dtorque, an exact identity in a sum that starts at +0.
+// Own-loop slots: GM dg, -LT (own spin), +LT (partner's spin), radiation,
+// -GM field_gp, -GM field_ring; reaction slots: -GM_p dg_p, +GM_p field_gp,
+// +GM_p field_ring.
+// One thread per body (k_main_serial) walks 3 n partners in one lane and
+// leaves most of the GPU idle; here the terms are formed in parallel and the
+// dependent additions of the non-zero entries are what is left.  504 bodies:
+// 1033 us per launch one thread per body, here together with the deformation
+// and the stage update 65 us per stage (28.2 -> 1.64 ms per RK12 step); 40
+// bodies with models 7.4 -> 0.85 ms per step against the persistent workgroup.
+constexpr int kSerSlots = 6;
+constexpr int kSerEntMax = 64 * kSerSlots;           // a multiple of 16: the padding fits too
+constexpr int kSerTile = 3 * kWpbPitch + kWpbEnt * kSerEntMax;
+
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *__restrict__ work) {
+    const Acc A{d.F, d.nbp};
+    const int s = work[blockIdx.x].x, il = work[blockIdx.x].y;
+    const SysMeta sm = d.sys[s];
+    const int n = sm.n, off = sm.off, gi = off + il;
+    const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+    __shared__ double term[W * kSerTile];
+    __shared__ int count[W];
+    __shared__ double wmax[2 * W];
+    __shared__ double gsum[3];
+    const IMain I = load_imain(A, gi);
+    const v3 naccc = A.ldv(F_NACCC, gi);
+    double mind0 = 0, maxi0 = 0;
+    if (wv == 0) { mind0 = A.ld(F_MIND, gi); maxi0 = A.ld(F_MAXI, gi); }
+    const int row_gp = d.san ? d.srow_gp[gi] : -1, row_ring = d.san ? d.srow_ring[gi] : -1;
+    const int ring_i = d.np_ring[gi];
+    double *myg = term + wv * kSerTile, *mye = myg + 3 * kWpbPitch;
+    constexpr int kGWave = W > 1 ? 1 : 0;
+    double acc = 0, gacc = 0, mind = 0, maxi = 0;
+    const int tiles = (n + 63) / 64;
+    const int below = (il + 63) / 64, above0 = (il + 1) / 64;
+    const int own_end = below + tiles;
+    const int total_v = own_end + (il + 1 < n ? tiles - above0 : 0);
+    for (int v0 = 0; v0 < total_v; v0 += W) {
+        const int v = v0 + wv;
+        const int kind = v < below ? 0 : v < own_end ? 1 : 2;
+        const int jl = 64 * (kind == 0 ? v : kind == 1 ? v - below : above0 + v - own_end) + lane;
+        const bool live = v < total_v && jl < n;
+        unsigned keep = 0;
+        v3 e[2 * kSerSlots];
+#pragma unroll
+        for (int k = 0; k < 2 * kSerSlots; ++k) e[k] = v3{0, 0, 0};
+        v3 G{0, 0, 0};
+        if (kind == 1) {
+            if (live && jl != il) {
+                JMain T;
+                load_jmain(A, T, off + jl);
+                const PairGeo p = relativity(I, T, G);
+                mind = checked_max_into(mind, p.rr);
+                maxi = checked_max_into(maxi, p.tp_dg);
+                const v3 dg = (p.rr3 * p.rr2 * I.R2) * quad_field(I.C, p);
+                e[0] = T.GM * dg;
+                e[1] = T.GM * cross(p.r, dg);
+                const double rcr32 = 2 * T.GM / kC * p.rr3;
+                const v3 GLb = cross(I.GL, p.b);
+                e[2] = -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r));
+                e[3] = -(rcr32 * cross(I.GL, cross(p.r, p.b)));
+                const v3 GLj{T.GLx, T.GLy, T.GLz};
+                e[4] = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
+                e[6] = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
+                if (row_gp >= 0) {
+                    const v3 an = san_at(d, row_gp, jl);
+                    e[8] = -(T.GM * an);
+                    e[9] = -(T.GM * cross(p.r, an));
+                }
+                if (row_ring >= 0) {
+                    const v3 an = san_at(d, row_ring, jl);
+                    e[10] = -(T.GM * an);
+                    e[11] = -(T.GM * cross(p.r, an));
+                }
+            }
+        } else if (live && (kind == 0 ? jl < il : jl > il)) {
+            const int gp_ = off + jl;
+            const m3 Cp = A.ldm(F_CPOT, gp_);
+            const double R2p = A.ld(F_R2, gp_), GMp = A.ld(F_GM, gp_);
+            const int rg = d.san ? d.srow_gp[gp_] : -1, rr_ = d.san ? d.srow_ring[gp_] : -1;
+            const double *c = &Cp.x.x;
+            bool quad = false;
+#pragma unroll
+            for (int q = 0; q < 9; ++q) quad = quad || c[q] != 0;
+            if (quad && R2p != 0) {                        // outer body p visiting partner i: r = r_i - r_p
+                PairGeo p;
+                p.r = diff(I.r, A.lddv(F_R, gp_));
+                p.rr2 = 1 / smax(dot(p.r, p.r), A.ld(F_SR2, gp_) + I.sR2);
+                p.rr = sqrt(p.rr2);
+                p.rr3 = p.rr * p.rr2;
+                e[0] = -(GMp * ((p.rr3 * p.rr2 * R2p) * quad_field(Cp, p)));
+            }
+            if (rg >= 0) e[2] = GMp * san_at(d, rg, il);
+            if (rr_ >= 0) e[4] = GMp * san_at(d, rr_, il);
+        }
+        auto nz = [](const v3 &a) { return a.x != 0 || a.y != 0 || a.z != 0; };
+#pragma unroll
+        for (int k = 0; k < kSerSlots; ++k)
+            if (nz(e[2 * k]) || nz(e[2 * k + 1])) keep |= 1u << k;
+        myg[lane] = G.x; myg[kWpbPitch + lane] = G.y; myg[2 * kWpbPitch + lane] = G.z;
+        int pos = 0, total = 0;
+#pragma unroll
+        for (int k = 0; k < kSerSlots; ++k) {
+            const uint64_t b = __ballot((keep >> k) & 1u);
+            pos += __popcll(b & ((1ull << lane) - 1));
+            total += __popcll(b);
+        }
+#pragma unroll
+        for (int k = 0; k < kSerSlots; ++k)
+            if ((keep >> k) & 1u) {
+                double *o = mye + kWpbEnt * pos++;
+                o[0] = e[2 * k].x; o[1] = e[2 * k].y; o[2] = e[2 * k].z;
+                o[3] = e[2 * k + 1].x; o[4] = e[2 * k + 1].y; o[5] = e[2 * k + 1].z;
+            }
+        const int padded = (total + 15) & ~15;
+        if (lane < padded - total) {
+            double *o = mye + kWpbEnt * (total + lane);
+#pragma unroll
+            for (int c = 0; c < kWpbEnt; ++c) o[c] = 0.0;
+        }
+        if (lane == 0) count[wv] = padded;
+        __syncthreads();
+        if (wv == 0 && lane < 6) {
+            for (int u = 0; u < W; ++u)
+                chain_add_strided<kWpbEnt>(term + u * kSerTile + 3 * kWpbPitch + lane,
+                                           __builtin_amdgcn_readfirstlane(count[u]), acc);
+        }
+        if (wv == kGWave && lane < 3) {
+            for (int u = max(0, below - v0); u < min(W, own_end - v0); ++u)
+                chain_add64(term + u * kSerTile + lane * kWpbPitch, gacc);
+        }
+        __syncthreads();
+    }
+    if (wv == kGWave && lane < 3) gsum[lane] = gacc;
+    mind = wave_checked_max(mind);
+    maxi = wave_checked_max(maxi);
+    if (lane == 0) { wmax[wv] = mind; wmax[W + wv] = maxi; }
+    __syncthreads();
+    if (wv != 0) return;
+    double v6[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v6[k] = __shfl(acc, k, 64);
+    if (lane != 0) return;
+    for (int u = 0; u < W; ++u) {
+        mind0 = checked_max_into(mind0, wmax[u]);
+        maxi0 = checked_max_into(maxi0, wmax[W + u]);
+    }
+    const v3 ga{gsum[0], gsum[1], gsum[2]}, nacc = naccc * kC2;
+    v3 da{v6[0], v6[1], v6[2]}, dq{v6[3], v6[4], v6[5]};
+    A.stv(F_GACC, gi, ga);
+    A.st(F_MIND, gi, mind0);
+    A.st(F_MAXI, gi, maxi0);
+    A.st(F_PHI, gi, I.phi * kC2);                          // FINALIZE_RELATIVITY
+    A.stv(F_NACC, gi, nacc);
+    if (ring_i >= 0) ring_correction(d.rings[ring_i], I.R2, I.GL, ga, nacc, da, dq);
+    A.stv(F_DACC, gi, da);
+    A.stv(F_DTQ, gi, dq);
+}
+
 // ---------------------------------------------------------------------------
 // non-point items, thread-pool order (mass.cpp:158-214, 253-307)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_np_field(View d, int nrows) {
+__global__ __launch_bounds__(64) void k_np_field(View d, int nrows, int npool) {
     // one thread per (item, partner): an = field of the item at r_j - r_p
     const Acc A{d.F, d.nbp};
     const int row = blockIdx.y;
     if (row >= nrows) return;
-    np_field_one(d, A, row, blockIdx.x * blockDim.x + threadIdx.x);
+    np_field_one(d, A, row, blockIdx.x * blockDim.x + threadIdx.x, npool);
 }
 
 // one wavefront per (item, round k): the item's partial sums over the slice
@@ -2316,8 +2488,8 @@ void set_rk_table(const double *tab650, hipStream_t st) {
 }
 
 void launch_deform_mixed(const View &d, const int2 *work, int nwork, const int4 *blk16, int nblk, int prepare,
-                         int np_rows, int max_n, hipStream_t st) {
-    const NpTail np{nwork + nblk, np_rows, (max_n + 63) / 64};
+                         int np_rows, int np_pool, int max_n, hipStream_t st) {
+    const NpTail np{nwork + nblk, np_rows, (max_n + 63) / 64, np_pool};
     const int grid = nwork + nblk + np_rows * np.chunks;
     if (grid) hipLaunchKernelGGL(k_deform_mixed, dim3(grid), dim3(64), 0, st, d, work, nwork, blk16, prepare, np);
 }
@@ -2357,13 +2529,13 @@ void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool
 // wavefront per body).  Four, not eight, for a 504-body system: two 256-lane
 // workgroups then share each CU, one round of workgroups instead of two
 // (31 us instead of 43-58 us per launch on one MI355X).
-void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, int np_rows, int waves,
-                       hipStream_t st) {
+void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, int np_rows, int np_pool,
+                       int waves, hipStream_t st) {
     if (!nwork && !np_rows) return;
     const int chunks = (max_n + 63) / 64;
     int W = waves;
     if (W == 0) W = (chunks >= 4 && nwork <= 1280) ? 4 : (chunks >= 2 && nwork <= 2816) ? 2 : 1;
-    const NpTail np{nwork, np_rows, (max_n + 63) / 64};
+    const NpTail np{nwork, np_rows, (max_n + 63) / 64, np_pool};
     const dim3 grid(nwork + (np_rows * np.chunks + W - 1) / W), block(64 * W);
     if (np_rows) {
         if (W == 4) hipLaunchKernelGGL((k_deform_wpb<4, true>), grid, block, 0, st, d, work, prepare, np);
@@ -2378,13 +2550,23 @@ void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, in
 void launch_main_serial(const View &d, const int2 *blk, int nblk, hipStream_t st) {
     if (nblk) hipLaunchKernelGGL(k_main_serial<kBS>, dim3(nblk), dim3(kBS), 0, st, d, blk);
 }
-void launch_np_field(const View &d, int nrows, int max_n, hipStream_t st) {
-    if (nrows) hipLaunchKernelGGL(k_np_field, dim3((max_n + 63) / 64, nrows), dim3(64), 0, st, d, nrows);
+// Wavefronts per body of the single-thread order: a system of up to 64 bodies
+// has at most three tiles per body, one round of four wavefronts; several
+// wavefronts only while every workgroup is resident at once (84 KB of LDS
+// with four, two workgroups per CU).
+void launch_main_serial_wpb(const View &d, const int2 *work, int nwork, hipStream_t st) {
+    if (!nwork) return;
+    if (nwork <= 1024) hipLaunchKernelGGL(k_main_serial_wpb<4>, dim3(nwork), dim3(256), 0, st, d, work);
+    else if (nwork <= 2048) hipLaunchKernelGGL(k_main_serial_wpb<2>, dim3(nwork), dim3(128), 0, st, d, work);
+    else hipLaunchKernelGGL(k_main_serial_wpb<1>, dim3(nwork), dim3(64), 0, st, d, work);
+}
+void launch_np_field(const View &d, int nrows, int np_pool, int max_n, hipStream_t st) {
+    if (nrows) hipLaunchKernelGGL(k_np_field, dim3((max_n + 63) / 64, nrows), dim3(64), 0, st, d, nrows, np_pool);
 }
 void launch_np(const View &d, int nrows, int max_n, int maxT, const int2 *recv_blk, int nrecv, bool with_field,
                hipStream_t st, bool with_item) {
     if (!nrows) return;
-    if (with_field) hipLaunchKernelGGL(k_np_field, dim3((max_n + 63) / 64, nrows), dim3(64), 0, st, d, nrows);
+    if (with_field) launch_np_field(d, nrows, nrows, max_n, st);
     if (with_item) hipLaunchKernelGGL(k_np_item, dim3(nrows * maxT), dim3(64), 0, st, d, nrows, maxT);
     if (nrecv) hipLaunchKernelGGL(k_np_recv, dim3(nrecv), dim3(kBS), 0, st, d, recv_blk, maxT);
 }

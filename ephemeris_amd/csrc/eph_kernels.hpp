@@ -54,7 +54,8 @@ struct View {
     // ring at every partner of its system, formed before the main force
     // (rows of 3 doubles per partner; -1: the body has no such model), or null
     const int32_t *srow_gp, *srow_ring;
-    const double *san;
+    double *san;
+    const NPItem *sitems;        // the models behind the rows, in row order
 };
 
 void set_rk_table(const double *tab650, hipStream_t st);
@@ -66,13 +67,15 @@ void launch_main_pool(const View &d, const int2 *blk, int nblk, hipStream_t st);
 // (system, first slot, count <= 16, 0) in the class-sorted slots) in one
 // launch, with the item fields
 void launch_deform_mixed(const View &d, const int2 *work, int nwork, const int4 *blk16, int nblk, int prepare,
-                         int np_rows, int max_n, hipStream_t st);
+                         int np_rows, int np_pool, int max_n, hipStream_t st);
 // four lanes per body; blk16 = (system, first body) of every 16 bodies
 void launch_main_k4(const View &d, const int2 *blk16, int nblk, hipStream_t st);
 // the same with the items' partial sums of launch_np (rows, rounds) in extra
 // workgroups of the launch
 void launch_main_k4_items(const View &d, const int2 *blk16, int nblk, int nrows, int maxT, hipStream_t st);
 void launch_main_serial(const View &d, const int2 *blk, int nblk, hipStream_t st);
+// single-thread order with one workgroup per body; work = {system, body}
+void launch_main_serial_wpb(const View &d, const int2 *work, int nwork, hipStream_t st);
 // latency path, one workgroup of 1-4 wavefronts per body; work = {system,
 // body index in system}
 // fused_np: the receiver and own-item sums of the non-point pass run inside
@@ -82,15 +85,16 @@ void launch_main_serial(const View &d, const int2 *blk, int nblk, hipStream_t st
 // waves: wavefronts per body, 0 = chosen from the batch's shape, else 1, 2 or
 // 4 (the fused kernel has at least 2)
 void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool fused_np, int waves, hipStream_t st);
-void launch_np_field(const View &d, int nrows, int max_n, hipStream_t st);
+void launch_np_field(const View &d, int nrows, int np_pool, int max_n, hipStream_t st);
 constexpr int kNpFusedMaxN_h = 512, kNpFusedMaxItems_h = 64;
 // one workgroup of up to 4 wavefronts per body (partner chunks evaluated in
 // parallel, summed in order); max_n = largest system of the batch
 // np_rows > 0: the launch also evaluates the non-point item fields
-// (launch_np_field) in extra workgroups
+// (launch_np_field) in extra workgroups: np_pool thread-pool-order items, then
+// the models of the single-thread-order systems
 // (waves as for launch_main_wpb)
-void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, int np_rows, int waves,
-                       hipStream_t st);
+void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, int np_rows, int np_pool,
+                       int waves, hipStream_t st);
 // with_item = false: the items' partial sums were formed already
 // (launch_main_k4_items)
 void launch_np(const View &d, int nrows, int max_n, int maxT, const int2 *recv_blk, int nrecv, bool with_field,

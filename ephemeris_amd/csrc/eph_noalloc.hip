@@ -226,7 +226,8 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
     v.perm = nullptr;                                     // (read only by the four-lane and one-thread-per-body deform kernels)
     v.srow_gp = dp->srow_gp;
     v.srow_ring = dp->srow_ring;
-    v.san = n_sitems ? (const double *)(base + kOffAn) : nullptr;      // rows of at most 64 models x n partners
+    v.san = n_sitems ? (double *)(base + kOffAn) : nullptr;            // rows of at most 64 models x n partners
+    v.sitems = dp->sitems;
     v.an = (double *)(base + kOffAn);
     v.part = (double *)(base + kOffPart);
     v.t0 = &dp->t0;
@@ -235,16 +236,10 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
     // the kernels of the resident path for a batch of one system: one
     // workgroup per body (the item fields in extra workgroups of the deform
     // launch), then the main force in the order asked for and the non-point pass
-    const int rows = serial ? 0 : (int)nnp;
-    launch_deform_wpb(v, dp->work, (int)n, (int)n, 1, rows, 0, st);
+    const int rows = serial ? n_sitems : (int)nnp, pool_rows = serial ? 0 : (int)nnp;
+    launch_deform_wpb(v, dp->work, (int)n, (int)n, 1, rows, pool_rows, 0, st);
     if (serial) {
-        if (n_sitems) {
-            View vs = v;
-            vs.items = dp->sitems;
-            vs.an = (double *)(base + kOffAn);
-            launch_np_field(vs, n_sitems, (int)n, st);
-        }
-        launch_main_serial(v, dp->blk_main, n_main, st);
+        launch_main_serial_wpb(v, dp->work, (int)n, st);
     } else {
         launch_main_wpb(v, dp->work, (int)n, (int)n, false, 0, st);
         if (nnp) launch_np(v, (int)nnp, (int)n, maxT, dp->blk_recv, n_recv, false, st);

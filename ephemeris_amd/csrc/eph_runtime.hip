@@ -196,7 +196,7 @@ int Batch::build_plan(int mode) {
     Plan &pl = plan[mode];
     std::vector<SysMeta> meta(n_sys);
     std::vector<NPItem> items;
-    std::vector<int2> blk_pool, blk_serial, blk_recv, work_pool;
+    std::vector<int2> blk_pool, blk_serial, blk_recv, work_pool, work_serial;
     int64_t an_rows = 0;
     std::vector<NPItem> sitems;
     std::vector<int32_t> srow_gp, srow_ring;
@@ -219,6 +219,7 @@ int Batch::build_plan(int mode) {
         m.serial = (mode == 1 || n_task <= 1) ? 1 : 0;
         if (m.serial) {
             append_blocks(blk_serial, (int)s, (int)n);
+            for (int64_t i = 0; i < n; ++i) work_serial.push_back(make_int2((int)s, (int)i));
             // each model's field at every partner, formed in parallel before
             // the main force (the single-thread kernel reads it per partner)
             for (int64_t i = 0; i < n; ++i) {
@@ -284,6 +285,8 @@ int Batch::build_plan(int mode) {
     if ((rc = dev_upload(*this, pl.d_blk_recv, blk_recv))) return rc;
     if ((rc = dev_upload(*this, pl.d_work_pool, work_pool))) return rc;
     pl.n_work_pool = (int)work_pool.size();
+    if ((rc = dev_upload(*this, pl.d_work_serial, work_serial))) return rc;
+    pl.n_work_serial = (int)work_serial.size();
     pl.n_pool = (int)blk_pool.size();
     pl.n_serial = (int)blk_serial.size();
     pl.n_recv = (int)blk_recv.size();
@@ -323,6 +326,7 @@ View Batch::view(int mode) const {
     v.srow_gp = pl.d_srow_gp;
     v.srow_ring = pl.d_srow_ring;
     v.san = pl.d_san;
+    v.sitems = pl.d_sitems;
     v.an = pl.d_an;
     v.part = pl.d_part;
     v.t0 = d_t0;
@@ -330,14 +334,17 @@ View Batch::view(int mode) const {
 }
 
 // The wave-per-body kernels win while the batch is too small to fill the
-// GPU with one thread per body (fewer than ~16k bodies in thread-pool order).
+// GPU with one thread per body (fewer than ~16k bodies in thread-pool order,
+// or in single-thread order where no system is in thread-pool order: 504
+// bodies 1033 -> 31 us per main-force launch).
 static constexpr int kWpbAutoBodies = 16384;
 
 bool Batch::use_wpb(int mode) const {
     const int variant = eff_variant();
     if (variant == 1 || variant == 4) return false;
     if (variant >= 2) return true;
-    return plan[mode].n_work_pool > 0 && plan[mode].n_work_pool <= kWpbAutoBodies;
+    const Plan &pl = plan[mode];
+    return pl.n_work_pool > 0 ? pl.n_work_pool <= kWpbAutoBodies : pl.n_work_serial <= kWpbAutoBodies;
 }
 
 int Batch::accel(int mode, bool prepare_only) {
@@ -347,12 +354,14 @@ int Batch::accel(int mode, bool prepare_only) {
     const bool wpb = use_wpb(mode);
     // the non-point item fields depend only on the stage's positions and
     // frames: they ride along in extra workgroups of the deform launch
-    const int np_rows = prepare_only ? 0 : pl.nrows;
+    // (pool items first, then the models of the single-thread-order systems)
+    const int np_rows = prepare_only ? 0 : pl.nrows + pl.n_sitems;
     bool field_done = false;
     {
         Scope sc(profiler, 1, stream);
         if (wpb) {
-            launch_deform_wpb(v, d_work_all, n_work_all, max_sys_n, prepare_only ? 0 : 1, np_rows, eff_waves(), stream);
+            launch_deform_wpb(v, d_work_all, n_work_all, max_sys_n, prepare_only ? 0 : 1, np_rows, pl.nrows, eff_waves(),
+                              stream);
             field_done = true;
         } else if (variant == 1) {
             launch_deform(v, d_blk_light, n_blk_light, d_blk_damped, n_blk_damped, prepare_only ? 0 : 1, stream);
@@ -361,7 +370,7 @@ int Batch::accel(int mode, bool prepare_only) {
             // one wavefront each; the rest four lanes each (that launch
             // carries the item fields)
             launch_deform_mixed(v, d_work_damped, n_work_damped, d_blk_light16, n_blk_light16,
-                                prepare_only ? 0 : 1, np_rows, pl.max_n, stream);
+                                prepare_only ? 0 : 1, np_rows, pl.nrows, pl.max_n, stream);
             field_done = true;
         }
     }
@@ -370,7 +379,7 @@ int Batch::accel(int mode, bool prepare_only) {
     bool items_done = false;
     if (fused_np && pl.nrows && !field_done) {
         Scope sc(profiler, 4, stream);
-        launch_np_field(v, pl.nrows, pl.max_n, stream);
+        launch_np_field(v, pl.nrows, pl.nrows, pl.max_n, stream);
     }
     if (pl.n_pool) {
         Scope sc(profiler, 2, stream);
@@ -383,13 +392,14 @@ int Batch::accel(int mode, bool prepare_only) {
     }
     if (pl.n_serial) {
         Scope sc(profiler, 3, stream);
-        if (pl.n_sitems) {                                 // the models' fields at every partner
+        if (pl.n_sitems && !field_done) {                  // the models' fields at every partner
             View vs = v;
             vs.items = pl.d_sitems;
             vs.an = pl.d_san;
-            launch_np_field(vs, pl.n_sitems, pl.max_n, stream);
+            launch_np_field(vs, pl.n_sitems, pl.n_sitems, pl.max_n, stream);
         }
-        launch_main_serial(v, pl.d_blk_serial, pl.n_serial, stream);
+        if (wpb) launch_main_serial_wpb(v, pl.d_work_serial, pl.n_work_serial, stream);
+        else launch_main_serial(v, pl.d_blk_serial, pl.n_serial, stream);
     }
     if (pl.nrows && !fused_np) {
         Scope sc(profiler, 4, stream);
@@ -415,6 +425,23 @@ DtK stage_dtk() {                                    // RungeKutta.impl:148-152
 bool Batch::all_small() const {
     return plan[0].n_pool == 0 && plan[0].n_serial > 0 &&
            *std::max_element(sys_n.begin(), sys_n.end()) <= kSmallMax;
+}
+
+// Systems of at most kSmallMax bodies, all in single-thread order, can run on
+// one persistent workgroup each or on the launches of the larger systems with
+// one workgroup per body.  The persistent workgroup forms its pairs in rounds
+// and its models' fields inside them, so its stage grows with the system's
+// size and models and not with their number; the launches cost about 27 us a
+// stage and then grow with the bodies.  Measured per stage, persistent
+// against launches: 9 bodies 24 / 27 us, 16 bodies 30 / 28 us, 25 bodies 51 /
+// 27 us, 40 bodies with models 295 / 34 us, 12 with models 70 / 29 us; 25
+// bodies x 64 systems 52 / 49 us, x 128 53 / 63 us; 25 with models x 64 131 /
+// 60 us, x 256 120 / 133 us.
+constexpr int64_t kSmallLaunchBodies = 2048;
+bool Batch::use_small(int mode) const {
+    if (force_generic || !(mode == 1 || plan[0].n_pool == 0) || !all_small()) return false;
+    const bool heavy = max_sys_n > 16 || plan[mode].n_sitems > 0;
+    return !(heavy && nb <= kSmallLaunchBodies);
 }
 
 // One launch runs many steps for every system (one workgroup per system).
@@ -560,8 +587,7 @@ int Batch::autotune(double dt, int mode) {
 
 int Batch::integrate(double dt, int64_t n_step, int mode) {
     if (n_step == 0) return EPH_OK;
-    if ((mode == 1 || plan[0].n_pool == 0) && all_small() && !force_generic)
-        return integrate_small(dt, n_step, nullptr, 0, nullptr, nullptr);
+    if (use_small(mode)) return integrate_small(dt, n_step, nullptr, 0, nullptr, nullptr);
     if (variant == 0 && use_autotune && !tune_done) {
         int rc = autotune(n_step < 0 ? -dt : dt, mode);
         if (rc) return rc;

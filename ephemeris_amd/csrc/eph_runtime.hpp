@@ -52,6 +52,8 @@ struct Plan {
     double *d_an = nullptr, *d_part = nullptr;
     int2 *d_work_pool = nullptr;     // (system, body) of every body of a pool-order system
     int n_work_pool = 0;
+    int2 *d_work_serial = nullptr;   // the same of the single-thread-order systems
+    int n_work_serial = 0;
     bool np_fusable = true;          // every pool system fits the fused non-point pass
     int2 *d_blk16 = nullptr;         // (system, first body) of 16-body blocks, largest systems first
     int n_blk16 = 0;
@@ -123,6 +125,7 @@ struct Batch {
     int integrate_small(double dt, int64_t n_step, JMain *rec, int64_t rec_steps,
                         void (*after_chunk)(void *, int64_t, int64_t), void *ctx);
     bool all_small() const;
+    bool use_small(int mode) const;      // integrate on the persistent path (see its definition)
     std::vector<int> small_ids;
     int *d_small_ids = nullptr;
     int upload(const eph_mass *masses);
