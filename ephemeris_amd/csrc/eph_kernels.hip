@@ -2470,6 +2470,87 @@ void launch_particles(const PView &pv, int n_steps, double dt, const DtK &dtk, h
 }
 
 // ---------------------------------------------------------------------------
+// bodies and particles between the caller's arrays of structs and the
+// field-major state
+// ---------------------------------------------------------------------------
+// Slot q of eph_mass (8 bytes each) holds field c_mass_field[q] of the state;
+// the slots without a field are the id and the model indices.
+constexpr int kMassSlots = (int)(sizeof(eph_mass) / 8);
+constexpr int kSlotSid = (int)(offsetof(eph_mass, sid) / 8), kSlotGp = (int)(offsetof(eph_mass, gp) / 8),
+              kSlotRing = (int)(offsetof(eph_mass, ring) / 8);
+__constant__ int c_mass_field[kMassSlots];
+
+// Sixteen bodies per workgroup meet in LDS, so that both sides are read and
+// written in whole 128-byte pieces; the transposition is bound by memory
+// (73k bodies, 87 MB each way, about 0.05 ms) where the host loop over the
+// fields took 28 ms.  The odd slot count keeps the LDS columns off one bank.
+constexpr int kPackBodies = 16;
+__global__ __launch_bounds__(256) void k_pack_bodies(const double *__restrict__ F, int64_t nbp, int nb,
+                                                     const double *__restrict__ sid, const int32_t *__restrict__ gp,
+                                                     const int32_t *__restrict__ ring, double *__restrict__ out) {
+    __shared__ double t[kPackBodies * kMassSlots];
+    const int g0 = (int)blockIdx.x * kPackBodies, cnt = min(kPackBodies, nb - g0);
+    for (int e = (int)threadIdx.x; e < kPackBodies * kMassSlots; e += 256) {
+        const int q = e / kPackBodies, b = e % kPackBodies, g = g0 + b;
+        if (b >= cnt) continue;
+        const int f = c_mass_field[q];
+        double x;
+        if (f >= 0) x = F[(int64_t)f * nbp + g];
+        else x = q == kSlotSid ? sid[g] : __longlong_as_double((int64_t)(q == kSlotGp ? gp[g] : ring[g]));
+        t[b * kMassSlots + q] = x;
+    }
+    __syncthreads();
+    for (int e = (int)threadIdx.x; e < cnt * kMassSlots; e += 256) out[(int64_t)g0 * kMassSlots + e] = t[e];
+}
+
+__global__ __launch_bounds__(256) void k_unpack_bodies(const double *__restrict__ in, int nb, int64_t nbp,
+                                                       double *__restrict__ F, double *__restrict__ sid) {
+    __shared__ double t[kPackBodies * kMassSlots];
+    const int g0 = (int)blockIdx.x * kPackBodies, cnt = min(kPackBodies, nb - g0);
+    for (int e = (int)threadIdx.x; e < cnt * kMassSlots; e += 256) t[e] = in[(int64_t)g0 * kMassSlots + e];
+    __syncthreads();
+    for (int e = (int)threadIdx.x; e < kPackBodies * kMassSlots; e += 256) {
+        const int q = e / kPackBodies, b = e % kPackBodies, g = g0 + b;
+        if (b >= cnt) continue;
+        const int f = c_mass_field[q];
+        const double x = t[b * kMassSlots + q];
+        if (f >= 0) F[(int64_t)f * nbp + g] = x;
+        else if (q == kSlotSid) sid[g] = x;
+        // phi / c^2 and naccel / c^2, the inputs of the 1PN term
+        if (f == F_PHI) F[(int64_t)F_PHIC * nbp + g] = x / kC2;
+        if (f >= F_NACC && f < F_NACC + 3) F[(int64_t)(F_NACCC + f - F_NACC) * nbp + g] = x * (1 / kC2);
+    }
+}
+
+// particles: r and v as n x 6 (hi, lo), extrema as n x 2; one thread per value
+__global__ void k_pack_particles(const double *__restrict__ P, int64_t npp, int64_t n, double *__restrict__ out) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= 14 * n) return;
+    int64_t p;
+    int row;
+    if (e < 12 * n) {
+        const int64_t q = e < 6 * n ? e : e - 6 * n;
+        p = q / 6;
+        row = (e < 6 * n ? P_R : P_V) + (int)(q - 6 * p);
+    } else {
+        const int64_t q = e - 12 * n;
+        p = q >> 1;
+        row = P_MIND + (int)(q & 1);
+    }
+    out[e] = P[row * npp + p];
+}
+// in: r then v, n x 3 each; every state row is written (lo parts, acceleration
+// and extrema zero, and the columns past the last particle)
+__global__ void k_unpack_particles(const double *__restrict__ in, int64_t n, int64_t npp, double *__restrict__ P) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int row = (int)blockIdx.y;
+    if (p >= npp) return;
+    double x = 0.0;
+    if (p < n && row < P_A && (row & 1) == 0) x = in[(row < P_V ? 0 : 3 * n) + 3 * p + (row % 6) / 2];
+    P[row * npp + p] = x;
+}
+
+// ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
 void set_rk_table(const double *tab650, hipStream_t st) {
@@ -2485,6 +2566,25 @@ void set_rk_table(const double *tab650, hipStream_t st) {
     row0[26] = e;
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_nzj), nzj, sizeof(nzj), 0, hipMemcpyHostToDevice, st);
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_row0), row0, sizeof(row0), 0, hipMemcpyHostToDevice, st);
+}
+
+void set_mass_fields(const int *field_of_slot, hipStream_t st) {
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mass_field), field_of_slot, sizeof(int) * kMassSlots, 0,
+                                 hipMemcpyHostToDevice, st);
+}
+void launch_pack_bodies(const View &d, const uint64_t *sid, eph_mass *out, hipStream_t st) {
+    hipLaunchKernelGGL(k_pack_bodies, dim3((d.nb + kPackBodies - 1) / kPackBodies), dim3(256), 0, st, d.F, d.nbp, d.nb,
+                       (const double *)sid, d.np_gp, d.np_ring, (double *)out);
+}
+void launch_unpack_bodies(const View &d, const eph_mass *in, uint64_t *sid, hipStream_t st) {
+    hipLaunchKernelGGL(k_unpack_bodies, dim3((d.nb + kPackBodies - 1) / kPackBodies), dim3(256), 0, st,
+                       (const double *)in, d.nb, d.nbp, d.F, (double *)sid);
+}
+void launch_pack_particles(const double *P, int64_t npp, int64_t n, double *out, hipStream_t st) {
+    if (n) hipLaunchKernelGGL(k_pack_particles, dim3((unsigned)((14 * n + 255) / 256)), dim3(256), 0, st, P, npp, n, out);
+}
+void launch_unpack_particles(const double *in, int64_t n, int64_t npp, double *P, hipStream_t st) {
+    hipLaunchKernelGGL(k_unpack_particles, dim3((unsigned)((npp + 255) / 256), P_COUNT), dim3(256), 0, st, in, n, npp, P);
 }
 
 void launch_deform_mixed(const View &d, const int2 *work, int nwork, const int4 *blk16, int nblk, int prepare,

@@ -59,6 +59,15 @@ struct View {
 };
 
 void set_rk_table(const double *tab650, hipStream_t st);
+// state field of every 8-byte slot of eph_mass (-1: id and model indices)
+void set_mass_fields(const int *field_of_slot, hipStream_t st);
+// bodies between eph_mass records in device memory and the state; the ids
+// live beside the state
+void launch_pack_bodies(const View &d, const uint64_t *sid, eph_mass *out, hipStream_t st);
+void launch_unpack_bodies(const View &d, const eph_mass *in, uint64_t *sid, hipStream_t st);
+// particle state to r (n x 6), v (n x 6), extrema (n x 2), and from r, v (n x 3 each)
+void launch_pack_particles(const double *P, int64_t npp, int64_t n, double *out, hipStream_t st);
+void launch_unpack_particles(const double *in, int64_t n, int64_t npp, double *P, hipStream_t st);
 void launch_deform(const View &d, const int4 *blk_light, int n_light, const int4 *blk_damped, int n_damped,
                    int prepare, hipStream_t st);
 void launch_main_pool(const View &d, const int2 *blk, int nblk, hipStream_t st);

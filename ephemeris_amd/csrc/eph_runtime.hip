@@ -693,49 +693,44 @@ int Batch::build_class_tables(const eph_mass *masses) {
     return EPH_OK;
 }
 
+// Whether the tidal classes behind the class tables are those of `masses`
+// (the tables and a captured step graph then stand).
+bool Batch::same_classes(const eph_mass *masses) const {
+    if ((int64_t)host_k2.size() != nb) return false;
+    for (int64_t g = 0; g < nb; ++g)
+        if ((host_k2[g] != 0 && host_td[g] != 0) != (masses[g].k2 != 0 && masses[g].tide_delay != 0)) return false;
+    return true;
+}
+
+// The records go to the device as they are and are transposed there.
 int Batch::upload(const eph_mass *masses) {
-    drop_graph();                        // the class tables are rebuilt below
+    const bool keep_tables = same_classes(masses);
     host_k2.resize(nb);
     host_td.resize(nb);
-    for (int64_t g = 0; g < nb; ++g) { host_k2[g] = masses[g].k2; host_td[g] = masses[g].tide_delay; }
-    {
+    sid.resize(nb);
+    for (int64_t g = 0; g < nb; ++g) {
+        host_k2[g] = masses[g].k2;
+        host_td[g] = masses[g].tide_delay;
+        sid[g] = masses[g].sid;
+    }
+    if (!keep_tables) {
+        drop_graph();
         int rc = build_class_tables(masses);
         if (rc) return rc;
     }
-    std::vector<double> buf((size_t)kMassFieldEnd * nbp, 0.0);
-    for (int64_t g = 0; g < nb; ++g) {
-        const char *m = (const char *)&masses[g];
-        for (const auto &f : fields()) {
-            double x;
-            memcpy(&x, m + f.offset, 8);
-            buf[(size_t)f.field * nbp + g] = x;
-        }
-        buf[(size_t)F_PHIC * nbp + g] = masses[g].phi / kC2;
-        buf[(size_t)F_NACCC * nbp + g] = masses[g].naccel.x * (1 / kC2);
-        buf[(size_t)(F_NACCC + 1) * nbp + g] = masses[g].naccel.y * (1 / kC2);
-        buf[(size_t)(F_NACCC + 2) * nbp + g] = masses[g].naccel.z * (1 / kC2);
-    }
-    HIP_CHECK(hipMemcpy(F, buf.data(), sizeof(double) * buf.size(), hipMemcpyHostToDevice));
-    sid.resize(nb);
-    for (int64_t g = 0; g < nb; ++g) sid[g] = masses[g].sid;
+    HIP_CHECK(hipStreamSynchronize(stream));
+    HIP_CHECK(hipMemcpyAsync(d_records(), masses, sizeof(eph_mass) * (size_t)nb, hipMemcpyHostToDevice, stream));
+    launch_unpack_bodies(view(0), d_records(), d_sid, stream);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(stream));
     return EPH_OK;
 }
 
 int Batch::download(eph_mass *masses) {
-    std::vector<double> buf((size_t)kMassFieldEnd * nbp);
+    launch_pack_bodies(view(0), d_sid, d_records(), stream);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpyAsync(masses, d_records(), sizeof(eph_mass) * (size_t)nb, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
-    HIP_CHECK(hipMemcpy(buf.data(), F, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-    for (int64_t g = 0; g < nb; ++g) {
-        char *m = (char *)&masses[g];
-        memset(m, 0, sizeof(eph_mass));
-        for (const auto &f : fields()) {
-            double x = buf[(size_t)f.field * nbp + g];
-            memcpy(m + f.offset, &x, 8);
-        }
-        masses[g].sid = sid[g];
-        masses[g].gp = host_gp_global[g];
-        masses[g].ring = host_ring_global[g];
-    }
     return EPH_OK;
 }
 
@@ -793,6 +788,8 @@ int create_batch(int64_t n_sys, const int64_t *sys_n, const eph_mass *masses,
     if ((rc = dev_upload(*b, b->d_np_gp, b->host_gp))) return bail(rc);
     if ((rc = dev_upload(*b, b->d_np_ring, b->host_ring))) return bail(rc);
     if ((rc = dev_upload(*b, b->d_bsys, bsys))) return bail(rc);
+    b->sid.assign(b->nb, 0);
+    if ((rc = dev_upload(*b, b->d_sid, b->sid))) return bail(rc);
     std::vector<double> t0(n_sys, 0.0);
     if ((rc = dev_upload(*b, b->d_t0, t0))) return bail(rc);
     std::vector<int2> blk_all;
@@ -811,6 +808,12 @@ int create_batch(int64_t n_sys, const int64_t *sys_n, const eph_mass *masses,
     }
     if ((rc = dev_upload(*b, b->d_small_ids, b->small_ids))) return bail(rc);
     set_rk_table(&kRK[0][0], b->stream);
+    static const std::vector<int> slot_field = [] {
+        std::vector<int> v(sizeof(eph_mass) / 8, -1);
+        for (const auto &f : fields()) v[f.offset / 8] = f.field;
+        return v;
+    }();
+    set_mass_fields(slot_field.data(), b->stream);
     if ((rc = b->upload(masses))) return bail(rc);
     if (hipStreamSynchronize(b->stream) != hipSuccess) return bail(fail(EPH_EDEVICE, "stream sync failed"));
     *out = b;
@@ -948,17 +951,18 @@ int create_particles(Batch *field, int64_t n, const double *r, const double *v, 
     if (ps->npp == 0) ps->npp = 256;
     ps->GM = GM;
     ps->R = R;
-    std::vector<double> host((size_t)P_COUNT_HOST * ps->npp, 0.0);
-    for (int64_t i = 0; i < n; ++i)
-        for (int c = 0; c < 3; ++c) {
-            host[(size_t)(2 * c) * ps->npp + i] = r[3 * i + c];
-            host[(size_t)(6 + 2 * c) * ps->npp + i] = v[3 * i + c];
-        }
     auto bail = [&](int code) { delete ps; return code; };
     if (hipMalloc(&ps->P, sizeof(double) * P_ALLOC_ROWS * ps->npp) != hipSuccess)
         return bail(fail(EPH_ENOMEM, "particle state allocation failed"));
-    if (hipMemcpy(ps->P, host.data(), sizeof(double) * host.size(), hipMemcpyHostToDevice) != hipSuccess)
-        return bail(fail(EPH_EDEVICE, "particle upload failed"));
+    {
+        double *in = ps->P + (int64_t)P_COUNT_HOST * ps->npp;    // the scratch rows, not in use yet
+        const size_t bytes = sizeof(double) * 3 * (size_t)n;
+        if (n && (hipMemcpyAsync(in, r, bytes, hipMemcpyHostToDevice, field->stream) != hipSuccess ||
+                  hipMemcpyAsync(in + 3 * n, v, bytes, hipMemcpyHostToDevice, field->stream) != hipSuccess))
+            return bail(fail(EPH_EDEVICE, "particle upload failed"));
+        launch_unpack_particles(in, n, ps->npp, ps->P, field->stream);
+        if (hipStreamSynchronize(field->stream) != hipSuccess) return bail(fail(EPH_EDEVICE, "particle upload failed"));
+    }
     ps->rec_steps = kRecChunk;
     const size_t rec_bytes = 2 * sizeof(JMain) * kSmallMax * (size_t)(25 * kRecChunk);
     if (hipMalloc(&ps->rec, rec_bytes) != hipSuccess) return bail(fail(EPH_ENOMEM, "field record allocation failed"));
@@ -1024,19 +1028,15 @@ int integrate_particles(Particles *ps, double dt, int64_t n_step) {
 }
 
 int download_particles(Particles *ps, double *r, double *v, double *extrema) {
-    std::vector<double> host((size_t)P_COUNT_HOST * ps->npp);
-    HIP_CHECK(hipStreamSynchronize(ps->field->stream));
-    HIP_CHECK(hipMemcpy(host.data(), ps->P, sizeof(double) * host.size(), hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < ps->np; ++i) {
-        for (int c = 0; c < 6; ++c) {
-            if (r) r[6 * i + c] = host[(size_t)c * ps->npp + i];
-            if (v) v[6 * i + c] = host[(size_t)(6 + c) * ps->npp + i];
-        }
-        if (extrema) {
-            extrema[2 * i] = host[(size_t)15 * ps->npp + i];
-            extrema[2 * i + 1] = host[(size_t)16 * ps->npp + i];
-        }
-    }
+    const int64_t n = ps->np;
+    double *out = ps->P + (int64_t)P_COUNT_HOST * ps->npp;       // the scratch rows: free between calls
+    const hipStream_t st = ps->field->stream;
+    launch_pack_particles(ps->P, ps->npp, n, out, st);
+    HIP_CHECK(hipGetLastError());
+    if (r && n) HIP_CHECK(hipMemcpyAsync(r, out, sizeof(double) * 6 * n, hipMemcpyDeviceToHost, st));
+    if (v && n) HIP_CHECK(hipMemcpyAsync(v, out + 6 * n, sizeof(double) * 6 * n, hipMemcpyDeviceToHost, st));
+    if (extrema && n) HIP_CHECK(hipMemcpyAsync(extrema, out + 12 * n, sizeof(double) * 2 * n, hipMemcpyDeviceToHost, st));
+    HIP_CHECK(hipStreamSynchronize(st));
     return EPH_OK;
 }
 

@@ -82,7 +82,11 @@ struct Batch {
     eph_geopotential *d_gps = nullptr;
     eph_ring *d_rings = nullptr;
     int32_t *d_np_gp = nullptr, *d_np_ring = nullptr, *d_bsys = nullptr;
+    uint64_t *d_sid = nullptr;
     double *d_t0 = nullptr;
+    // eph_mass records of an upload or download: the rows from F_X0R on are
+    // per-step scratch, free between calls, and larger than the records
+    eph_mass *d_records() const { return (eph_mass *)(F + (int64_t)F_X0R * nbp); }
     int2 *d_blk_all = nullptr;
     int n_blk_all = 0;
     // deform work split by tidal class (see build_class_tables)
@@ -118,6 +122,7 @@ struct Batch {
     ~Batch();
     int build_plan(int mode);
     int build_class_tables(const eph_mass *masses);
+    bool same_classes(const eph_mass *masses) const;
     View view(int mode) const;
     int accel(int mode, bool deform_only);
     int integrate(double dt, int64_t n_step, int mode);
@@ -170,6 +175,8 @@ int download_particles(Particles *ps, double *r, double *v, double *extrema);
 // [0, kMassFieldEnd) except phi / c^2 and naccel / c^2
 struct FieldMap { int field; size_t offset; };
 constexpr int kMassFieldEnd = F_X0R;   // fields [0, F_X0R) carry eph_mass data
+static_assert((size_t)(F_COUNT - F_X0R) * 8 >= sizeof(eph_mass), "the per-step scratch rows hold the records of a transfer");
+static_assert(P_STAGE_ROWS >= 14, "the particles' scratch rows hold their records");
 const std::vector<FieldMap> &mass_field_map();
 // set-up of the allocation-free entry point on the current device
 int noalloc_init_device(int device);
