@@ -199,6 +199,7 @@ JMain jmain_of(const eph_mass &m) {
     memset(&T, 0, sizeof T);
     T.rxh = m.r.x.hi; T.rxl = m.r.x.lo; T.ryh = m.r.y.hi; T.ryl = m.r.y.lo; T.rzh = m.r.z.hi; T.rzl = m.r.z.lo;
     T.GM = m.GM; T.sR2 = m.sR2;
+    T.GM2c = 2 * m.GM / kC;
     T.phi = m.phi; T.beta2 = m.beta2;
     T.bx = m.beta.x; T.by = m.beta.y; T.bz = m.beta.z;
     T.nx = m.naccel.x; T.ny = m.naccel.y; T.nz = m.naccel.z;

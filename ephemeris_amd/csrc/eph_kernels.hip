@@ -10,6 +10,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace eph {
 
 // ---------------------------------------------------------------------------
@@ -19,6 +21,13 @@ __constant__ double2 c_rk[325];                    // Feagin RK12, {hi, lo}
 // Non-zero coefficients of each row k = 1..25: entries c_row0[k] ..
 // c_row0[k + 1] - 1 of c_nzj hold their column j, ascending (set with c_rk)
 __constant__ int c_nzj[325];
+// The same with every row padded to a multiple of four columns by zero
+// coefficients on the row's last column: entries c_pad0[k] .. c_pad0[k + 1] -
+// 1 of c_padj and c_padc (four more may be read past the last row)
+constexpr int kPadCols = 325 + 3 * 25 + 4;
+__constant__ int c_padj[kPadCols];
+__constant__ double2 c_padc[kPadCols];
+__constant__ int c_pad0[27];
 __constant__ int c_row0[27];
 
 __device__ const float g_fz[32 * 64 * 16] = {
@@ -54,6 +63,8 @@ struct Acc {
     __device__ void stddv(int f, int g, ddv3 a) const { std_(f, g, a.x); std_(f + 2, g, a.y); std_(f + 4, g, a.z); }
     __device__ ddm3 lddm(int f, int g) const { return ddm3{lddv(f, g), lddv(f + 6, g), lddv(f + 12, g)}; }
     __device__ void stddm(int f, int g, const ddm3 &a) const { stddv(f, g, a.x); stddv(f + 6, g, a.y); stddv(f + 12, g, a.z); }
+    __device__ v3 ldgl(int g) const { return todbl(lddv(F_GL, g)); }          // GL rounded to double
+    __device__ double ldgm2c(int g) const { return 2 * ld(F_GM, g) / kC; }
 };
 
 // ---------------------------------------------------------------------------
@@ -68,11 +79,12 @@ struct DevRingTab {
     __device__ static double kserkm(double x) { return padesum(x, c_kserkm); }
     __device__ static double kser0(double x) { return padesum(x, c_kser0); }
 };
-__device__ v3 ring_sum(const eph_ring &rg, double host_R, v3 r) { return ring_sum_t<DevRingTab>(rg, host_R, r); }
+__device__ __forceinline__ v3 ring_sum(const eph_ring &rg, double host_R, v3 r) { return ring_sum_t<DevRingTab>(rg, host_R, r); }
 
 // world-frame acceleration (per unit GM of the non-point body p) at offset r
 // from p: geopotential (mass.cpp:186-188) or ring (mass.cpp:200-203)
-__device__ __forceinline__ v3 nonpoint_field_inl(const View &d, const Acc &A, int p, int kind, int model, v3 r) {
+template <class Access>
+__device__ __forceinline__ v3 nonpoint_field_inl(const View &d, const Access &A, int p, int kind, int model, v3 r) {
     double R = A.ld(F_RAD, p);
     if (kind == 0) {
         m3 fmis = todbl(A.lddm(F_S, p));
@@ -182,7 +194,8 @@ struct PartnerBlock {
 struct JDeform { double rxh, rxl, ryh, ryl, rzh, rzl, vxh, vxl, vyh, vyl, vzh, vzl, GM, sR2, tdf, pad; };
 
 // Per-body constants of UPDATE_HARMONICS (mass.impl:48-61) from the state
-__device__ __forceinline__ Harmonics harmonics_load(const Acc &Ac, int g) {
+template <class Access>
+__device__ __forceinline__ Harmonics harmonics_load(const Access &Ac, int g) {
     Harmonics h;
     h.set(Ac.ld(F_K2R, g), Ac.ld(F_RAD, g), Ac.ld(F_R2, g), Ac.ld(F_A, g), Ac.ld(F_GM, g), Ac.ld(F_EXJ2, g),
           Ac.ldm(F_CST, g), todbl(Ac.lddm(F_S, g)));
@@ -190,7 +203,8 @@ __device__ __forceinline__ Harmonics harmonics_load(const Acc &Ac, int g) {
 }
 
 // UPDATE_ANGULAR_VELOCITY (mass.impl:63-72); returns should_break
-__device__ __forceinline__ bool update_spin(const Acc &A, int g, const m3 &GI, v3 &w, const ddv3 &GL) {
+template <class Access>
+__device__ __forceinline__ bool update_spin(const Access &A, int g, const m3 &GI, v3 &w, const ddv3 &GL) {
     bool gl_from_w;
     const bool brk = spin_step(GI, w, GL, gl_from_w);
     if (gl_from_w) A.stddv(F_GL, g, mkddv(GI * w));
@@ -207,7 +221,8 @@ __device__ __forceinline__ void load_jdeform(const Acc &A, JDeform &T, int gj) {
     T.GM = A.ld(F_GM, gj); T.sR2 = A.ld(F_SR2, gj); T.tdf = A.ld(F_TDF, gj);
 }
 
-__device__ __forceinline__ void deform_write(const Acc &A, int g, int prepare, const ddv3 &vi, double phi, v3 nacc,
+template <class Access>
+__device__ __forceinline__ void deform_write(const Access &A, int g, int prepare, const ddv3 &vi, double phi, v3 nacc,
                                              const m3 &C, const m3 &GI, v3 w) {
     A.stm(F_CPOT, g, C);
     A.stm(F_GI, g, GI);
@@ -256,8 +271,8 @@ __global__ __launch_bounds__(BS) void k_deform_light(View d, const int4 *__restr
             const JDeform &T = tile[q];
             const ddv3 rj{dd{T.rxh, T.rxl}, dd{T.ryh, T.ryl}, dd{T.rzh, T.rzl}};
             const v3 r = diff(rj, ri);
-            const double rr2 = 1 / smax(dot(r, r), sR2 + T.sR2);
-            const double rr = sqrt(rr2);
+            double rr2, rr;
+            recip_and_root(smax(dot(r, r), sR2 + T.sR2), rr2, rr);
             const double tp_dphi = rr * T.GM;
             const double tp_dg = rr2 * tp_dphi;
             phi -= tp_dphi;                                // _NK2 (mass.impl:38-46) / _NDELAY (:25-36)
@@ -277,7 +292,7 @@ __global__ __launch_bounds__(BS) void k_deform_light(View d, const int4 *__restr
     int iters = 4;                                         // MAX_ANGULAR_VELOCITY_ITER
     for (;;) {
         H.apply(Csum, w, C, GI);
-        if (!prepare || update_spin(A, gi, GI, w, GL) || --iters == 0) break;
+        if (!prepare || update_spin(A, gi, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
     }
     deform_write(A, gi, prepare, A.lddv(F_V, gi), phi, nacc, C, GI, w);
 }
@@ -332,8 +347,8 @@ __device__ __forceinline__ void deform_k4_body(View d, const int4 *__restrict__ 
             const double *J = jb + k * Blk::P;
             const ddv3 rj{dd{J[0], J[1]}, dd{J[2], J[3]}, dd{J[4], J[5]}};
             const v3 r = diff(rj, ri);
-            const double rr2 = 1 / smax(dot(r, r), sR2 + J[6]);
-            const double rr = sqrt(rr2);
+            double rr2, rr;
+            recip_and_root(smax(dot(r, r), sR2 + J[6]), rr2, rr);
             const double tp_dphi = rr * J[7];
             const double tp_dg = rr2 * tp_dphi;
             const v3 na = tp_dg * r;
@@ -389,7 +404,7 @@ __device__ __forceinline__ void deform_k4_body(View d, const int4 *__restrict__ 
     int iters = 4;                                         // MAX_ANGULAR_VELOCITY_ITER
     for (;;) {
         H.apply(Csum, w, C, GI);
-        if (!prepare || update_spin(A, gi, GI, w, GL) || --iters == 0) break;
+        if (!prepare || update_spin(A, gi, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
     }
     deform_write(A, gi, prepare, A.lddv(F_V, gi), phi, nacc, C, GI, w);
 }
@@ -434,8 +449,8 @@ __global__ __launch_bounds__(BS) void k_deform_damped(View d, const int4 *__rest
                 const ddv3 vj{dd{T.vxh, T.vxl}, dd{T.vyh, T.vyl}, dd{T.vzh, T.vzl}};
                 const v3 r = diff(rj, ri);
                 const v3 v = diff(vj, vi);
-                const double rr2 = 1 / smax(dot(r, r), sR2 + T.sR2);
-                const double rr = sqrt(rr2);
+                double rr2, rr;
+                recip_and_root(smax(dot(r, r), sR2 + T.sR2), rr2, rr);
                 const double tp_dphi = rr * T.GM;
                 phi -= tp_dphi;
                 const double tp_dg = rr2 * tp_dphi;
@@ -471,7 +486,8 @@ __global__ __launch_bounds__(BS) void k_deform_damped(View d, const int4 *__rest
 // ---------------------------------------------------------------------------
 // main force, thread-pool summation order (mass.cpp:136-157)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void load_jmain(const Acc &A, JMain &T, int gj) {
+template <class Access>
+__device__ __forceinline__ void load_jmain(const Access &A, JMain &T, int gj) {
     T.rxh = A.ld(F_R + 0, gj); T.rxl = A.ld(F_R + 1, gj);
     T.ryh = A.ld(F_R + 2, gj); T.ryl = A.ld(F_R + 3, gj);
     T.rzh = A.ld(F_R + 4, gj); T.rzl = A.ld(F_R + 5, gj);
@@ -482,19 +498,20 @@ __device__ __forceinline__ void load_jmain(const Acc &A, JMain &T, int gj) {
 #pragma unroll
     for (int q = 0; q < 9; ++q) T.C[q] = A.ld(F_CPOT + q, gj);
     T.R2 = A.ld(F_R2, gj);
-    T.GLx = todbl(dd{A.ld(F_GL + 0, gj), A.ld(F_GL + 1, gj)});
-    T.GLy = todbl(dd{A.ld(F_GL + 2, gj), A.ld(F_GL + 3, gj)});
-    T.GLz = todbl(dd{A.ld(F_GL + 4, gj), A.ld(F_GL + 5, gj)});
+    const v3 gl = A.ldgl(gj);
+    T.GLx = gl.x; T.GLy = gl.y; T.GLz = gl.z;
     T.lum = A.ld(F_LUM, gj);
+    T.GM2c = A.ldgm2c(gj);
 }
 
-__device__ __forceinline__ IMain load_imain(const Acc &A, int gi) {
+template <class Access>
+__device__ __forceinline__ IMain load_imain(const Access &A, int gi) {
     IMain I;
     I.r = A.lddv(F_R, gi);
     I.sR2 = A.ld(F_SR2, gi); I.phi = A.ld(F_PHIC, gi); I.beta2 = A.ld(F_BETA2, gi);
     I.R2 = A.ld(F_R2, gi); I.GM = A.ld(F_GM, gi); I.rR2G4c = A.ld(F_RR2G4C, gi);
     I.beta = A.ldv(F_BETA, gi);
-    I.GL = todbl(A.lddv(F_GL, gi));
+    I.GL = A.ldgl(gi);
     I.C = A.ldm(F_CPOT, gi);
     return I;
 }
@@ -579,7 +596,7 @@ __device__ __forceinline__ PairTerms pair_terms_k4(const IMain &I, bool own_quad
         const m3 Cj{v3{T.C[0], T.C[1], T.C[2]}, v3{T.C[3], T.C[4], T.C[5]}, v3{T.C[6], T.C[7], T.C[8]}};
         o.gj = (T.GM * p.rr3 * p.rr2 * T.R2) * quad_field(Cj, p);
     }
-    const double rcr32 = 2 * T.GM / kC * p.rr3;
+    const double rcr32 = T.GM2c * p.rr3;
     const v3 GLb = cross(I.GL, p.b);
     o.lt1 = rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r);
     o.lt2 = rcr32 * cross(I.GL, cross(p.r, p.b));
@@ -808,7 +825,7 @@ constexpr int kNpHead = 15 * kNpFusedMaxItems + 8;
 constexpr int kNpScratch = kNpHead + 6 * kNpFusedMaxN;
 
 template <bool NP, int W>
-__global__ __launch_bounds__(64 * W) void k_main_wpb(View d, const int2 *__restrict__ work) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 1))) void k_main_wpb(View d, const int2 *__restrict__ work) {
     static_assert(!NP || W * kWpbTile >= kNpScratch, "term tiles double as non-point scratch");
     const Acc A{d.F, d.nbp};
     const int s = work[blockIdx.x].x, il = work[blockIdx.x].y;
@@ -1140,8 +1157,8 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
     auto pair_geo = [&](int jl) {
         const int gj = off + jl;
         pr = diff(A.lddv(F_R, gj), ri);
-        prr2 = 1 / smax(dot(pr, pr), sR2 + A.ld(F_SR2, gj));
-        const double rr = sqrt(prr2);
+        double rr;
+        recip_and_root(smax(dot(pr, pr), sR2 + A.ld(F_SR2, gj)), prr2, rr);
         ptp_dphi = rr * A.ld(F_GM, gj);
         ptp_dg = prr2 * ptp_dphi;
         if (damped) {
@@ -1261,7 +1278,7 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
                 int iters = 4;
                 for (;;) {
                     H.apply(Csum, w, C, GI);
-                    if (!prepare || update_spin(A, gi, GI, w, GL) || --iters == 0) break;
+                    if (!prepare || update_spin(A, gi, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
                 }
                 brk = true;
             }
@@ -1325,8 +1342,7 @@ __device__ __forceinline__ SerialReact serial_reaction_terms(const View &d, cons
     const ddv3 rp{dd{T.rxh, T.rxl}, dd{T.ryh, T.ryl}, dd{T.rzh, T.rzl}};
     PairGeo p;
     p.r = diff(I.r, rp);
-    p.rr2 = 1 / smax(dot(p.r, p.r), T.sR2 + I.sR2);
-    p.rr = sqrt(p.rr2);
+    recip_and_root(smax(dot(p.r, p.r), T.sR2 + I.sR2), p.rr2, p.rr);
     p.rr3 = p.rr * p.rr2;
     const m3 Cp{v3{T.C[0], T.C[1], T.C[2]}, v3{T.C[3], T.C[4], T.C[5]}, v3{T.C[6], T.C[7], T.C[8]}};
     const v3 dg = (p.rr3 * p.rr2 * T.R2) * quad_field(Cp, p);
@@ -1476,7 +1492,7 @@ __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *
                 const v3 dg = (p.rr3 * p.rr2 * I.R2) * quad_field(I.C, p);
                 e[0] = T.GM * dg;
                 e[1] = T.GM * cross(p.r, dg);
-                const double rcr32 = 2 * T.GM / kC * p.rr3;
+                const double rcr32 = T.GM2c * p.rr3;
                 const v3 GLb = cross(I.GL, p.b);
                 e[2] = -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r));
                 e[3] = -(rcr32 * cross(I.GL, cross(p.r, p.b)));
@@ -1506,8 +1522,7 @@ __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *
             if (quad && R2p != 0) {                        // outer body p visiting partner i: r = r_i - r_p
                 PairGeo p;
                 p.r = diff(I.r, A.lddv(F_R, gp_));
-                p.rr2 = 1 / smax(dot(p.r, p.r), A.ld(F_SR2, gp_) + I.sR2);
-                p.rr = sqrt(p.rr2);
+                recip_and_root(smax(dot(p.r, p.r), A.ld(F_SR2, gp_) + I.sR2), p.rr2, p.rr);
                 p.rr3 = p.rr * p.rr2;
                 e[0] = -(GMp * ((p.rr3 * p.rr2 * R2p) * quad_field(Cp, p)));
             }
@@ -1733,102 +1748,9 @@ __global__ __launch_bounds__(kBS) void k_np_recv(View d, const int2 *__restrict_
 // one (r, v, the stage's acceleration, GM(t), exJ2(t)) and the rotational one
 // (GL, the frame s, w, torque, Egrad).  Neither reads a field the other
 // writes, so k_stage runs them in different workgroups.
-__device__ __forceinline__ void stage_translational(const View &d, const Acc &A, int g, int k, double dt, double tadd) {
-    const ddv3 v = A.lddv(F_V, g);
-    if (k == 1) {
-        A.stddv(F_X0R, g, A.lddv(F_R, g));
-        A.stddv(F_X0V, g, v);
-    }
-    const v3 a_now = (A.ldv(F_GACC, g) + A.ldv(F_DACC, g)) + A.ldv(F_NACC, g);
-    {
-        const int fb = F_STAGE + (k - 1) * kStageFields;
-        A.stddv(fb, g, v);
-        A.stv(fb + 6, g, a_now);
-    }
-    const ddv3 r0 = A.lddv(F_X0R, g), v0 = A.lddv(F_X0V, g);
-    const double gm0 = A.ld(F_GM0, g), dgm = A.ld(F_DGM, g), dj2 = A.ld(F_DJ2, g);
-    const double t = d.t0[d.bsys[g]] + tadd;
-    ddv3 cv = mkddv(v3{0, 0, 0});
-    v3 ca{0, 0, 0};
-    const int base = k * (k - 1) / 2;
-    const int e1 = c_row0[k + 1];
-#pragma unroll 4
-    for (int e = c_row0[k]; e < e1; ++e) {              // non-zero columns, ascending
-        const int j = c_nzj[e];
-        const double2 c = c_rk[base + j];
-        const dd ckj{c.x, c.y};
-        const double fc = c.x + c.y;
-        const int fb = F_STAGE + j * kStageFields;
-        const bool now = j == k - 1;                    // this stage's record, still in registers
-        cv = add(cv, scale(ckj, now ? v : A.lddv(fb, g)));
-        ca += fc * (now ? a_now : A.ldv(fb + 6, g));
-    }
-    A.stddv(F_R, g, add(r0, scale(mkdd(dt), cv)));
-    A.stddv(F_V, g, add(v0, mkddv(dt * ca)));
-    A.st(F_GM, g, gm0 + dgm * t);
-    A.st(F_EXJ2, g, dj2 * t);
-}
-
-__device__ __forceinline__ void stage_rotational(const Acc &A, int g, int k, double dt, double dt_k) {
-    if (k == 1) {
-        A.stddv(F_X0GL, g, A.lddv(F_GL, g));
-        A.stddm(F_X0S, g, A.lddm(F_S, g));
-        A.stv(F_X0W, g, A.ldv(F_W, g));
-        A.stv(F_EGRAD, g, A.ldv(F_DTQ, g));
-    }
-    const v3 w_now = A.ldv(F_W, g), tq_now = A.ldv(F_DTQ, g);
-    {
-        const int fb = F_STAGE + (k - 1) * kStageFields;
-        A.stv(fb + 9, g, w_now);
-        A.stv(fb + 12, g, tq_now);
-    }
-    v3 egrad = A.ldv(F_EGRAD, g);
-    if (k == 25) {
-        egrad = egrad_k25(A.ldm(F_GI, g), todbl(A.lddv(F_GL, g)), w_now, tq_now, egrad, dt);
-        A.stv(F_EGRAD, g, egrad);
-    }
-    const ddv3 gl0 = A.lddv(F_X0GL, g);
-    const v3 w0 = A.ldv(F_X0W, g);
-    ddm3 sm = A.lddm(F_X0S, g);
-    v3 cw{0, 0, 0}, ct{0, 0, 0};
-    const int base = k * (k - 1) / 2;
-    const int e1 = c_row0[k + 1];
-#pragma unroll 4
-    for (int e = c_row0[k]; e < e1; ++e) {              // non-zero columns, ascending
-        const int j = c_nzj[e];
-        const double2 c = c_rk[base + j];
-        const double fc = c.x + c.y;
-        const int fb = F_STAGE + j * kStageFields;
-        const bool now = j == k - 1;                    // this stage's record, still in registers
-        cw += fc * (now ? w_now : A.ldv(fb + 9, g));
-        ct += fc * (now ? tq_now : A.ldv(fb + 12, g));
-    }
-    const v3 w = cw / dt_k;
-    const v3 dw = (2.0 / 3) * (w - w0);
-    sm = add(sm, rotation_matrix(w - dw, dt * dt_k / 2, DevSin{}) * todbl(sm));
-    sm = add(sm, rotation_matrix(w + dw, dt * dt_k / 2, DevSin{}) * todbl(sm));
-    A.stddv(F_GL, g, add(gl0, mkddv(dt * ct)));
-    if (k == 25) {
-        sm = add(sm, rotation_matrix(egrad, 1.0 / 72, DevSin{}) * todbl(sm));
-        sm = orthogonalized(sm);
-    }
-    A.stddm(F_S, g, sm);
-    A.stv(F_W, g, w);
-}
-
-// the persistent small-system kernel keeps the two halves of the stage
-// update out of line and runs them on different threads
-__device__ __noinline__ void stage_translational_ool(const View &d, const Acc &A, int g, int k, double dt, double tadd) {
-    stage_translational(d, A, g, k, dt, tadd);
-}
-__device__ __noinline__ void stage_rotational_ool(const Acc &A, int g, int k, double dt, double dt_k) {
-    stage_rotational(A, g, k, dt, dt_k);
-}
-
-// Component c (0, 1, 2 = x, y, z) of the translational stage update: the
-// same operations as stage_translational on that component of every
-// vector (they never mix components), so each thread's results are the
-// bits of the one-thread update.
+//
+// Component c (0, 1, 2 = x, y, z) of the translational stage update
+// (its operations never mix components).
 __device__ __forceinline__ void stage_translational_c(const View &d, const Acc &A, int g, int c, int k, double dt,
                                                       double tadd) {
     const dd v = A.ldd(F_V + 2 * c, g);
@@ -1875,7 +1797,7 @@ __device__ __forceinline__ void stage_translational_c(const View &d, const Acc &
 // vector component c, so the long dependent sums over the stage records run
 // on three lanes per body instead of one.  In the rotational half the
 // component sums of the spin meet in LDS and wavefront 0 then forms the
-// rotation of the frame (stage_rotational's operations, in its order).
+// rotation of the frame.
 __global__ __launch_bounds__(192) void k_stage(View d, int k, double dt, double dt_k, double tadd,
                                                const int64_t *__restrict__ istep) {
     const Acc A{d.F, d.nbp};
@@ -1961,316 +1883,7 @@ __global__ void k_step_count(int64_t *istep) {
     if (threadIdx.x == 0) *istep += 1;
 }
 
-// ---------------------------------------------------------------------------
-// whole-system-in-one-workgroup path: every body of the system sits in one
-// LDS tile, so deform and main force need no further tile traffic
-// ---------------------------------------------------------------------------
-// Deformation of a small system by the whole workgroup, pass by pass: in
-// each pass the threads form the terms of the pairs (i, q) of the bodies
-// still iterating -- -phi, naccel and the subtracted tidal matrix of
-// deform_by (mass.cpp:78-103), the last one at the body's current spin for a
-// constant-time-lag body -- into LDS, thirteen threads per body add them in
-// partner order, and the body's own thread runs UPDATE_HARMONICS and
-// UPDATE_ANGULAR_VELOCITY.  A body without delayed tides sums once and
-// iterates its spin on those sums (its terms do not depend on the spin);
-// a constant-time-lag body re-sums its tidal matrix at every pass, as the
-// reference does, up to MAX_ANGULAR_VELOCITY_ITER passes (phi and naccel do
-// not change between passes).
-struct SmallDefShared {
-    double w[kSmallMax * 3], k2[kSmallMax], td[kSmallMax];
-    int act[kSmallMax], list[kSmallMax], na;
-};
-
-__device__ __forceinline__ void small_deform_terms(const JDeform &Ti, const JDeform &T, double k2, double td, v3 w,
-                                                   bool first, double *o) {
-    const ddv3 ri{dd{Ti.rxh, Ti.rxl}, dd{Ti.ryh, Ti.ryl}, dd{Ti.rzh, Ti.rzl}};
-    const ddv3 rj{dd{T.rxh, T.rxl}, dd{T.ryh, T.ryl}, dd{T.rzh, T.rzl}};
-    const v3 r = diff(rj, ri);
-    const double rr2 = 1 / smax(dot(r, r), Ti.sR2 + T.sR2);
-    const double rr = sqrt(rr2);
-    const double tp_dphi = rr * T.GM;
-    const double tp_dg = rr2 * tp_dphi;
-    if (first) {
-        const v3 na = tp_dg * r;
-        o[0] = -tp_dphi;                                   // phi -= tp_dphi
-        o[1] = na.x; o[2] = na.y; o[3] = na.z;             // naccel += tp_dg r
-    }
-    m3 X = mzero();                                        // Csum -= X
-    if (k2 != 0 && td != 0) {                              // DAMPED_TIDAL_DEFORMATION_MATRIX
-        const ddv3 vi{dd{Ti.vxh, Ti.vxl}, dd{Ti.vyh, Ti.vyl}, dd{Ti.vzh, Ti.vzl}};
-        const ddv3 vj{dd{T.vxh, T.vxl}, dd{T.vyh, T.vyl}, dd{T.vzh, T.vzl}};
-        const v3 v = diff(vj, vi);
-        const double fmj = -3 * tp_dg;
-        v3 dw = rr2 * cross(r, cross(w, r) - v);
-        double dwt = normalize(dw);
-        dwt *= td * T.tdf;
-        const double ecwt2 = 1 + 4 * dwt * dwt,
-                     secwt2 = sqrt(ecwt2),
-                     x0 = sqrt((1 + secwt2) / (2 * ecwt2)),
-                     y0 = dwt * sqrt(2 / (ecwt2 * (1 + secwt2))),
-                     z02 = dwt * dwt * (2 / (ecwt2 + secwt2));
-        const v3 dr = x0 * r + y0 * cross(dw, r);
-        m3 t = outer(rr2 * dr, dr) - outer(z02 * dw, dw);
-        t = adddiag(t, z02 - 1.0 / 3);
-        X = (fmj * k2) * t;
-    } else if (k2 != 0) {                                  // _NDELAY
-        const double fmj = -3 * tp_dg;
-        X = (fmj * k2) * subdiag(outer(rr2 * r, r), 1.0 / 3);
-    }
-    const double *x = &X.x.x;
-#pragma unroll
-    for (int c = 0; c < 9; ++c) o[4 + c] = -x[c];
-}
-
-// called by every thread of the workgroup of NT threads (it synchronises)
-template <int NT>
-__device__ void deform_small(const Acc &A, int off, int n, const JDeform *tile, double *terms, double *sums,
-                             SmallDefShared &sh) {
-    const int tid = (int)threadIdx.x;
-    const bool body = tid < n;
-    const int gi = off + (body ? tid : 0);
-    // the body's own state, held by its thread across the passes
-    ddv3 vi{}, GL{};
-    Harmonics H{};
-    v3 w{0, 0, 0}, nacc{0, 0, 0};
-    double phi = 0, k2 = 0, td = 0;
-    m3 C = mzero(), GI = mzero();
-    if (body) {
-        vi = A.lddv(F_V, gi);
-        k2 = A.ld(F_K2, gi);
-        td = A.ld(F_TD, gi);
-        GL = A.lddv(F_GL, gi);
-        H = harmonics_load(A, gi);
-        w = A.ldv(F_W, gi);
-        sh.w[3 * tid] = w.x; sh.w[3 * tid + 1] = w.y; sh.w[3 * tid + 2] = w.z;
-        sh.k2[tid] = k2;
-        sh.td[tid] = td;
-        sh.act[tid] = 1;
-        sh.list[tid] = tid;
-    }
-    if (tid == 0) sh.na = n;
-    __syncthreads();
-    const int m = n - 1;                                   // pairs per body
-    const int bpr = m > 0 ? min(NT / m, NT / 13) : 1;      // bodies per round
-    for (int pass = 0; pass < 4; ++pass) {
-        const int na = sh.na;
-        if (na == 0) break;
-        const bool first = pass == 0;
-        for (int b0 = 0; b0 < na && m > 0; b0 += bpr) {
-            const int nb = min(bpr, na - b0);
-            if (tid < nb * m) {
-                const int il = sh.list[b0 + tid / m], qq = tid - (tid / m) * m;
-                const int q = qq < il ? qq : qq + 1;
-                small_deform_terms(tile[il], tile[q], sh.k2[il], sh.td[il],
-                                   v3{sh.w[3 * il], sh.w[3 * il + 1], sh.w[3 * il + 2]}, first, terms + tid * 13);
-            }
-            __syncthreads();
-            if (tid < 13 * nb) {
-                const int j = tid / 13, c = tid - j * 13;
-                const int il = sh.list[b0 + j];
-                if (first || c >= 4) {
-                    const double *P = terms + j * m * 13 + c;
-                    double acc = 0;
-                    for (int qq = 0; qq < m; ++qq) acc += P[qq * 13];
-                    sums[il * 13 + c] = acc;
-                }
-            }
-            __syncthreads();
-        }
-        if (m == 0 && body) {                              // no partner: the sums stay +0
-            for (int c = 0; c < 13; ++c) sums[tid * 13 + c] = 0.0;
-        }
-        __syncthreads();
-        if (body && sh.act[tid]) {
-            const double *S = sums + tid * 13;
-            if (first) {
-                phi = S[0];
-                nacc = v3{S[1], S[2], S[3]};
-            }
-            const m3 Csum{v3{S[4], S[5], S[6]}, v3{S[7], S[8], S[9]}, v3{S[10], S[11], S[12]}};
-            if (!(k2 != 0 && td != 0)) {                   // the spin iterates on the same sums
-                int iters = 4;                             // MAX_ANGULAR_VELOCITY_ITER
-                for (;;) {
-                    H.apply(Csum, w, C, GI);
-                    if (update_spin(A, gi, GI, w, GL) || --iters == 0) break;
-                }
-                sh.act[tid] = 0;
-            } else {
-                H.apply(Csum, w, C, GI);
-                const bool brk = update_spin(A, gi, GI, w, GL);
-                sh.act[tid] = (brk || pass == 3) ? 0 : 1;
-                sh.w[3 * tid] = w.x; sh.w[3 * tid + 1] = w.y; sh.w[3 * tid + 2] = w.z;
-            }
-        }
-        __syncthreads();
-        if (tid == 0) {
-            int k = 0;
-            for (int i = 0; i < n; ++i)
-                if (sh.act[i]) sh.list[k++] = i;
-            sh.na = k;
-        }
-        __syncthreads();
-    }
-    if (body) deform_write(A, gi, 1, vi, phi, nacc, C, GI, w);
-}
-
-// Main force of a small system in the single-thread order, by the whole
-// workgroup: each thread forms every term of one ordered pair (i, q) -- the
-// own-loop terms of i's partner q and the reaction terms of outer body q on
-// i -- into LDS; then ten threads per body add them in the order of the
-// sequential loop (mass.cpp:329-374): daccel takes the reactions of q < i,
-// the own-loop terms of every q, the reactions of q > i; dtorque and gaccel
-// the own-loop terms; the running maxima go over the partners.  A body's
-// pairs fall in one round, so its sums are never split.  Terms of a model
-// the body does not have are +0, an exact identity in these sums.
-constexpr int kSmallTerm = 44;                         // doubles per pair
-// pair slots: 0-2 G; 3-20 daccel own terms (GM dg, -LT own spin, +LT
-// partner spin, radiation, -GM field_gp, -GM field_ring); 21-32 dtorque
-// own terms (GM r x dg, -LT torque, -GM r x field_gp, -GM r x field_ring);
-// 33-41 daccel reaction terms (-GM_q dg_q, +GM_q field_gp, +GM_q field_ring);
-// 42 1/r, 43 GM/r^3
-__device__ void small_pair_terms(const View &d, const Acc &A, int off, int il, int q, const JMain &T, double *o) {
-    const int gi = off + il;
-    const IMain I = load_imain(A, gi);
-    const int my_gp = d.np_gp[gi], my_ring = d.np_ring[gi];
-    v3 unused{0, 0, 0};
-    const PairGeo p = relativity(I, T, unused);
-    v3 ta[6], tq[4];
-    const v3 dg = (p.rr3 * p.rr2 * I.R2) * quad_field(I.C, p);
-    ta[0] = T.GM * dg;
-    tq[0] = T.GM * cross(p.r, dg);
-    // LENSE_THIRRING and RADIATION_PRESSURE as lt_rad forms them
-    const double rcr32 = 2 * T.GM / kC * p.rr3;
-    const v3 GLb = cross(I.GL, p.b);
-    ta[1] = -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r));
-    tq[1] = -(rcr32 * cross(I.GL, cross(p.r, p.b)));
-    const v3 GLj{T.GLx, T.GLy, T.GLz};
-    ta[2] = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
-    ta[3] = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
-    ta[4] = ta[5] = tq[2] = tq[3] = v3{0, 0, 0};
-    if (my_gp >= 0) {
-        const v3 an = nonpoint_field_call(d, A, gi, 0, my_gp, p.r);
-        ta[4] = -(T.GM * an);
-        tq[2] = -(T.GM * cross(p.r, an));
-    }
-    if (my_ring >= 0) {
-        const v3 an = nonpoint_field_call(d, A, gi, 1, my_ring, p.r);
-        ta[5] = -(T.GM * an);
-        tq[3] = -(T.GM * cross(p.r, an));
-    }
-    const SerialReact r = serial_reaction_terms(d, A, off + q, il, T, I, false);
-    o[0] = p.G.x; o[1] = p.G.y; o[2] = p.G.z;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) { o[3 + 3 * k] = ta[k].x; o[4 + 3 * k] = ta[k].y; o[5 + 3 * k] = ta[k].z; }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { o[21 + 3 * k] = tq[k].x; o[22 + 3 * k] = tq[k].y; o[23 + 3 * k] = tq[k].z; }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) { o[33 + 3 * k] = r.t[k].x; o[34 + 3 * k] = r.t[k].y; o[35 + 3 * k] = r.t[k].z; }
-    o[42] = p.rr;
-    o[43] = p.tp_dg;
-}
-
-// called by every thread of the workgroup of NT threads (it synchronises)
-template <int NT>
-__device__ void main_serial_small(const View &d, const Acc &A, int off, int n, const JMain *tile, double *terms,
-                                  double *sums) {
-    const int tid = (int)threadIdx.x;
-    if (n > 1) {
-        const int m = n - 1;                                // pairs per body
-        const int bpr = min(12, NT / m);                    // bodies per round (10 sum threads each)
-        for (int b0 = 0; b0 < n; b0 += bpr) {
-            const int nb = min(bpr, n - b0);
-            if (tid < nb * m) {
-                const int il = b0 + tid / m, qq = tid - (tid / m) * m;
-                const int q = qq < il ? qq : qq + 1;
-                small_pair_terms(d, A, off, il, q, tile[q], terms + tid * kSmallTerm);
-            }
-            __syncthreads();
-            if (tid < 10 * nb) {
-                const int il = b0 + tid / 10, c = tid - (tid / 10) * 10;
-                const double *P = terms + (il - b0) * m * kSmallTerm;   // this body's pairs, q ascending
-                double acc = 0;
-                if (c < 3) {                                // daccel
-                    for (int qq = 0; qq < il; ++qq)
-                        for (int k = 0; k < 3; ++k) acc += P[qq * kSmallTerm + 33 + 3 * k + c];
-                    for (int qq = 0; qq < m; ++qq)
-                        for (int k = 0; k < 6; ++k) acc += P[qq * kSmallTerm + 3 + 3 * k + c];
-                    for (int qq = il; qq < m; ++qq)
-                        for (int k = 0; k < 3; ++k) acc += P[qq * kSmallTerm + 33 + 3 * k + c];
-                } else if (c < 6) {                         // dtorque
-                    for (int qq = 0; qq < m; ++qq)
-                        for (int k = 0; k < 4; ++k) acc += P[qq * kSmallTerm + 21 + 3 * k + (c - 3)];
-                } else if (c < 9) {                         // gaccel
-                    for (int qq = 0; qq < m; ++qq) acc += P[qq * kSmallTerm + (c - 6)];
-                } else {                                    // running maxima
-                    const int gi = off + il;
-                    double mind = A.ld(F_MIND, gi), maxi = A.ld(F_MAXI, gi);
-                    for (int qq = 0; qq < m; ++qq) {
-                        mind = checked_max_into(mind, P[qq * kSmallTerm + 42]);
-                        maxi = checked_max_into(maxi, P[qq * kSmallTerm + 43]);
-                    }
-                    sums[il * 11 + 10] = maxi;
-                    acc = mind;
-                }
-                sums[il * 11 + c] = acc;
-            }
-            __syncthreads();
-        }
-    }
-    if (tid < n) {
-        const int gi = off + tid;
-        const double *S = sums + tid * 11;
-        const bool any = n > 1;
-        A.stv(F_GACC, gi, any ? v3{S[6], S[7], S[8]} : v3{0, 0, 0});
-        if (any) {
-            A.st(F_MIND, gi, S[9]);
-            A.st(F_MAXI, gi, S[10]);
-        }
-        finalize_body(d, A, gi, any ? v3{S[0], S[1], S[2]} : v3{0, 0, 0}, any ? v3{S[3], S[4], S[5]} : v3{0, 0, 0});
-    }
-}
-
-// One workgroup integrates one system (N <= kSmallMax bodies, single-thread
-// summation order) for n_steps RK12 steps with no launch per stage: thread
-// t < N takes body t, and threads kSmallMax + t the rotational half of the
-// stage update of body t (the two halves touch different fields).  With
-// `rec`, the partner data (JMain) of every body after each stage's deform is
-// recorded: entry e = 25*step + (k-1) of the launch, workgroup b, body t at
-// rec[(e*nrec_sys + b)*kSmallMax + t].
-template <int NT>
-__global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sys_ids, int n_steps,
-                                                     double dt, DtK dtk, int64_t i_step0, JMain *rec, int nrec_sys) {
-    const Acc A{d.F, d.nbp};
-    const int s = sys_ids[blockIdx.x];
-    const SysMeta sm = d.sys[s];
-    const int n = sm.n, off = sm.off, t = (int)threadIdx.x;
-    const bool valid = t < n;
-    __shared__ JDeform tdf[kSmallMax];
-    __shared__ JMain tmn[kSmallMax];
-    __shared__ double terms[NT * kSmallTerm];
-    __shared__ double sums[kSmallMax * 13];
-    __shared__ SmallDefShared dsh;
-    for (int step = 0; step < n_steps; ++step) {
-        for (int k = 1; k <= 25; ++k) {
-            const double tadd = dt * (dtk.v[k] + (double)(i_step0 + step));
-            if (valid) stage_translational_ool(d, A, off + t, k, dt, tadd);
-            else if (t >= kSmallMax && t - kSmallMax < n) stage_rotational_ool(A, off + t - kSmallMax, k, dt, dtk.v[k]);
-            __syncthreads();
-            if (valid) load_jdeform(A, tdf[t], off + t);
-            __syncthreads();
-            deform_small<NT>(A, off, n, tdf, terms, sums, dsh);
-            __syncthreads();
-            if (valid) load_jmain(A, tmn[t], off + t);
-            __syncthreads();
-            main_serial_small<NT>(d, A, off, n, tmn, terms, sums);
-            if (rec && valid) {
-                const int64_t e = 25 * (int64_t)step + (k - 1);
-                rec[(e * nrec_sys + blockIdx.x) * kSmallMax + t] = tmn[t];
-            }
-            __syncthreads();
-        }
-    }
-}
+#include "eph_small.hpp"
 
 __global__ void k_extrema(View d, int invert) {
     const Acc A{d.F, d.nbp};
@@ -2300,8 +1913,8 @@ __device__ __forceinline__ v3 particle_accel(const JMain *__restrict__ T, int nf
     for (int j = 0; j < nf; ++j) {                          // deform_by, _NK2 class
         const ddv3 rj{dd{T[j].rxh, T[j].rxl}, dd{T[j].ryh, T[j].ryl}, dd{T[j].rzh, T[j].rzl}};
         const v3 d = diff(rj, r);
-        const double rr2 = 1 / smax(dot(d, d), sR2 + T[j].sR2);
-        const double rr = sqrt(rr2);
+        double rr2, rr;
+        recip_and_root(smax(dot(d, d), sR2 + T[j].sR2), rr2, rr);
         const double tp_dphi = rr * T[j].GM;
         const double tp_dg = rr2 * tp_dphi;
         phi -= tp_dphi;
@@ -2324,8 +1937,7 @@ __device__ __forceinline__ v3 particle_accel(const JMain *__restrict__ T, int nf
         const ddv3 rp{dd{Tp.rxh, Tp.rxl}, dd{Tp.ryh, Tp.ryl}, dd{Tp.rzh, Tp.rzl}};
         PairGeo g;
         g.r = diff(r, rp);
-        g.rr2 = 1 / smax(dot(g.r, g.r), Tp.sR2 + sR2);
-        g.rr = sqrt(g.rr2);
+        recip_and_root(smax(dot(g.r, g.r), Tp.sR2 + sR2), g.rr2, g.rr);
         g.rr3 = g.rr * g.rr2;
         const m3 Cp{v3{Tp.C[0], Tp.C[1], Tp.C[2]}, v3{Tp.C[3], Tp.C[4], Tp.C[5]}, v3{Tp.C[6], Tp.C[7], Tp.C[8]}};
         da -= Tp.GM * ((g.rr3 * g.rr2 * Tp.R2) * quad_field(Cp, g));
@@ -2336,7 +1948,7 @@ __device__ __forceinline__ v3 particle_accel(const JMain *__restrict__ T, int nf
         mind = checked_max_into(mind, g.rr);
         maxi = checked_max_into(maxi, g.tp_dg);
         if (Tj.GLx != 0 || Tj.GLy != 0 || Tj.GLz != 0) {    // LENSE_THIRRING, the partner's spin
-            const double rcr32 = 2 * Tj.GM / kC * g.rr3;
+            const double rcr32 = Tj.GM2c * g.rr3;
             const v3 GLj{Tj.GLx, Tj.GLy, Tj.GLz};
             da += cross(rcr32 * (GLj - (3 * dot(GLj, g.r) * g.rr2) * g.r), g.b);
         }
@@ -2354,8 +1966,6 @@ enum PField : int { P_R = 0, P_V = 6, P_A = 12, P_MIND = 15, P_MAXI = 16, P_COUN
 // every access names its address space, so no access goes through a
 // generic pointer.
 static_assert(kPartLdsStages == 8, "the LDS share and the occupancy hint of k_particles go together");
-typedef __attribute__((address_space(3))) double lds_f64;
-typedef __attribute__((address_space(1))) double glb_f64;
 
 // n_steps > 0: advance; n_steps < 0: compute the first acceleration from
 // the records; 0: leave the workgroup's particles alone.
@@ -2555,17 +2165,35 @@ __global__ void k_unpack_particles(const double *__restrict__ in, int64_t n, int
 // ---------------------------------------------------------------------------
 void set_rk_table(const double *tab650, hipStream_t st) {
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_rk), tab650, sizeof(double) * 650, 0, hipMemcpyHostToDevice, st);
-    static int nzj[325], row0[27];
-    int e = 0;
-    for (int k = 0; k <= 25; ++k) {
-        row0[k] = e;
-        if (k == 0) continue;
-        for (int j = 0; j < k; ++j)
-            if (tab650[2 * (k * (k - 1) / 2 + j)] != 0) nzj[e++] = j;
-    }
-    row0[26] = e;
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_nzj), nzj, sizeof(nzj), 0, hipMemcpyHostToDevice, st);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_row0), row0, sizeof(row0), 0, hipMemcpyHostToDevice, st);
+    struct Tables {
+        int nzj[325] = {}, row0[27] = {}, padj[kPadCols] = {}, pad0[27] = {};
+        double padc[2 * kPadCols] = {};
+    };
+    static const Tables t = [&] {
+        Tables t;
+        int e = 0, p = 0;
+        for (int k = 0; k <= 25; ++k) {
+            t.row0[k] = e;
+            t.pad0[k] = p;
+            for (int j = 0; j < k; ++j) {
+                const double *c = tab650 + 2 * (k * (k - 1) / 2 + j);
+                if (c[0] == 0) continue;
+                t.nzj[e++] = j;
+                t.padc[2 * p] = c[0];
+                t.padc[2 * p + 1] = c[1];
+                t.padj[p++] = j;
+            }
+            for (; p & 3; ++p) t.padj[p] = t.padj[p - 1];
+        }
+        t.row0[26] = e;
+        t.pad0[26] = p;
+        return t;
+    }();
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_nzj), t.nzj, sizeof(t.nzj), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_row0), t.row0, sizeof(t.row0), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_padj), t.padj, sizeof(t.padj), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_padc), t.padc, sizeof(t.padc), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pad0), t.pad0, sizeof(t.pad0), 0, hipMemcpyHostToDevice, st);
 }
 
 void set_mass_fields(const int *field_of_slot, hipStream_t st) {
@@ -2676,18 +2304,28 @@ void launch_stage(const View &d, int k, double dt, double dt_k, double tadd, con
 void launch_step_count(int64_t *istep, hipStream_t st) {
     hipLaunchKernelGGL(k_step_count, dim3(1), dim3(64), 0, st, istep);
 }
-// 128 threads for systems of at most 16 bodies (their pairs fit one round),
-// 256 above (fewer rounds of pairs; the extra waves cost the small ones time
-// at every barrier)
-void launch_small(const View &d, const int *sys_ids, int nsys, int max_n, int n_steps, double dt, const DtK &dtk,
-                  int64_t i_step0, JMain *rec, hipStream_t st) {
+// Systems of at most 16 bodies: 256 threads (their 240 pairs in one round) and
+// the stage records in LDS; above: 512 threads and as many pairs a round as
+// the LDS left by the state holds.
+template <int NB, int NT, bool NP>
+static void launch_small_t(const View &d, const int *sys_ids, int nsys, int max_n, int n_steps, double dt, const DtK &dtk,
+                           int64_t i_step0, JMain *rec, hipStream_t st) {
+    constexpr int kLds = 160 * 1024 - 1024;              // LDS of a CU less the static share
+    constexpr int kState = 8 * NB * (S_COUNT + (NB == 16 ? 25 * kStageFields : 0)), kPair = 8 * SmallSlots<NP>::pitch;
+    const int m = max_n > 1 ? max_n - 1 : 1;
+    const int want = std::min(NT / m, max_n) * m;         // pairs of one round if the LDS allows
+    // (one pair more for the odd strides, kSmallSlack after the last)
+    const int cap = (kLds - kState) / kPair - kSmallSlack;
+    const int pairs = std::max(std::min(want + 1, cap), m + 1);
+    hipLaunchKernelGGL((k_small<NB, NT, NP>), dim3(nsys), dim3(NT), kState + (pairs + kSmallSlack) * kPair, st, d, sys_ids, n_steps, dt,
+                       dtk, i_step0, rec, nsys, pairs);
+}
+void launch_small(const View &d, const int *sys_ids, int nsys, int max_n, bool models, int n_steps, double dt,
+                  const DtK &dtk, int64_t i_step0, JMain *rec, hipStream_t st) {
     if (!nsys) return;
-    if (max_n <= 16)
-        hipLaunchKernelGGL(k_small<2 * kSmallMax>, dim3(nsys), dim3(2 * kSmallMax), 0, st, d, sys_ids, n_steps, dt, dtk,
-                           i_step0, rec, nsys);
-    else
-        hipLaunchKernelGGL(k_small<4 * kSmallMax>, dim3(nsys), dim3(4 * kSmallMax), 0, st, d, sys_ids, n_steps, dt, dtk,
-                           i_step0, rec, nsys);
+    const auto go = max_n <= 16 ? (models ? launch_small_t<16, 256, true> : launch_small_t<16, 256, false>)
+                                : (models ? launch_small_t<kSmallBodies, 512, true> : launch_small_t<kSmallBodies, 512, false>);
+    go(d, sys_ids, nsys, max_n, n_steps, dt, dtk, i_step0, rec, st);
 }
 void launch_extrema(const View &d, int invert, hipStream_t st) {
     hipLaunchKernelGGL(k_extrema, dim3((d.nb + 255) / 256), dim3(256), 0, st, d, invert);

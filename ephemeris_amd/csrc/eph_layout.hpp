@@ -64,6 +64,7 @@ struct SysMeta {
     int32_t item0, nitem;  // non-point items [item0, item0+nitem), creation order
     int32_t T;             // pooled non-point rounds (0 = none)
     int32_t serial;        // 1: single-thread summation order
+    int32_t sitem0, nsitem;  // its models' rows in View::sitems (single-thread order)
 };
 
 }  // namespace eph

@@ -60,6 +60,38 @@ EPH_HD dd div(dd x, dd y) {
 }
 EPH_HD bool finite(dd a) { return !((0 * a.hi) != 0 || (0 * a.lo) != 0); }
 
+// ---- correctly rounded pairs of reciprocal and root ----------------------------
+// q = 1 / d and s = sqrt(q), both correctly rounded.  The device takes one
+// reciprocal square root estimate for both (the division and the square root
+// of the language take one each and scale their operands): a third-order step
+// brings y = d^-1/2 to about an ulp, two residual steps give q from y^2 and
+// two give s from y, each ending on an exact residual (Markstein, IBM J. Res.
+// Dev. 34, 1990).  What those steps need -- no underflow, and no significand
+// of all ones, the one case where the last step of a reciprocal can round the
+// wrong way -- is checked in the two words of d; anything else (0, infinities
+// and NaN too) takes the language's operations.
+EPH_HD void recip_and_root(double d, double &q, double &s) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const uint32_t hi = (uint32_t)__double2hiint(d);
+    if (hi - 0x20000000u < 0x40000000u && (uint32_t)__double2loint(d) != 0xffffffffu) {
+        const double y0 = __builtin_amdgcn_rsq(d);
+        const double r = fma(-(d * y0), y0, 1.0);
+        const double y = fma(y0 * r, fma(0.375, r, 0.5), y0);
+        double p = y * y;
+        p = fma(p, fma(-d, p, 1.0), p);
+        p = fma(p, fma(-d, p, 1.0), p);
+        const double h = 0.5 * (d * y);
+        double g = fma(fma(-y, y, p), h, y);
+        g = fma(fma(-g, g, p), h, g);
+        q = p;
+        s = g;
+        return;
+    }
+#endif
+    q = 1 / d;
+    s = sqrt(q);
+}
+
 // ---- vectors ----------------------------------------------------------------
 EPH_HD v3 mkv(double x, double y, double z) { return v3{x, y, z}; }
 EPH_HD v3 operator+(v3 a, v3 b) { return v3{a.x + b.x, a.y + b.y, a.z + b.z}; }
@@ -74,6 +106,33 @@ EPH_HD v3 cross(v3 a, v3 b) {
 EPH_HD double dot(v3 a, v3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 EPH_HD v3 &operator+=(v3 &a, v3 b) { a = a + b; return a; }
 EPH_HD v3 &operator-=(v3 &a, v3 b) { a = a - b; return a; }
+
+// s = sqrt(r) and q = 1 / s, both correctly rounded: recip_and_root's steps
+// the other way round, with the same checks (on r, and on s for the final
+// reciprocal step) and the language's operations where they fail.
+EPH_HD void root_and_recip(double r, double &s, double &q) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const uint32_t hi = (uint32_t)__double2hiint(r);
+    if (hi - 0x20000000u < 0x40000000u) {
+        const double y0 = __builtin_amdgcn_rsq(r);
+        const double d = fma(-(r * y0), y0, 1.0);
+        double y = fma(y0 * d, fma(0.375, d, 0.5), y0);
+        const double h = 0.5 * y;
+        double g = r * y;
+        g = fma(fma(-g, g, r), h, g);
+        g = fma(fma(-g, g, r), h, g);
+        if ((uint32_t)__double2loint(g) != 0xffffffffu) {
+            y = fma(y, fma(-g, y, 1.0), y);
+            y = fma(y, fma(-g, y, 1.0), y);
+            s = g;
+            q = y;
+            return;
+        }
+    }
+#endif
+    s = sqrt(r);
+    q = 1 / s;
+}
 
 // hypot_t<double>::_normalize (vec_t.h:53-81): scaled for tiny/huge norms;
 // the zero vector becomes (0,0,1) for three arguments, (0,1) for two.
@@ -93,7 +152,8 @@ EPH_HD double normalize(v3 &a) {
         r = x * x + y * y + z * z;
         f = kHypMul;
     }
-    double s = sqrt(r), rs = 1 / s;
+    double s, rs;
+    root_and_recip(r, s, rs);
     a = v3{x * rs, y * rs, z * rs};
     return f == 1 ? s : f * s;
 }
@@ -207,8 +267,17 @@ EPH_HD m3 rotation_matrix(v3 w, double t, SinF sinf_) {
 EPH_HD ddv3 mkddv(v3 a) { return ddv3{mkdd(a.x), mkdd(a.y), mkdd(a.z)}; }
 EPH_HD v3 todbl(ddv3 a) { return v3{todbl(a.x), todbl(a.y), todbl(a.z)}; }
 EPH_HD ddv3 add(ddv3 a, ddv3 b) { return ddv3{add(a.x, b.x), add(a.y, b.y), add(a.z, b.z)}; }
+// todbl(sub(x, y)) without its last three operations: with r = x.hi - y.hi and
+// e its error plus x.lo - y.lo, sub returns h = r + e rounded and the exact
+// rest l (normalised operands have |e| <= |r|, or r + e is exact), and h + l
+// rounds back to h.  9 of 12 operations of every pair's separation.
+EPH_HD double diff(dd x, dd y) {
+    const double r = x.hi - y.hi, t = r - x.hi;
+    const double e = (x.hi - (r - t)) - (y.hi + t);
+    return r + (e + (x.lo - y.lo));
+}
 EPH_HD v3 diff(ddv3 a, ddv3 b) {                   // fast_mpvec(a - b)
-    return v3{todbl(sub(a.x, b.x)), todbl(sub(a.y, b.y)), todbl(sub(a.z, b.z))};
+    return v3{diff(a.x, b.x), diff(a.y, b.y), diff(a.z, b.z)};
 }
 EPH_HD ddv3 scale(dd s, ddv3 a) { return ddv3{mul(s, a.x), mul(s, a.y), mul(s, a.z)}; }
 EPH_HD ddv3 sub(ddv3 a, ddv3 b) { return ddv3{sub(a.x, b.x), sub(a.y, b.y), sub(a.z, b.z)}; }

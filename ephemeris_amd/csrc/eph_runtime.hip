@@ -212,6 +212,8 @@ int Batch::build_plan(int mode) {
         m.item0 = (int32_t)items.size();
         m.nitem = 0;
         m.T = 0;
+        m.sitem0 = (int32_t)sitems.size();
+        m.nsitem = 0;
         pl.max_n = std::max<int>(pl.max_n, (int)n);
         // msystem::accel task count, mass.cpp:226-231
         int64_t sq = (n * n + 2303) / 2304;
@@ -233,6 +235,7 @@ int Batch::build_plan(int mode) {
                     san_rows += n;
                 }
             }
+            m.nsitem = (int32_t)sitems.size() - m.sitem0;
             continue;
         }
         n_task = std::min<int64_t>(n_task, 64);
@@ -427,21 +430,21 @@ bool Batch::all_small() const {
            *std::max_element(sys_n.begin(), sys_n.end()) <= kSmallMax;
 }
 
-// Systems of at most kSmallMax bodies, all in single-thread order, can run on
-// one persistent workgroup each or on the launches of the larger systems with
-// one workgroup per body.  The persistent workgroup forms its pairs in rounds
-// and its models' fields inside them, so its stage grows with the system's
-// size and models and not with their number; the launches cost about 27 us a
-// stage and then grow with the bodies.  Measured per stage, persistent
-// against launches: 9 bodies 24 / 27 us, 16 bodies 30 / 28 us, 25 bodies 51 /
-// 27 us, 40 bodies with models 295 / 34 us, 12 with models 70 / 29 us; 25
-// bodies x 64 systems 52 / 49 us, x 128 53 / 63 us; 25 with models x 64 131 /
-// 60 us, x 256 120 / 133 us.
-constexpr int64_t kSmallLaunchBodies = 2048;
+// Systems all in single-thread order in both plans (at most 48 bodies each)
+// can run on one persistent workgroup each or on the launches of the larger
+// systems with one workgroup per body.  The persistent workgroup's stage grows
+// with the pairs of the largest system, and with its models, whose fields the
+// one workgroup forms alone; one system fills a CU.  The launches cost about
+// 27 us a stage and then grow with all the bodies.  Measured us per stage,
+// persistent / launches: 9 bodies 6.9 / 26, 16 8.8 / 26, 25 15 / 26, 32 24 /
+// 27, 48 49 / 27; with models 6 bodies 20 / 28, 16 31 / 34, 25 53 / 33, 40 88 /
+// 34; 25 bodies x 64 systems 15 / 46, x 256 15 / 98, 48 x 64 49 / 55, 9 x 500
+// 14 / 74; with models 25 x 64 53 / 60, 40 x 64 90 / 67, 40 x 200 88 / 141.
 bool Batch::use_small(int mode) const {
     if (force_generic || !(mode == 1 || plan[0].n_pool == 0) || !all_small()) return false;
-    const bool heavy = max_sys_n > 16 || plan[mode].n_sitems > 0;
-    return !(heavy && nb <= kSmallLaunchBodies);
+    const double n2 = (double)max_sys_n * max_sys_n, rounds = (double)((n_sys + 255) / 256);
+    const double persistent = rounds * (plan[mode].n_sitems > 0 ? 15 + 0.05 * n2 : 6 + 0.018 * n2);
+    return persistent <= 27 + 0.016 * (double)nb;
 }
 
 // One launch runs many steps for every system (one workgroup per system).
@@ -462,7 +465,8 @@ int Batch::integrate_small(double dt, int64_t n_step, JMain *rec, int64_t rec_st
         const int64_t ns = std::min(chunk, n_step - s0);
         {
             Scope sc(profiler, 5, stream);
-            launch_small(v, d_small_ids, (int)small_ids.size(), max_sys_n, (int)ns, dt, dtk, s0, rec, stream);
+            launch_small(v, d_small_ids, (int)small_ids.size(), max_sys_n, plan[0].n_sitems > 0, (int)ns, dt, dtk, s0,
+                         rec, stream);
         }
         if (after_chunk) after_chunk(ctx, s0, ns);
     }
@@ -734,6 +738,25 @@ int Batch::download(eph_mass *masses) {
     return EPH_OK;
 }
 
+// The constant tables of the kernels (tableau, record layout), set once per
+// device: six symbol copies cost 0.1 ms, a fifth of the creation of a small
+// system.
+static int device_tables(int dev) {
+    static std::mutex mu;
+    static std::vector<bool> done;
+    std::lock_guard<std::mutex> lk(mu);
+    if ((int)done.size() <= dev) done.resize((size_t)dev + 1, false);
+    if (done[(size_t)dev]) return EPH_OK;
+    std::vector<int> slot_field(sizeof(eph_mass) / 8, -1);
+    for (const auto &f : fields()) slot_field[f.offset / 8] = f.field;
+    set_rk_table(&kRK[0][0], 0);
+    set_mass_fields(slot_field.data(), 0);
+    HIP_CHECK(hipStreamSynchronize(0));
+    HIP_CHECK(hipGetLastError());
+    done[(size_t)dev] = true;
+    return EPH_OK;
+}
+
 int create_batch(int64_t n_sys, const int64_t *sys_n, const eph_mass *masses,
                  const eph_geopotential *gps, int64_t n_gp, const eph_ring *rings, int64_t n_ring,
                  const double *t_eph, Batch **out) {
@@ -807,13 +830,7 @@ int create_batch(int64_t n_sys, const int64_t *sys_n, const eph_mass *masses,
         b->n_work_all = (int)work_all.size();
     }
     if ((rc = dev_upload(*b, b->d_small_ids, b->small_ids))) return bail(rc);
-    set_rk_table(&kRK[0][0], b->stream);
-    static const std::vector<int> slot_field = [] {
-        std::vector<int> v(sizeof(eph_mass) / 8, -1);
-        for (const auto &f : fields()) v[f.offset / 8] = f.field;
-        return v;
-    }();
-    set_mass_fields(slot_field.data(), b->stream);
+    if ((rc = device_tables(dev))) return bail(rc);
     if ((rc = b->upload(masses))) return bail(rc);
     if (hipStreamSynchronize(b->stream) != hipSuccess) return bail(fail(EPH_EDEVICE, "stream sync failed"));
     *out = b;
@@ -917,6 +934,7 @@ int field_epoch_record(Batch *field, JMain *dst) {
         memset(&T, 0, sizeof T);
         T.rxh = m.r.x.hi; T.rxl = m.r.x.lo; T.ryh = m.r.y.hi; T.ryl = m.r.y.lo; T.rzh = m.r.z.hi; T.rzl = m.r.z.lo;
         T.GM = m.GM; T.sR2 = m.sR2;
+        T.GM2c = 2 * m.GM / kC;
         T.beta2 = m.beta2;
         T.bx = m.beta.x; T.by = m.beta.y; T.bz = m.beta.z;
         T.R2 = m.R2;
@@ -1008,7 +1026,8 @@ int integrate_particles(Particles *ps, double dt, int64_t n_step) {
         if (c >= 2) HIP_CHECK(hipStreamWaitEvent(f->stream, ps->ev_free[b], 0));
         {
             Scope sc(f->profiler, 5, f->stream);
-            launch_small(v, f->d_small_ids, (int)f->small_ids.size(), f->max_sys_n, (int)ns, dt, dtk, s0, rec, f->stream);
+            launch_small(v, f->d_small_ids, (int)f->small_ids.size(), f->max_sys_n, f->plan[0].n_sitems > 0, (int)ns, dt,
+                         dtk, s0, rec, f->stream);
         }
         HIP_CHECK(hipEventRecord(ps->ev_rec[b], f->stream));
         HIP_CHECK(hipStreamWaitEvent(ps->pstream, ps->ev_rec[b], 0));

@@ -1,0 +1,545 @@
+// One workgroup integrates one small system (device code, included by
+// eph_kernels.hip after the kernels whose helpers it shares).
+//
+// A small system's stage is bound by latency: the pair terms of 9 bodies are
+// two wavefronts' work, so what counts is the length of the dependent chain
+// from one stage to the next.  The state therefore lives in LDS for the whole
+// launch (global memory is read at its start and written at its end; the
+// stage records of systems above 16 bodies stay in global memory), every
+// phase that can is spread over pairs, components or axes, and a stage is six
+// barriers:
+//   1  stage sums, one thread per body and component
+//   2  terms of the deformation, one thread per ordered pair; the frame's two
+//      rotation matrices, one thread each
+//   3  their ordered sums, thirteen threads per body; the rotations applied,
+//      one thread per body and axis
+//   4  spin step, one thread per body (phases 2-4 repeat for constant-time-lag
+//      bodies); then, for systems with models, their fields at every partner
+//   5  terms of the main force, one thread per ordered pair
+//   6  their ordered sums, eleven threads per body, a wavefront (or two) per
+//      kind of sum
+// Pairs beyond the threads or the LDS go through 2-3 and 5-6 in rounds of
+// whole bodies.  Per stage, before (state in global memory, sums one thread
+// per chain) and now: 9 bodies 24 -> 6.9 us, 16 30 -> 8.8, 25 51 -> 15, 40 with
+// models 295 -> 88.  What bounds it now: with 9 bodies the lengths of the
+// phases (cycles: stage sums 3800, terms 2200, sums 1300, spin 3400, main terms
+// 3200, sums 2500); with 25 the two rounds of main-force terms and sums (9500
+// and 10000 of 37000), near the LDS traffic of about 77 accesses per pair.
+#pragma once
+
+// single-thread-order systems have at most 48 bodies (min(N, ceil(N^2 / 2304)) = 1)
+constexpr int kSmallBodies = 48;
+
+// fields of the LDS state, after those of the state that are kept
+enum SmallField : int {
+    S_GLD = 106,            // 3: GL rounded to double
+    S_GM2C = 109,           // 2 GM / c
+    S_X0 = 110,             // 39: step-start r, v, GL, s, w (F_X0R .. F_X0W + 2)
+    S_CW = 149,             // 3: stage sums of the spin
+    S_SUM = 152,            // 13: phi, naccel, tidal matrix sums
+    S_COUNT = 165
+};
+// LDS slot of state field f: the inertia, receptance, final phi and reaction
+// partials are not kept
+__host__ __device__ constexpr int small_slot(int f) {
+    return f < F_INERTIA ? f : f >= F_X0R ? f - F_X0R + S_X0 : f >= F_MIND ? f - F_MIND + 104 : f - F_PHIC + F_INERTIA;
+}
+static_assert(small_slot(F_EGRAD + 2) == 103 && small_slot(F_MAXI) == 105 && small_slot(F_X0W + 2) == S_CW - 1, "LDS fields");
+
+typedef __attribute__((address_space(3))) double lds_f64;
+typedef __attribute__((address_space(1))) double glb_f64;
+
+// field access of the LDS state with the names of Acc; field f is a constant
+// wherever it matters, so the slot is an immediate offset
+template <int NB>
+struct SmallAcc {
+    lds_f64 *L;
+    __device__ __forceinline__ lds_f64 &at(int slot, int g) const { return L[slot * NB + g]; }
+    __device__ __forceinline__ double ld(int f, int g) const { return at(small_slot(f), g); }
+    __device__ __forceinline__ void st(int f, int g, double v) const { at(small_slot(f), g) = v; }
+    __device__ __forceinline__ v3 ldv(int f, int g) const { return v3{ld(f, g), ld(f + 1, g), ld(f + 2, g)}; }
+    __device__ __forceinline__ void stv(int f, int g, v3 a) const { st(f, g, a.x); st(f + 1, g, a.y); st(f + 2, g, a.z); }
+    __device__ __forceinline__ m3 ldm(int f, int g) const { return m3{ldv(f, g), ldv(f + 3, g), ldv(f + 6, g)}; }
+    __device__ __forceinline__ void stm(int f, int g, const m3 &a) const { stv(f, g, a.x); stv(f + 3, g, a.y); stv(f + 6, g, a.z); }
+    __device__ __forceinline__ dd ldd(int f, int g) const { return dd{ld(f, g), ld(f + 1, g)}; }
+    __device__ __forceinline__ void std_(int f, int g, dd a) const { st(f, g, a.hi); st(f + 1, g, a.lo); }
+    __device__ __forceinline__ ddv3 lddv(int f, int g) const { return ddv3{ldd(f, g), ldd(f + 2, g), ldd(f + 4, g)}; }
+    __device__ __forceinline__ void stddv(int f, int g, ddv3 a) const { std_(f, g, a.x); std_(f + 2, g, a.y); std_(f + 4, g, a.z); }
+    __device__ __forceinline__ ddm3 lddm(int f, int g) const { return ddm3{lddv(f, g), lddv(f + 6, g), lddv(f + 12, g)}; }
+    __device__ __forceinline__ v3 ldgl(int g) const { return v3{at(S_GLD, g), at(S_GLD + 1, g), at(S_GLD + 2, g)}; }
+    __device__ __forceinline__ double ldgm2c(int g) const { return at(S_GM2C, g); }
+};
+
+// the 25 stage records of the step, 15 values each, in LDS (LR) or in the
+// body's scratch rows in global memory
+template <int NB, bool LR>
+struct SmallRec {
+    lds_f64 *l;
+    glb_f64 *g;
+    int64_t nbp;
+    __device__ __forceinline__ double ld(int j, int f, int b) const {
+        if (LR) return l[(j * kStageFields + f) * NB + b];
+        return g[(int64_t)(j * kStageFields + f) * nbp + b];
+    }
+    __device__ __forceinline__ void st(int j, int f, int b, double v) const {
+        if (LR) l[(j * kStageFields + f) * NB + b] = v;
+        else g[(int64_t)(j * kStageFields + f) * nbp + b] = v;
+    }
+};
+
+// acc += the K values p[0], p[3], ... of the pairs 0 .. cnt - 1 (S apart), one
+// dependent addition at a time in order.  The next U pairs are read before
+// this U are added; the last block's reads run past the count (kSmallSlack
+// pairs of LDS follow the last pair) and count as +0, an exact identity.
+constexpr int kSmallSlack = 8;
+template <int K, int U, int S>
+__device__ __forceinline__ void small_chain(const lds_f64 *p, int cnt, double &acc) {
+    static_assert(U <= kSmallSlack, "reads past the last pair");
+    if (cnt <= 0) return;
+    double a[K * U], b[K * U];
+    auto load = [&](double (&x)[K * U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < K; ++k) x[u * K + k] = p[u * S + 3 * k];
+        p += U * S;
+    };
+    auto sum = [&](double (&x)[K * U], int left) {
+        if (left < U) {
+#pragma unroll
+            for (int u = 1; u < U; ++u)
+#pragma unroll
+                for (int k = 0; k < K; ++k) x[u * K + k] = u < left ? x[u * K + k] : 0.0;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < K * U; ++i) acc += x[i];
+    };
+    load(a);
+    for (int left = cnt; left > 0; left -= 2 * U) {
+        if (left > U) load(b);
+        sum(a, left);
+        if (left <= U) break;
+        if (left > 2 * U) load(a);
+        sum(b, left - U);
+    }
+}
+
+// What partner q adds to body i's phi, naccel (first pass) and tidal matrix
+// sum (deform_by, mass.cpp:78-103), subtracted terms negated; w is the body's
+// spin of this pass.
+template <class A>
+__device__ __forceinline__ void small_deform_terms(const A &S, int i, int q, v3 w, bool first, lds_f64 *o) {
+    const ddv3 ri = S.lddv(F_R, i), rj = S.lddv(F_R, q);
+    const double k2 = S.ld(F_K2, i), td = S.ld(F_TD, i);
+    const v3 r = diff(rj, ri);
+    double rr2, rr;
+    recip_and_root(smax(dot(r, r), S.ld(F_SR2, i) + S.ld(F_SR2, q)), rr2, rr);
+    const double tp_dphi = rr * S.ld(F_GM, q);
+    const double tp_dg = rr2 * tp_dphi;
+    if (first) {
+        const v3 na = tp_dg * r;
+        o[0] = -tp_dphi;                                   // phi -= tp_dphi
+        o[1] = na.x; o[2] = na.y; o[3] = na.z;             // naccel += tp_dg r
+    }
+    m3 X = mzero();                                        // Csum -= X
+    if (k2 != 0 && td != 0) {                              // DAMPED_TIDAL_DEFORMATION_MATRIX
+        const v3 v = diff(S.lddv(F_V, q), S.lddv(F_V, i));
+        const double fmj = -3 * tp_dg;
+        v3 dw = rr2 * cross(r, cross(w, r) - v);
+        double dwt = normalize(dw);
+        dwt *= td * S.ld(F_TDF, q);
+        const double ecwt2 = 1 + 4 * dwt * dwt,
+                     secwt2 = sqrt(ecwt2),
+                     x0 = sqrt((1 + secwt2) / (2 * ecwt2)),
+                     y0 = dwt * sqrt(2 / (ecwt2 * (1 + secwt2))),
+                     z02 = dwt * dwt * (2 / (ecwt2 + secwt2));
+        const v3 dr = x0 * r + y0 * cross(dw, r);
+        m3 t = outer(rr2 * dr, dr) - outer(z02 * dw, dw);
+        t = adddiag(t, z02 - 1.0 / 3);
+        X = (fmj * k2) * t;
+    } else if (k2 != 0) {                                  // _NDELAY
+        const double fmj = -3 * tp_dg;
+        X = (fmj * k2) * subdiag(outer(rr2 * r, r), 1.0 / 3);
+    }
+    const double *x = &X.x.x;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) o[4 + c] = -x[c];
+}
+
+// Slots of a main-force pair (i, q): G; the own-loop daccel terms (GM dg, -LT
+// own spin, +LT partner spin, radiation, -GM field_gp, -GM field_ring); the
+// own-loop dtorque terms (GM r x dg, -LT torque, -GM r x field_gp, -GM r x
+// field_ring); the daccel reactions of outer body q on i (-GM_q dg_q, +GM_q
+// field_gp, +GM_q field_ring); 1/r; GM/r^3.  A system without models has no
+// field slots.  The pitch is odd, so pairs start in different banks.
+template <bool NP>
+struct SmallSlots {
+    static constexpr int kDa = NP ? 6 : 4, kDq = NP ? 4 : 2, kRe = NP ? 3 : 1;
+    static constexpr int da = 3, dq = da + 3 * kDa, re = dq + 3 * kDq, mx = re + 3 * kRe, pitch = (mx + 2) | 1;
+};
+
+template <bool NP, class A>
+__device__ __forceinline__ void small_pair_terms(const View &d, const A &S, int off, int i, int q, lds_f64 *o) {
+    using SL = SmallSlots<NP>;
+    const IMain I = load_imain(S, i);
+    JMain T;
+    load_jmain(S, T, q);
+    auto put = [&](int slot, v3 a) { o[slot] = a.x; o[slot + 1] = a.y; o[slot + 2] = a.z; };
+    v3 unused{0, 0, 0};
+    const PairGeo p = relativity(I, T, unused);
+    put(0, p.G);
+    const double k5 = p.rr3 * p.rr2;
+    const v3 dg = (k5 * I.R2) * quad_field(I.C, p);
+    put(SL::da, T.GM * dg);
+    put(SL::dq, T.GM * cross(p.r, dg));
+    const double rcr32 = T.GM2c * p.rr3;                   // LENSE_THIRRING, RADIATION_PRESSURE as in lt_rad
+    const v3 GLb = cross(I.GL, p.b);
+    put(SL::da + 3, -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r)));
+    put(SL::dq + 3, -(rcr32 * cross(I.GL, cross(p.r, p.b))));
+    const v3 GLj{T.GLx, T.GLy, T.GLz};
+    put(SL::da + 6, cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b));
+    v3 rad{0, 0, 0};
+    if (T.lum != 0) rad = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;   // (a dark partner's term is a zero)
+    put(SL::da + 9, rad);
+    // the reaction: outer body q visiting i, r = r_i - r_q = -p.r exactly
+    // (negation commutes with every rounding), so 1/r^2 and 1/r are the same
+    PairGeo pr = p;
+    pr.r = -p.r;
+    const m3 Cq{v3{T.C[0], T.C[1], T.C[2]}, v3{T.C[3], T.C[4], T.C[5]}, v3{T.C[6], T.C[7], T.C[8]}};
+    put(SL::re, -(T.GM * ((k5 * T.R2) * quad_field(Cq, pr))));
+    if constexpr (NP) {
+        const int gpi = d.srow_gp[off + i], rgi = d.srow_ring[off + i], gpq = d.srow_gp[off + q], rgq = d.srow_ring[off + q];
+        const v3 z{0, 0, 0};
+        const v3 a0 = gpi >= 0 ? san_at(d, gpi, q) : z, a1 = rgi >= 0 ? san_at(d, rgi, q) : z;
+        put(SL::da + 12, gpi >= 0 ? -(T.GM * a0) : z);
+        put(SL::dq + 6, gpi >= 0 ? -(T.GM * cross(p.r, a0)) : z);
+        put(SL::da + 15, rgi >= 0 ? -(T.GM * a1) : z);
+        put(SL::dq + 9, rgi >= 0 ? -(T.GM * cross(p.r, a1)) : z);
+        put(SL::re + 3, gpq >= 0 ? T.GM * san_at(d, gpq, i) : z);
+        put(SL::re + 6, rgq >= 0 ? T.GM * san_at(d, rgq, i) : z);
+    }
+    o[SL::mx] = p.rr;
+    o[SL::mx + 1] = p.tp_dg;
+}
+
+// field of model row `row` at partner jl, into its row of View::san
+template <class A>
+__device__ __forceinline__ void np_field_small(const View &d, const A &S, int off, int row, int jl) {
+    const NPItem it = d.sitems[row];
+    const int p = it.body - off;
+    v3 an{0, 0, 0};
+    if (jl != p) an = nonpoint_field_inl(d, S, p, it.kind, it.model, diff(S.lddv(F_R, jl), S.lddv(F_R, p)));
+    double *o = d.san + 3 * ((int64_t)it.an_off + jl);
+    o[0] = an.x; o[1] = an.y; o[2] = an.z;
+}
+
+// The stage sums over columns [e0, e1) of the padded table, in order: the
+// records of four columns are read together (`load` fills NV values of column
+// j), the column numbers and coefficients of the next four are fetched while
+// these are added.  Padding columns have a zero coefficient: adding their
+// exact zero changes nothing.
+template <int NV, class Load, class Add>
+__device__ __forceinline__ void small_columns(int e0, int e1, Load load, Add sum) {
+    int j[4];
+    double2 ck[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { j[u] = c_padj[e0 + u]; ck[u] = c_padc[e0 + u]; }
+    for (int e = e0; e < e1; e += 4) {
+        double x[4][NV];
+        double2 cn[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load(j[u], x[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { j[u] = c_padj[e + 4 + u]; cn[u] = c_padc[e + 4 + u]; }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { sum(ck[u], x[u]); ck[u] = cn[u]; }
+    }
+}
+
+// the state fields that are kept in LDS
+__device__ __forceinline__ bool small_kept(int f) {
+    return f < F_INERTIA || (f >= F_PHIC && f < F_IDACC) || f == F_MIND || f == F_MAXI;
+}
+
+// NB: LDS pitch (bodies), NT threads; NP: the system has geopotentials or
+// rings.  LDS: S_COUNT rows of NB, the stage records where NB == 16, then
+// `pairs` pairs of terms.  With `rec`, the partner data (JMain) of every body
+// after each stage's deform is recorded: entry e = 25*step + (k-1) of the
+// launch, workgroup b, body t at rec[(e*nrec_sys + b)*kSmallMax + t].
+template <int NB, int NT, bool NP>
+__global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sys_ids, int n_steps, double dt, DtK dtk,
+                                              int64_t i_step0, JMain *rec, int nrec_sys, int pairs) {
+    constexpr bool LR = NB == 16;
+    using SL = SmallSlots<NP>;
+    extern __shared__ double smem[];
+    lds_f64 *base = (lds_f64 *)smem;
+    const SmallAcc<NB> S{base};
+    lds_f64 *terms = base + NB * (S_COUNT + (LR ? 25 * kStageFields : 0));
+    const Acc A{d.F, d.nbp};
+    const int s = sys_ids[blockIdx.x];
+    const SysMeta sm = d.sys[s];
+    const int n = sm.n, off = sm.off, tid = (int)threadIdx.x;
+    const SmallRec<NB, LR> R{base + NB * S_COUNT, (glb_f64 *)(d.F + (int64_t)F_STAGE * d.nbp + off), d.nbp};
+    __shared__ int list[NB], n_act;
+    for (int e = tid; e < F_X0R * NB; e += NT) {
+        const int f = e / NB, b = e % NB;
+        if (b < n && small_kept(f)) S.st(f, b, A.ld(f, off + b));
+    }
+    const int m = n - 1;                                   // pairs per body
+    const int pair_i = m > 0 ? tid / m : 0, pair_q = tid - pair_i * m;     // this thread's pair of a round
+    // thread roles: (component, body) of the stage sums, (rotation, body) of the
+    // frame's two rotation matrices beside the first round's terms, (axis,
+    // body) of their application beside its sums
+    constexpr int kRole = NB == 16 ? 64 : 3 * NB;          // the rotational sums start on a wavefront of their own
+    const int cb = tid % NB;
+    constexpr int kRot0 = NT - 3 * NB;
+    const int rb = (tid - kRot0) % NB, rc = tid >= kRot0 ? (tid - kRot0) / NB : 3;
+    const int rmb = (tid - (NT - 2 * NB)) % NB, rm = tid >= NT - 2 * NB ? (tid - (NT - 2 * NB)) / NB : 2;
+    const bool has_ring = NP && tid < n && d.np_ring[off + tid] >= 0;
+    // an odd stride between bodies: their sums read different banks
+    const int stride_d = (m * 13) | 1, stride_m = (m * SL::pitch) | 1;
+    const int bpr_d = m > 0 ? min(min(NT / m, pairs * SL::pitch / stride_d), kRot0 / 13) : 1;    // bodies per round
+    const int bpr_m = m > 0 ? min(min(NT / m, pairs * SL::pitch / stride_m), NT / 12) : 1;
+    __syncthreads();
+    for (int step = 0; step < n_steps; ++step) {
+        for (int k = 1; k <= 25; ++k) {
+            const double dt_k = dtk.v[k];
+            // ---- 1: stage sums (stage_translational_c and the sums of k_stage)
+            const int e0 = c_pad0[k], e1 = c_pad0[k + 1];
+            if (tid < 3 * NB && cb < n) {
+                const int c = tid / NB, b = cb;
+                const dd v = S.ldd(F_V + 2 * c, b);
+                if (k == 1) {
+                    S.std_(F_X0R + 2 * c, b, S.ldd(F_R + 2 * c, b));
+                    S.std_(F_X0V + 2 * c, b, v);
+                }
+                const double a_now = (S.ld(F_GACC + c, b) + S.ld(F_DACC + c, b)) + S.ld(F_NACC + c, b);
+                R.st(k - 1, 2 * c, b, v.hi);
+                R.st(k - 1, 2 * c + 1, b, v.lo);
+                R.st(k - 1, 6 + c, b, a_now);
+                dd cv = mkdd(0.0);
+                double ca = 0;
+                small_columns<3>(e0, e1, [&](int j, double *x) {
+                    x[0] = R.ld(j, 2 * c, b); x[1] = R.ld(j, 2 * c + 1, b); x[2] = R.ld(j, 6 + c, b);
+                }, [&](double2 ck, const double *x) {
+                    cv = add(cv, mul(dd{ck.x, ck.y}, dd{x[0], x[1]}));
+                    ca += (ck.x + ck.y) * x[2];
+                });
+                S.std_(F_R + 2 * c, b, add(S.ldd(F_X0R + 2 * c, b), mul(mkdd(dt), cv)));
+                S.std_(F_V + 2 * c, b, add(S.ldd(F_X0V + 2 * c, b), mkdd(dt * ca)));
+                if (c == 0) {
+                    const double t = d.t0[s] + dt * (dt_k + (double)(i_step0 + step));
+                    const double gm = S.ld(F_GM0, b) + S.ld(F_DGM, b) * t;
+                    S.st(F_GM, b, gm);
+                    S.st(F_EXJ2, b, S.ld(F_DJ2, b) * t);
+                    S.at(S_GM2C, b) = 2 * gm / kC;
+                }
+            } else if (tid >= kRole && tid < kRole + 3 * NB && cb < n) {
+                const int c = (tid - kRole) / NB, b = cb;
+                if (k == 1) {
+                    S.std_(F_X0GL + 2 * c, b, S.ldd(F_GL + 2 * c, b));
+                    S.stddv(F_X0S + 6 * c, b, S.lddv(F_S + 6 * c, b));
+                    S.st(F_X0W + c, b, S.ld(F_W + c, b));
+                    S.st(F_EGRAD + c, b, S.ld(F_DTQ + c, b));
+                }
+                const double w_now = S.ld(F_W + c, b), tq_now = S.ld(F_DTQ + c, b);
+                R.st(k - 1, 9 + c, b, w_now);
+                R.st(k - 1, 12 + c, b, tq_now);
+                double cw = 0, ct = 0;
+                small_columns<2>(e0, e1, [&](int j, double *x) {
+                    x[0] = R.ld(j, 9 + c, b); x[1] = R.ld(j, 12 + c, b);
+                }, [&](double2 ck, const double *x) {
+                    const double fc = ck.x + ck.y;
+                    cw += fc * x[0];
+                    ct += fc * x[1];
+                });
+                S.std_(F_GL + 2 * c, b, add(S.ldd(F_X0GL + 2 * c, b), mkdd(dt * ct)));
+                S.at(S_CW + c, b) = cw;
+            }
+            if (tid < n) list[tid] = tid;
+            if (tid == 0) n_act = n;
+            __syncthreads();
+            // ---- 2-4: deformation and spin, pass by pass
+            for (int pass = 0; pass < 4; ++pass) {
+                const int na = n_act;
+                if (na == 0) break;
+                const bool first = pass == 0;
+                for (int b0 = 0; b0 == 0 || (m > 0 && b0 < na); b0 += bpr_d) {
+                    const int nbr = m > 0 ? min(bpr_d, na - b0) : 0;
+                    if (tid < nbr * m) {
+                        const int i = list[b0 + pair_i], qq = pair_q;
+                        const v3 w = first ? v3{S.at(S_CW, i), S.at(S_CW + 1, i), S.at(S_CW + 2, i)} / dt_k : S.ldv(F_W, i);
+                        small_deform_terms(S, i, qq < i ? qq : qq + 1, w, first, terms + pair_i * stride_d + pair_q * 13);
+                    }
+                    if (first && b0 == 0 && rm < 2 && rmb < n) {   // the two rotations of the frame (stage update)
+                        const v3 w0 = S.ldv(F_X0W, rmb);
+                        const v3 w = v3{S.at(S_CW, rmb), S.at(S_CW + 1, rmb), S.at(S_CW + 2, rmb)} / dt_k;
+                        const v3 dw = (2.0 / 3) * (w - w0);
+                        const m3 rot = rotation_matrix(rm == 0 ? w - dw : w + dw, dt * dt_k / 2, DevSin{});
+                        if (rm == 0) S.stm(F_CPOT, rmb, rot);
+                        else { S.stv(F_GACC, rmb, rot.x); S.stv(F_DACC, rmb, rot.y); S.stv(F_NACC, rmb, rot.z); }
+                    }
+                    __syncthreads();
+                    if (tid < 13 * nbr) {
+                        const int j = tid / 13, c = tid - j * 13, i = list[b0 + j];
+                        if (first || c >= 4) {
+                            double acc = 0;
+                            const lds_f64 *P = terms + j * stride_d + c;
+                            small_chain<1, 8, 13>(P, m, acc);
+                            S.at(S_SUM + c, i) = acc;
+                        }
+                    } else if (m == 0 && tid < 13) {
+                        S.at(S_SUM + tid, 0) = 0.0;        // no partner: the sums stay +0
+                    }
+                    if (first && b0 == 0 && rc < 3 && rb < n) {    // the frame's rotation, axis rc (stage_rotational)
+                        const v3 w = v3{S.at(S_CW, rb), S.at(S_CW + 1, rb), S.at(S_CW + 2, rb)} / dt_k;
+                        const m3 r0 = S.ldm(F_CPOT, rb);
+                        const m3 r1{S.ldv(F_GACC, rb), S.ldv(F_DACC, rb), S.ldv(F_NACC, rb)};
+                        ddv3 ax = S.lddv(F_X0S + 6 * rc, rb);
+                        ax = add(ax, mkddv(r0 * todbl(ax)));
+                        ax = add(ax, mkddv(r1 * todbl(ax)));
+                        if (k == 25) {
+                            const v3 egrad = egrad_k25(S.ldm(F_GI, rb), S.ldgl(rb),
+                                                       v3{R.ld(24, 9, rb), R.ld(24, 10, rb), R.ld(24, 11, rb)},
+                                                       v3{R.ld(24, 12, rb), R.ld(24, 13, rb), R.ld(24, 14, rb)},
+                                                       S.ldv(F_EGRAD, rb), dt);
+                            ax = add(ax, mkddv(rotation_matrix(egrad, 1.0 / 72, DevSin{}) * todbl(ax)));
+                        }
+                        S.stddv(F_S + 6 * rc, rb, ax);
+                        S.st(F_W + rc, rb, rc == 0 ? w.x : rc == 1 ? w.y : w.z);
+                    }
+                    __syncthreads();
+                }
+                if (first && k == 25) {                    // the last stage orthogonalises the frame and keeps Egrad
+                    if (tid < n) {
+                        const v3 eg = egrad_k25(S.ldm(F_GI, tid), S.ldgl(tid),
+                                                v3{R.ld(24, 9, tid), R.ld(24, 10, tid), R.ld(24, 11, tid)},
+                                                v3{R.ld(24, 12, tid), R.ld(24, 13, tid), R.ld(24, 14, tid)},
+                                                S.ldv(F_EGRAD, tid), dt);
+                        S.stv(F_EGRAD, tid, eg);
+                        const ddm3 f = orthogonalized(S.lddm(F_S, tid));
+                        S.stddv(F_S, tid, f.x);
+                        S.stddv(F_S + 6, tid, f.y);
+                        S.stddv(F_S + 12, tid, f.z);
+                    }
+                    __syncthreads();
+                }
+                bool again = false;
+                const int b = tid < na ? list[tid] : 0;
+                if (tid < na) {
+                    const double k2 = S.ld(F_K2, b), td = S.ld(F_TD, b);
+                    const bool damped = k2 != 0 && td != 0;
+                    auto sum = [&](int c) { return (double)S.at(S_SUM + c, b); };
+                    const m3 Csum{v3{sum(4), sum(5), sum(6)}, v3{sum(7), sum(8), sum(9)}, v3{sum(10), sum(11), sum(12)}};
+                    const Harmonics H = harmonics_load(S, b);
+                    const ddv3 GL = S.lddv(F_GL, b);
+                    v3 w = S.ldv(F_W, b);
+                    m3 C, GI;
+                    bool done = true;
+                    if (!damped) {                         // the spin iterates on the same sums
+                        int iters = 4;                     // MAX_ANGULAR_VELOCITY_ITER
+                        for (;;) {
+                            H.apply(Csum, w, C, GI);
+                            if (update_spin(S, b, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
+                        }
+                    } else {
+                        H.apply(Csum, w, C, GI);
+                        done = update_spin(S, b, GI, w, GL) || pass == 3;
+                    }
+                    again = !done;
+                    if (done) {
+                        S.stm(F_CPOT, b, C);
+                        S.stm(F_GI, b, GI);
+                        const v3 gl = todbl(S.lddv(F_GL, b));
+                        S.at(S_GLD, b) = gl.x; S.at(S_GLD + 1, b) = gl.y; S.at(S_GLD + 2, b) = gl.z;
+                    }
+                    S.stv(F_W, b, w);
+                } else if (first && tid >= 64 && tid - 64 < n) {   // PREPARE_RELATIVITY and the final naccel
+                    const int g = tid - 64;
+                    const v3 beta = todbl(S.lddv(F_V, g)) / kC;
+                    S.stv(F_BETA, g, beta);
+                    S.st(F_BETA2, g, dot(beta, beta));
+                    S.st(F_PHIC, g, S.at(S_SUM, g) / kC2);
+                    const v3 naccc = v3{S.at(S_SUM + 1, g), S.at(S_SUM + 2, g), S.at(S_SUM + 3, g)} / kC2;
+                    S.stv(F_NACCC, g, naccc);
+                    S.stv(F_NACC, g, naccc * kC2);
+                }
+                if (tid < 64) {                            // the bodies that take another pass (all in wave 0)
+                    const uint64_t mask = __ballot(again);
+                    if (again) list[__popcll(mask & ((1ull << tid) - 1))] = b;
+                    if (tid == 0) n_act = __popcll(mask);
+                }
+                __syncthreads();
+            }
+            if (NP) {                                      // fields of the models at every partner
+                for (int e = tid; e < sm.nsitem * n; e += NT) np_field_small(d, S, off, sm.sitem0 + e / n, e % n);
+                __syncthreads();
+            }
+            // ---- 5-6: main force in the single-thread order (mass.cpp:329-374)
+            if (m == 0 && tid == 0) {
+                S.stv(F_GACC, 0, v3{0, 0, 0});
+                S.stv(F_DACC, 0, v3{0, 0, 0});
+                S.stv(F_DTQ, 0, v3{0, 0, 0});
+            }
+            for (int b0 = 0; m > 0 && b0 < n; b0 += bpr_m) {
+                const int nbr = min(bpr_m, n - b0);
+                if (tid < nbr * m) {
+                    const int i = b0 + pair_i, qq = pair_q;
+                    small_pair_terms<NP>(d, S, off, i, qq < i ? qq : qq + 1,
+                                         terms + pair_i * stride_m + pair_q * SL::pitch);
+                }
+                __syncthreads();
+                // the sums of one kind on wavefronts of their own, so that none waits
+                // for another's branch
+                const int kind = tid / (NT / 4), e = tid % (NT / 4);
+                if (kind < 3 ? e < 3 * nbr : e < 2 * nbr) {
+                    const int j = kind < 3 ? e / 3 : e >> 1, c = kind < 3 ? e - 3 * j : e & 1, i = b0 + j;
+                    const lds_f64 *P = terms + j * stride_m;            // this body's pairs, q ascending
+                    double acc = 0;
+                    if (kind == 0) {                       // daccel: reactions of q < i, own loop, reactions of q > i
+                        small_chain<SL::kRe, 4, SL::pitch>(P + SL::re + c, i, acc);
+                        small_chain<SL::kDa, 4, SL::pitch>(P + SL::da + c, m, acc);
+                        small_chain<SL::kRe, 4, SL::pitch>(P + i * SL::pitch + SL::re + c, m - i, acc);
+                        S.st(F_DACC + c, i, acc);
+                    } else if (kind == 1) {                // dtorque
+                        small_chain<SL::kDq, 4, SL::pitch>(P + SL::dq + c, m, acc);
+                        S.st(F_DTQ + c, i, acc);
+                    } else if (kind == 2) {                // gaccel
+                        small_chain<1, 8, SL::pitch>(P + c, m, acc);
+                        S.st(F_GACC + c, i, acc);
+                    } else {                               // running maxima
+                        double x = S.ld(F_MIND + c, i);
+#pragma unroll 8
+                        for (int qq = 0; qq < m; ++qq) x = checked_max_into(x, P[qq * SL::pitch + SL::mx + c]);
+                        S.st(F_MIND + c, i, x);
+                    }
+                }
+                if (rec && b0 == 0 && tid >= NT - NB && tid - (NT - NB) < n) {
+                    JMain T;
+                    const int b = tid - (NT - NB);
+                    load_jmain(S, T, b);
+                    const int64_t e = 25 * (int64_t)step + (k - 1);
+                    rec[(e * nrec_sys + blockIdx.x) * kSmallMax + b] = T;
+                }
+                __syncthreads();
+            }
+            if (NP) {                                      // RING_CORRECTION of a ring host
+                if (has_ring) {
+                    v3 da = S.ldv(F_DACC, tid), dq = S.ldv(F_DTQ, tid);
+                    ring_correction(d.rings[d.np_ring[off + tid]], S.ld(F_R2, tid), S.ldgl(tid), S.ldv(F_GACC, tid),
+                                    S.ldv(F_NACC, tid), da, dq);
+                    S.stv(F_DACC, tid, da);
+                    S.stv(F_DTQ, tid, dq);
+                }
+            }
+            if (NP || m == 0) __syncthreads();
+        }
+    }
+    for (int e = tid; e < F_X0R * NB; e += NT) {
+        const int f = e / NB, b = e % NB;
+        if (b < n && small_kept(f)) A.st(f, off + b, S.ld(f, b));
+        if (b < n && f == F_PHI) A.st(F_PHI, off + b, S.ld(F_PHIC, b) * kC2);
+    }
+}

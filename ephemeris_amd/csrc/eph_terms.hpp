@@ -16,7 +16,7 @@ namespace eph {
 struct JMain {
     double rxh, rxl, ryh, ryl, rzh, rzl, GM, sR2;
     double phi, beta2, bx, by, bz, nx, ny, nz;
-    double C[9], R2, GLx, GLy, GLz, lum, pad0, pad1;
+    double C[9], R2, GLx, GLy, GLz, lum, GM2c, pad;   // GM2c: 2 GM / c, of every Lense-Thirring term
 };
 
 // own-body data of the main force
@@ -34,8 +34,7 @@ EPH_HD PairGeo relativity(const IMain &I, const JMain &T, v3 &gaccel) {
     PairGeo p;
     const ddv3 rj{dd{T.rxh, T.rxl}, dd{T.ryh, T.ryl}, dd{T.rzh, T.rzl}};
     p.r = diff(rj, I.r);
-    p.rr2 = 1 / smax(dot(p.r, p.r), I.sR2 + T.sR2);
-    p.rr = sqrt(p.rr2);
+    recip_and_root(smax(dot(p.r, p.r), I.sR2 + T.sR2), p.rr2, p.rr);
     p.rr3 = p.rr * p.rr2;
     const double tp_dphi = p.rr * T.GM;
     p.tp_dg = p.rr2 * tp_dphi;
@@ -59,7 +58,7 @@ EPH_HD v3 quad_field(const m3 &C, const PairGeo &p) {
 
 // LENSE_THIRRING (mass.impl:99-106) and RADIATION_PRESSURE (:108-109)
 EPH_HD void lt_rad(const IMain &I, const JMain &T, const PairGeo &p, v3 &da, v3 &dq) {
-    const double rcr32 = 2 * T.GM / kC * p.rr3;
+    const double rcr32 = T.GM2c * p.rr3;
     const v3 GLb = cross(I.GL, p.b);
     da -= rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r);
     dq -= rcr32 * cross(I.GL, cross(p.r, p.b));
@@ -83,7 +82,7 @@ EPH_HD PairTerms pair_terms(const IMain &I, const JMain &T) {
     o.rxdg = cross(p.r, o.dg);
     const m3 Cj{v3{T.C[0], T.C[1], T.C[2]}, v3{T.C[3], T.C[4], T.C[5]}, v3{T.C[6], T.C[7], T.C[8]}};
     o.gj = (T.GM * p.rr3 * p.rr2 * T.R2) * quad_field(Cj, p);
-    const double rcr32 = 2 * T.GM / kC * p.rr3;
+    const double rcr32 = T.GM2c * p.rr3;
     const v3 GLb = cross(I.GL, p.b);
     o.lt1 = rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r);
     o.lt2 = rcr32 * cross(I.GL, cross(p.r, p.b));
@@ -130,8 +129,8 @@ struct DeformSum {
 EPH_HD void deform_pair(int cls, const ddv3 &ri, const ddv3 &vi, double sR2i, double k2, double td, v3 w,
                         const ddv3 &rj, const ddv3 &vj, double sR2j, double GMj, double tdfj, DeformSum &s) {
     const v3 r = diff(rj, ri);
-    const double rr2 = 1 / smax(dot(r, r), sR2i + sR2j);
-    const double rr = sqrt(rr2);
+    double rr2, rr;
+    recip_and_root(smax(dot(r, r), sR2i + sR2j), rr2, rr);
     const double tp_dphi = rr * GMj;
     const double tp_dg = rr2 * tp_dphi;
     s.phi -= tp_dphi;
@@ -184,14 +183,19 @@ struct Harmonics {
 };
 
 // UPDATE_ANGULAR_VELOCITY (mass.impl:63-72); returns should_break.  When GL
-// is not finite, gl_from_w is set: the caller stores GL = GI w.
+// is not finite, gl_from_w is set: the caller stores GL = GI w.  A spin that
+// comes back unchanged ends the iteration too: every further pass would
+// repeat the same operations on the same values (a body at rest, whose
+// relative bound 1e-18 |w|^2 is zero, would otherwise take all of them).  For
+// the same reason a caller whose sums do not depend on the spin stops after
+// one step where k2r = 0.
 EPH_HD bool spin_step(const m3 &GI, v3 &w, const ddv3 &GL, bool &gl_from_w) {
     if (finite(GL)) {
         gl_from_w = false;
         const v3 oldw = w;
         w = inverse(GI) * todbl(GL);
         const v3 dwv = w - oldw;
-        return dot(dwv, dwv) < 1e-18 * dot(oldw, oldw);
+        return dot(dwv, dwv) < 1e-18 * dot(oldw, oldw) || (w.x == oldw.x && w.y == oldw.y && w.z == oldw.z);
     }
     gl_from_w = true;
     return true;
@@ -229,9 +233,9 @@ EPH_HD v3 egrad_k25(const m3 &GI, v3 GL, v3 w_now, v3 tq_now, v3 egrad, double d
 // ---------------------------------------------------------------------------
 EPH_HD v3 gp_sum(const eph_geopotential &gp, double R, v3 r) {
     double rho2 = r.x * r.x + r.y * r.y;
-    double rr2 = 1 / (rho2 + r.z * r.z);
+    double rr2, rr1;
+    recip_and_root(rho2 + r.z * r.z, rr2, rr1);
     double rho1 = sqrt(rho2);
-    double rr1 = sqrt(rr2);
     double rb1 = R * rr1;
     double rbn = rb1;
     double cphi = rho1 * rr1;

@@ -40,7 +40,33 @@ def test_accel_equals_one_thread_per_body(n, copies):
     assert not _both(_subset(n, copies), lambda g: g.accel(_lib.SUMMATION_SERIAL))
 
 
-@pytest.mark.parametrize("n,copies", [(3, 1), (17, 1), (40, 3), (48, 1)])
-def test_small_systems_integrate_alike(n, copies):
-    print(f"\n[case] {copies} x {n} bodies, 3 steps", flush=True)
-    assert not _both(_subset(n, copies), lambda g: g.integrate(300.0, 3))
+@pytest.mark.parametrize("n,copies", [(1, 1), (2, 1), (3, 1), (16, 1), (17, 1), (33, 1), (40, 3), (48, 1), (48, 60)])
+@pytest.mark.parametrize("models,lag", [(True, True), (False, True), (False, False)])
+def test_small_systems_integrate_alike(n, copies, models, lag):
+    """On the path that the library chooses (the persistent workgroup or the
+    launches), with and without models and time lags, against one thread per
+    body; the sizes are the edges of its 16- and 48-body layouts."""
+    print(f"\n[case] {copies} x {n} bodies, models {models}, time lags {lag}, 3 steps", flush=True)
+    m, sys_n, gps, rings = _subset(n, copies)
+    if not models:
+        m["gp"], m["ring"] = -1, -1
+    if not lag:
+        m["tide_delay"] = 0.0
+    assert not _both((m, sys_n, gps, rings), lambda g: g.integrate(300.0, 3))
+
+
+def test_spin_at_rest_and_undefined():
+    """Bodies without spin take one spin step instead of four, and a body
+    whose GL is not finite has it set from its spin: the bits of one thread
+    per body, persistent and in launches."""
+    print("\n[case] 12 bodies, some at rest, one with GL undefined, 3 steps", flush=True)
+    for models in (True, False):
+        m, sys_n, gps, rings = _subset(12)
+        for c in "xyz":
+            m[f"w_{c}"][3:6] = 0.0
+            for part in ("hi", "lo"):
+                m[f"GL_{c}_{part}"][3:6] = 0.0
+            m[f"GL_{c}_hi"][7] = np.nan
+        if not models:
+            m["gp"], m["ring"] = -1, -1
+        assert not _both((m, sys_n, gps, rings), lambda g: (g.accel(), g.integrate(300.0, 3)))
