@@ -696,84 +696,113 @@ __global__ __launch_bounds__(64) void k_main_k4(View d, const int2 *__restrict__
 // ---------------------------------------------------------------------------
 // latency path: one workgroup of 1-4 wavefronts per body.  Each lane
 // evaluates one partner of a 64-partner tile and leaves that pair's terms in
-// LDS; then one lane per accumulator adds them in partner order, so every
-// sum is formed exactly as in the in-order loop above.
+// LDS; then they are added in partner order, so every sum is formed exactly as
+// in the in-order loop above.
 //
 // gaccel (+G per partner) is one chain per component over the tile's G rows.
-// daccel and dtorque take up to five additions per partner, in the reference
-// order of the pair (mass.cpp:147-155, RELATIVITY .. RADIATION_PRESSURE of
-// mass.impl); slot k is one addition for each of the six lanes:
-//   slot 0  +dg (own quadrupole)         +r x dg
-//   slot 1  +gj (partner's quadrupole)    .
-//   slot 2  -LT (own spin)               -LT torque
-//   slot 3  +LT (partner's spin)          .
-//   slot 4  +radiation                    .
-// ('.' adds +0).  The lane that evaluates a partner stores only the slots
-// with a non-zero term, as consecutive six-value entries: a sum that starts
-// at +0 never holds -0 in round-to-nearest, so adding a zero of either sign
-// is an exact identity and leaving it out changes nothing (most partners
-// have no quadrupole, no spin or no luminosity, so the dependent chain that
-// bounds this kernel is shorter).  The self pair and partners past the end
-// store nothing (G: +0).  a - b is a + (-b) exactly, so subtracted terms are
-// stored negated.  The running maxima do not depend on order (ties are equal
-// values, NaN wins either way) and are reduced across the wave at the end.
+// daccel and dtorque take up to five and two additions per partner, in the
+// reference order of the pair (mass.cpp:147-155, RELATIVITY ..
+// RADIATION_PRESSURE of mass.impl): daccel +dg (own quadrupole), +gj
+// (partner's quadrupole), -LT (own spin), +LT (partner's spin), +radiation;
+// dtorque +r x dg, -LT torque.  The lane that evaluates a partner stores only
+// its non-zero terms, as consecutive entries of the tile's daccel and dtorque
+// rows: a sum that starts at +0 never holds -0 in round-to-nearest, so adding
+// a zero of either sign is an exact identity and leaving it out changes
+// nothing (most partners have no quadrupole, no spin or no luminosity, so the
+// dependent chain that bounds this kernel is shorter).  The self pair and
+// partners past the end store nothing (G: +0).  a - b is a + (-b) exactly, so
+// subtracted terms are stored negated.  The running maxima do not depend on
+// order (ties are equal values, NaN wins either way) and are reduced across
+// the wave at the end.
 // ---------------------------------------------------------------------------
-constexpr int kWpbPitch = 65;                        // G row pitch: rows start in different LDS banks
-constexpr int kWpbSlots = 5;
-constexpr int kWpbEnt = 6;                           // doubles per entry
-constexpr int kWpbEntMax = 64 * kWpbSlots + 16;      // entries of one tile, padded to a multiple of 16
-constexpr int kWpbTile = 3 * kWpbPitch + kWpbEnt * kWpbEntMax;
 
-// acc += row[0] + ... + row[63], one dependent addition at a time in index
-// order; the reads of the next sixteen values are issued before this
-// sixteen are added (the scheduling barriers keep the compiler from
-// gathering all reads ahead of one wait), so the chain does not wait for LDS.
-__device__ __forceinline__ void chain_add64(const double *row, double &acc) {
-    double b0[16], b1[16];
+// One term tile in LDS: three G rows of 64, then DA daccel and DQ dtorque
+// slots per partner, compacted, as three rows (x, y, z) each.
+template <int DA, int DQ>
+struct TermTile {
+    static constexpr int kDaRow = 64 * DA, kDqRow = 64 * DQ;
+    static constexpr int kDa = 3 * 64, kDq = kDa + 3 * kDaRow, kSize = kDq + 3 * kDqRow;
+};
+
+// Compacts one slot list into its rows, in partner and slot order, padded
+// with zeros to a multiple of sixteen entries; returns the padded count.
+template <int N>
+__device__ __forceinline__ int compact_rows(double *rows, int pitch, const v3 (&e)[N], int lane) {
+    unsigned keep = 0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) b0[i] = row[i];
+    for (int k = 0; k < N; ++k)
+        if (e[k].x != 0 || e[k].y != 0 || e[k].z != 0) keep |= 1u << k;
+    int pos = 0, total = 0;
 #pragma unroll
-    for (int q = 0; q < 64; q += 32) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) b1[i] = row[q + 16 + i];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc += b0[i];
-        if (q + 32 < 64) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) b0[i] = row[q + 32 + i];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc += b1[i];
+    for (int k = 0; k < N; ++k) {
+        const uint64_t b = __ballot((keep >> k) & 1u);
+        pos += __popcll(b & ((1ull << lane) - 1));
+        total += __popcll(b);
     }
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        if ((keep >> k) & 1u) {
+            rows[pos] = e[k].x; rows[pitch + pos] = e[k].y; rows[2 * pitch + pos] = e[k].z;
+            ++pos;
+        }
+    const int padded = (total + 15) & ~15;
+    if (lane < padded - total) {
+        rows[total + lane] = 0.0; rows[pitch + total + lane] = 0.0; rows[2 * pitch + total + lane] = 0.0;
+    }
+    return padded;
 }
-// acc += p[0] + p[S] + ... + p[(cnt - 1) * S], one dependent addition at a
-// time in index order (cnt a multiple of 16, uniform across the wave); the
-// reads of the next sixteen are issued before this sixteen are added.
-template <int S>
-__device__ __forceinline__ void chain_add_strided(const double *p, int cnt, double &acc) {
+template <int DA, int DQ>
+__device__ __forceinline__ void store_terms(double *t, int *count, const v3 &G, const v3 (&da)[DA], const v3 (&dq)[DQ],
+                                            int lane) {
+    using TT = TermTile<DA, DQ>;
+    t[lane] = G.x; t[64 + lane] = G.y; t[128 + lane] = G.z;
+    const int nd = compact_rows<DA>(t + TT::kDa, TT::kDaRow, da, lane);
+    const int nq = compact_rows<DQ>(t + TT::kDq, TT::kDqRow, dq, lane);
+    if (lane == 0) { count[0] = nd; count[1] = nq; }
+}
+
+// acc += x of lane 0, 1, ... 15 of each row of sixteen lanes, one dependent
+// addition at a time.  The multiply-add with 1.0 is the rounded sum, and its
+// operand comes from the row's lane by DPP: one LDS read per lane feeds
+// sixteen additions of up to four rows, where reading every value in every
+// lane took 16 cycles an addition (now 9, the latency of a dependent FP64
+// addition being 8).  The wait states cover a vector write of x or of the
+// execution mask right before.
+#define EPH_ROW16(OP)                                                                                             \
+    OP(0) OP(1) OP(2) OP(3) OP(4) OP(5) OP(6) OP(7) OP(8) OP(9) OP(10) OP(11) OP(12) OP(13) OP(14) OP(15)
+__device__ __forceinline__ void row_add16(double &acc, double x) {
+#define EPH_OP(N) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 4\n\t" EPH_ROW16(EPH_OP) : "+v"(acc) : "v"(x), "v"(1.0));
+#undef EPH_OP
+}
+// the same for two sums at once (their additions fill each other's latency)
+__device__ __forceinline__ void row_add16x2(double &acc0, double x0, double &acc1, double x1) {
+#define EPH_OP(N)                                                                     \
+    "v_fmac_f64_dpp %0, %2, %4 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_fmac_f64_dpp %1, %3, %4 row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 4\n\t" EPH_ROW16(EPH_OP) : "+v"(acc0), "+v"(acc1) : "v"(x0), "v"(x1), "v"(1.0));
+#undef EPH_OP
+}
+// acc += p[0], p[1], ... in order, cnt a multiple of 16 and uniform across the
+// wavefront; p is the lane's row plus its place among the row's sixteen
+// lanes.  Called with every lane of the wavefront active.
+__device__ __forceinline__ void row_chain(const double *p, int cnt, double &acc) {
     if (cnt <= 0) return;
-    double b0[16], b1[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) b0[i] = p[i * S];
-    for (int e = 0; e < cnt; e += 32) {
-        if (e + 16 < cnt) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) b1[i] = p[(e + 16 + i) * S];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc += b0[i];
-        if (e + 16 >= cnt) break;
-        if (e + 32 < cnt) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) b0[i] = p[(e + 32 + i) * S];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc += b1[i];
+    double x = p[0];
+    for (int e = 16; e < cnt; e += 16) {
+        const double next = p[e];
+        row_add16(acc, x);
+        x = next;
     }
+    row_add16(acc, x);
+}
+// a chain of cnt0 and one of cnt1 values side by side
+__device__ __forceinline__ void row_chain2(const double *p0, int cnt0, double &acc0, const double *p1, int cnt1,
+                                           double &acc1) {
+    const int both = min(cnt0, cnt1);
+    for (int e = 0; e < both; e += 16) row_add16x2(acc0, p0[e], acc1, p1[e]);
+    row_chain(p0 + both, cnt0 - both, acc0);
+    row_chain(p1 + both, cnt1 - both, acc1);
 }
 
 __device__ __forceinline__ double wave_checked_max(double x) {
@@ -783,6 +812,7 @@ __device__ __forceinline__ double wave_checked_max(double x) {
 }
 
 constexpr int kNpFusedMaxN = 512;     // systems up to this size take the fused non-point pass
+constexpr int kNpFusedMaxN4 = 1024;   // the same with four wavefronts per body
 constexpr int kNpFusedMaxItems = 64;
 
 // Non-point pass of body i inside its own workgroup (mass.cpp:283-307),
@@ -822,133 +852,153 @@ __device__ __forceinline__ void np_finalize_pre(const View &d, const Acc &A, int
 // rf, ring inputs, two own items' round sums, then per own item the
 // products of every partner (6 doubles each)
 constexpr int kNpHead = 15 * kNpFusedMaxItems + 8;
-constexpr int kNpScratch = kNpHead + 6 * kNpFusedMaxN;
+constexpr int kNpScratch = kNpHead + 6 * kNpFusedMaxN, kNpScratch4 = kNpHead + 6 * kNpFusedMaxN4;
 
+// With four wavefronts the partners go through in chunks of four tiles: the
+// first chunk's terms come from all four wavefronts, then wave 0 adds the
+// chunk's daccel entries and wave 1 its dtorque entries and G rows while waves
+// 2 and 3 evaluate the next chunk, two tiles each -- the first into the two
+// spare of six tile buffers, the second in registers until the chunk's own
+// buffers are free.  With fewer wavefronts each round of W tiles is evaluated
+// and then added.
 template <bool NP, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 1))) void k_main_wpb(View d, const int2 *__restrict__ work) {
-    static_assert(!NP || W * kWpbTile >= kNpScratch, "term tiles double as non-point scratch");
+    using TT = TermTile<5, 2>;
+    constexpr bool kPipe = W == 4;
+    constexpr int kBufs = kPipe ? 6 : W;
+    constexpr int kTerm = NP && kBufs * TT::kSize < kNpScratch ? kNpScratch : kBufs * TT::kSize;
+    static_assert(!NP || W != 4 || kTerm >= kNpScratch4, "term tiles double as non-point scratch");
     const Acc A{d.F, d.nbp};
     const int s = work[blockIdx.x].x, il = work[blockIdx.x].y;
     const SysMeta sm = d.sys[s];
     const int n = sm.n, off = sm.off, gi = off + il;
-    const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
-    __shared__ double term[W * kWpbTile];
-    __shared__ int count[W];
+    const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    __shared__ double term[kTerm];
+    __shared__ int count[2 * kBufs];
     __shared__ double wmax[2 * W];
-    __shared__ double gsum[3];
+    __shared__ double gsum[9];
     __shared__ int own_s[2];
     const IMain I = load_imain(A, gi);
     double mind0 = 0, maxi0 = 0;
     if (wv == 0) { mind0 = A.ld(F_MIND, gi); maxi0 = A.ld(F_MAXI, gi); }
     const int ring_i = NP ? d.np_ring[gi] : -1;            // read early: the tail needs it last
-    double *myg = term + wv * kWpbTile, *mye = myg + 3 * kWpbPitch;
-    double acc = 0, gacc = 0;                              // lanes 0-5 of wave 0: daccel, dtorque; gaccel
+    double acc_d = 0, acc_q = 0, acc_g = 0;                // component lane / 16 of daccel, dtorque, gaccel
     double mind = 0, maxi = 0;                             // lane-local maxima (>= +0: identities)
-    constexpr int kGWave = W > 1 ? 1 : 0;                  // the wave that adds the G chains
     // the waves that gather the non-point inputs during the last tile's chains
     constexpr int kHA = W > 2 ? 2 : W - 1, kHB = W > 3 ? 3 : kHA;
     const bool np = NP && sm.nitem > 0;
-    v3 rfv{0, 0, 0}, tdA{0, 0, 0}, tqA{0, 0, 0}, tdB{0, 0, 0}, tqB{0, 0, 0};
+    v3 rfv{0, 0, 0};
     double ring8[8];
     int own0 = -1, own1 = -1;
-    // with four wavefronts, waves 2 and 3 also form the first own item's
-    // partner products during the last chains (partners lane + 128 m of their
-    // 128 lanes; a second own item, a ring, is formed after the loop)
-    constexpr bool kPre = W == 4;
+    // with four wavefronts and at most 512 partners, waves 2 and 3 also form
+    // the first own item's partner products during the last chains (partners
+    // lane + 128 m of their 128 lanes; a second own item, a ring, is formed
+    // after the loop)
+    const bool pre = W == 4 && n <= kNpFusedMaxN;
     double P0[4][6];
-    for (int t0 = 0; t0 < n; t0 += 64 * W) {
-        const int jl = t0 + 64 * wv + lane;
-        unsigned keep = 0;
-        v3 e[2 * kWpbSlots];
-        v3 G{0, 0, 0};
+    auto evaluate = [&](int jl, v3 &G, v3 (&da)[5], v3 (&dq)[2]) {
+        G = v3{0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 5; ++k) da[k] = v3{0, 0, 0};
+        dq[0] = dq[1] = v3{0, 0, 0};
         if (jl < n && jl != il) {
             JMain T;
             load_jmain(A, T, off + jl);
             const PairTerms pt = pair_terms(I, T);
             G = pt.G;
-            e[0] = pt.dg; e[1] = pt.rxdg;
-            e[2] = pt.gj; e[3] = v3{0, 0, 0};
-            e[4] = -pt.lt1; e[5] = -pt.lt2;
-            e[6] = pt.lt3; e[7] = v3{0, 0, 0};
-            e[8] = pt.rad; e[9] = v3{0, 0, 0};
-            auto nz = [](const v3 &a) { return a.x != 0 || a.y != 0 || a.z != 0; };
-#pragma unroll
-            for (int k = 0; k < kWpbSlots; ++k)
-                if (nz(e[2 * k]) || nz(e[2 * k + 1])) keep |= 1u << k;
+            da[0] = pt.dg; da[1] = pt.gj; da[2] = -pt.lt1; da[3] = pt.lt3; da[4] = pt.rad;
+            dq[0] = pt.rxdg; dq[1] = -pt.lt2;
             mind = checked_max_into(mind, pt.rr);
             maxi = checked_max_into(maxi, pt.tp_dg);
         }
-        myg[lane] = G.x; myg[kWpbPitch + lane] = G.y; myg[2 * kWpbPitch + lane] = G.z;
-        // this tile's entries: partner order, slot order within a partner
-        int pos = 0, total = 0;
-#pragma unroll
-        for (int k = 0; k < kWpbSlots; ++k) {
-            const uint64_t b = __ballot((keep >> k) & 1u);
-            pos += __popcll(b & ((1ull << lane) - 1));
-            total += __popcll(b);
-        }
-#pragma unroll
-        for (int k = 0; k < kWpbSlots; ++k)
-            if ((keep >> k) & 1u) {
-                double *o = mye + kWpbEnt * pos++;
-                o[0] = e[2 * k].x; o[1] = e[2 * k].y; o[2] = e[2 * k].z;
-                o[3] = e[2 * k + 1].x; o[4] = e[2 * k + 1].y; o[5] = e[2 * k + 1].z;
+    };
+    int b0 = 0, b1 = 1, b2 = 2, b3 = 3, s0 = 4, s1 = 5;     // buffers of the chunk's tiles, and the spare ones
+    const int rowc = min(lane >> 4, 2), row16 = lane & 15;
+    // the chunk's ordered additions, daccel on wave 0, dtorque and gaccel on wave 1
+    auto add_chunk = [&] {
+        if (wv == 0) {
+            for (int u = 0; u < W; ++u) {
+                const int b = !kPipe ? u : u == 0 ? b0 : u == 1 ? b1 : u == 2 ? b2 : b3;
+                row_chain(term + b * TT::kSize + TT::kDa + rowc * TT::kDaRow + row16,
+                          __builtin_amdgcn_readfirstlane(count[2 * b]), acc_d);
             }
-        const int padded = (total + 15) & ~15;
-        if (lane < padded - total) {
-            double *o = mye + kWpbEnt * (total + lane);
-#pragma unroll
-            for (int c = 0; c < kWpbEnt; ++c) o[c] = 0.0;
         }
-        if (lane == 0) count[wv] = padded;
-        __syncthreads();
-        if (wv == 0 && lane < 6) {
-            for (int u = 0; u < W; ++u)
-                chain_add_strided<kWpbEnt>(term + u * kWpbTile + 3 * kWpbPitch + lane,
-                                           __builtin_amdgcn_readfirstlane(count[u]), acc);
-        }
-        if (wv == kGWave && lane < 3) {
-            const int nw = min(W, (n - t0 + 63) / 64);
-            for (int u = 0; u < nw; ++u) chain_add64(term + u * kWpbTile + lane * kWpbPitch, gacc);
-        }
-        if (np && t0 + 64 * W >= n && (wv == kHA || (kPre && wv == kHB))) {
-            int kind = -1;
-            if (lane < sm.nitem) {
-                const v3 f = np_recv_term(d, A, sm, il, gi, lane, kind);
-                if (wv == kHA) rfv = f;
+        if (wv == (W > 1 ? 1 : 0)) {
+            for (int u = 0; u < W; ++u) {
+                const int b = !kPipe ? u : u == 0 ? b0 : u == 1 ? b1 : u == 2 ? b2 : b3;
+                const double *t = term + b * TT::kSize + row16;
+                row_chain2(t + TT::kDq + rowc * TT::kDqRow, __builtin_amdgcn_readfirstlane(count[2 * b + 1]), acc_q,
+                           t + rowc * 64, 64, acc_g);      // (tiles past the end hold +0)
             }
-            const uint64_t b0 = __ballot(kind == 0), b1 = __ballot(kind == 1);
-            own0 = b0 ? __ffsll((unsigned long long)b0) - 1 : -1;
-            own1 = b1 ? __ffsll((unsigned long long)b1) - 1 : -1;
-            if (wv == kHA && lane == 0) np_finalize_pre(d, A, gi, I.phi, ring8);
-            if (kPre && own0 >= 0) {
-                const int off0 = d.items[sm.item0 + own0].an_off;
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const int jl = (wv - kHA) * 64 + lane + 128 * m;
-#pragma unroll
-                    for (int c = 0; c < 6; ++c) P0[m][c] = 0;
-                    if (jl < n && jl != il) {
-                        const int gj = off + jl;
-                        const double GMj = A.ld(F_GM, gj);
-                        const v3 rij = diff(A.lddv(F_R, gj), I.r);
-                        const double *a = d.an + 3 * ((int64_t)off0 + jl);
-                        const v3 an{a[0], a[1], a[2]};
-                        const v3 ta = GMj * an, tt = GMj * cross(rij, an);
-                        P0[m][0] = ta.x; P0[m][1] = ta.y; P0[m][2] = ta.z;
-                        P0[m][3] = tt.x; P0[m][4] = tt.y; P0[m][5] = tt.z;
-                    }
-                }
+        }
+    };
+    auto evaluate_into = [&](int jl, int b) {
+        v3 G, da[5], dq[2];
+        evaluate(jl, G, da, dq);
+        store_terms<5, 2>(term + b * TT::kSize, count + 2 * b, G, da, dq, lane);
+    };
+    evaluate_into(64 * wv + lane, wv);
+    __syncthreads();
+    for (int t1 = 64 * W; t1 < n; t1 += 64 * W) {           // t1: the next chunk
+        add_chunk();
+        if constexpr (kPipe) {
+            v3 G, da[5], dq[2];
+            if (wv >= 2) {
+                evaluate_into(t1 + 64 * (wv - 2) + lane, wv == 2 ? s0 : s1);
+                evaluate(t1 + 64 * wv + lane, G, da, dq);
             }
+            __syncthreads();
+            if (wv >= 2) {                                 // its first two tiles' buffers are free now
+                const int b = wv == 2 ? b0 : b1;
+                store_terms<5, 2>(term + b * TT::kSize, count + 2 * b, G, da, dq, lane);
+            }
+            const int o0 = b0, o1 = b1, o2 = b2, o3 = b3;
+            b0 = s0; b1 = s1; b2 = o0; b3 = o1; s0 = o2; s1 = o3;
+        } else {
+            __syncthreads();
+            evaluate_into(t1 + 64 * wv + lane, wv);
         }
         __syncthreads();
     }
+    add_chunk();
+    if (np && (wv == kHA || (pre && wv == kHB))) {
+        int kind = -1;
+        if (lane < sm.nitem) {
+            const v3 f = np_recv_term(d, A, sm, il, gi, lane, kind);
+            if (wv == kHA) rfv = f;
+        }
+        const uint64_t k0 = __ballot(kind == 0), k1 = __ballot(kind == 1);
+        own0 = k0 ? __ffsll((unsigned long long)k0) - 1 : -1;
+        own1 = k1 ? __ffsll((unsigned long long)k1) - 1 : -1;
+        if (wv == kHA && lane == 0) np_finalize_pre(d, A, gi, I.phi, ring8);
+        if (W == 4 && pre && own0 >= 0) {
+            const int off0 = d.items[sm.item0 + own0].an_off;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const int jl = (wv - kHA) * 64 + lane + 128 * m;
+#pragma unroll
+                for (int c = 0; c < 6; ++c) P0[m][c] = 0;
+                if (jl < n && jl != il) {
+                    const int gj = off + jl;
+                    const double GMj = A.ld(F_GM, gj);
+                    const v3 rij = diff(A.lddv(F_R, gj), I.r);
+                    const double *a = d.an + 3 * ((int64_t)off0 + jl);
+                    const v3 an{a[0], a[1], a[2]};
+                    const v3 ta = GMj * an, tt = GMj * cross(rij, an);
+                    P0[m][0] = ta.x; P0[m][1] = ta.y; P0[m][2] = ta.z;
+                    P0[m][3] = tt.x; P0[m][4] = tt.y; P0[m][5] = tt.z;
+                }
+            }
+        }
+    }
+    __syncthreads();
     // the non-point inputs into the (now free) tiles
     double *rf = term, *ringS = rf + 3 * kNpFusedMaxItems, *partA = ringS + 8,
            *partB = partA + 6 * kNpFusedMaxItems, *pq = term + kNpHead;
-    constexpr bool kBoth = W * kWpbTile >= kNpHead + 12 * kNpFusedMaxN;   // both own items' products at once
-    static_assert(!kPre || kBoth, "the products formed during the chains use both items' regions");
-    if (kPre && np && (wv == kHA || wv == kHB) && own0 >= 0) {
+    // both own items' products at once where they fit, else one at a time
+    const bool both = W == 4 && n <= kNpFusedMaxN;
+    static_assert(W != 4 || kTerm >= kNpHead + 12 * kNpFusedMaxN, "both items' products");
+    if (W == 4 && pre && np && (wv == kHA || wv == kHB) && own0 >= 0) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             const int jl = (wv - kHA) * 64 + lane + 128 * m;
@@ -968,12 +1018,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
         }
     }
     // gather the nine sums in lanes 0-8 of wave 0: gaccel, daccel, dtorque
-    if (wv == kGWave && lane < 3) gsum[lane] = gacc;
+    if (wv == 0 && row16 == 0 && lane < 48) gsum[3 + rowc] = acc_d;
+    if (wv == (W > 1 ? 1 : 0) && row16 == 0 && lane < 48) { gsum[rowc] = acc_g; gsum[6 + rowc] = acc_q; }
     __syncthreads();
-    if (wv == 0) {
-        const double a6 = __shfl(acc, lane >= 3 ? lane - 3 : 0, 64);
-        acc = lane < 3 ? gsum[lane] : a6;
-    }
+    double acc = wv == 0 && lane < 9 ? gsum[lane] : 0.0;
     mind = wave_checked_max(mind);
     maxi = wave_checked_max(maxi);
     if (lane == 0) { wmax[wv] = mind; wmax[W + wv] = maxi; }
@@ -985,13 +1033,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
         const int T = sm.T;
         const int tid = (int)threadIdx.x;
         const int q0 = own_s[0], q1 = own_s[1];
-        for (int pass = 0; pass < (kBoth ? 1 : 2); ++pass) {
-            const bool do0 = q0 >= 0 && (kBoth || pass == 0), do1 = q1 >= 0 && (kBoth || pass == 1);
-            const bool f0 = do0 && !kPre;          // item 0's products are formed already (kPre)
+        for (int pass = 0; pass < (both ? 1 : 2); ++pass) {
+            const bool do0 = q0 >= 0 && (both || pass == 0), do1 = q1 >= 0 && (both || pass == 1);
+            const bool f0 = do0 && !pre;           // (formed already during the last chains)
             if (f0 || do1) {
                 const int off0 = f0 ? d.items[sm.item0 + q0].an_off : 0;
                 const int off1 = do1 ? d.items[sm.item0 + q1].an_off : 0;
-                double *p0 = pq, *p1 = pq + (kBoth ? 6 * kNpFusedMaxN : 0);
+                double *p0 = pq, *p1 = pq + (both ? 6 * kNpFusedMaxN : 0);
                 for (int jl = tid; jl < n; jl += 64 * W) {
                     v3 a0{0, 0, 0}, t0v{0, 0, 0}, a1{0, 0, 0}, t1v{0, 0, 0};
                     if (jl != il) {
@@ -1023,10 +1071,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
             }
             __syncthreads();
             // item 0's rounds in wave 0, item 1's in wave 1 (both in wave 0 for one item at a time)
-            const int k2 = kBoth ? tid >> 6 : pass;
+            const int k2 = both ? tid >> 6 : pass;
             const int q = k2 == 0 ? q0 : q1;
-            if ((kBoth ? k2 < 2 : tid < 64) && q >= 0 && (kBoth || (k2 == 0 ? do0 : do1))) {
-                const double *pk = k2 == 0 ? pq : pq + (kBoth ? 6 * kNpFusedMaxN : 0);
+            if ((both ? k2 < 2 : tid < 64) && q >= 0 && (both || (k2 == 0 ? do0 : do1))) {
+                const double *pk = k2 == 0 ? pq : pq + (both ? 6 * kNpFusedMaxN : 0);
                 const int chain = d.items[sm.item0 + q].chain;
                 double *part = k2 == 0 ? partA : partB;
                 for (int u = tid & 63; u < 6 * T; u += 64) {
@@ -1040,7 +1088,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
                     part[6 * r + c] = x;
                 }
             }
-            if (!kBoth && pass == 0) __syncthreads();      // the products of item 1 overwrite item 0's
+            if (!both && pass == 0) __syncthreads();      // the products of item 1 overwrite item 0's
         }
     }
     __syncthreads();
@@ -1113,6 +1161,31 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     }
 }
 
+// acc += row[0] + ... + row[63], one dependent addition at a time in index
+// order; the reads of the next sixteen values are issued before this
+// sixteen are added (the scheduling barriers keep the compiler from
+// gathering all reads ahead of one wait), so the chain does not wait for LDS.
+__device__ __forceinline__ void chain_add64(const double *row, double &acc) {
+    double b0[16], b1[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) b0[i] = row[i];
+#pragma unroll
+    for (int q = 0; q < 64; q += 32) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) b1[i] = row[q + 16 + i];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc += b0[i];
+        if (q + 32 < 64) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) b0[i] = row[q + 32 + i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc += b1[i];
+    }
+}
+
 // deform + spin fixed point + PREPARE_RELATIVITY, one wavefront per body.
 // Accumulators: lane 0 phi, 1-3 naccel, 4-12 the tidal matrix; the
 // subtracted terms (phi, tidal matrix) are stored negated and the self pair
@@ -1120,7 +1193,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
 constexpr int kWpbDefPitch = 65;
 
 // W waves per body: in each round wave w evaluates partner chunk
-// (round * W + w); wave 0 then adds the W chunks in partner order.
+// (round * W + w); then the W chunks are added in partner order, with several
+// waves four chains on each (row_chain), with one thirteen lanes a chain each.
 // TAIL: the launch carries the non-point item fields in extra workgroups
 // (without them the kernel needs no scratch).  Work items with il < 0 are
 // padding of an XCD-dealt list.
@@ -1132,7 +1206,7 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
     if (il < 0) return;
     const SysMeta sm = d.sys[s];
     const int n = sm.n, off = sm.off, gi = off + il;
-    const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+    const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     __shared__ double sums[13];
     __shared__ int again_s;
     __shared__ double wsh[3];
@@ -1145,6 +1219,7 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
     const double sR2 = A.ld(F_SR2, gi), k2 = A.ld(F_K2, gi), td = A.ld(F_TD, gi);
     const bool damped = k2 != 0 && td != 0, ndelay = k2 != 0 && td == 0;
     const int nacc_chains = (k2 != 0) ? 13 : 4;
+    constexpr int kGroups = W == 1 ? 1 : (4 + W - 1) / W;  // groups of four chains per wavefront
     v3 w = A.ldv(F_W, gi);
     Harmonics H;
     m3 C, GI;
@@ -1172,7 +1247,10 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
     }
     bool first_pass = true;
     for (;;) {
-        double acc = (wv == 0 && lane < 4 && !first_pass) ? sums[lane] : 0.0;
+        double acc = (wv == 0 && lane < 4 && !first_pass) ? sums[lane] : 0.0;      // (one wavefront)
+        double accr[kGroups];                              // component 4 (wv + W g) + lane / 16 (several)
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) accr[g] = 0.0;
         for (int t0 = 0; t0 < n; t0 += 64 * W) {
             const int jl = t0 + 64 * wv + lane;
             double t[13];
@@ -1230,14 +1308,21 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
                 for (int q = 0; q < 13; ++q) term[wv][q * kWpbDefPitch + lane] = t[q];
             }
             __syncthreads();
-            if (wv == 0 && lane < nacc_chains && (first_pass || lane >= 4)) {
-                const int nw = min(W, (n - t0 + 63) / 64);
-                for (int u = 0; u < nw; ++u) chain_add64(term[u] + lane * kWpbDefPitch, acc);
+            const int nw = min(W, (n - t0 + 63) / 64);
+            if (W == 1) {
+                if (lane < nacc_chains && (first_pass || lane >= 4)) chain_add64(term[0] + lane * kWpbDefPitch, acc);
+            } else {
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    const int c0 = 4 * (wv + W * g);       // components c0 .. c0 + 3 on the four rows of sixteen lanes
+                    if (c0 >= nacc_chains || (c0 == 0 && !first_pass)) continue;
+                    const int c = min(c0 + (lane >> 4), 12);
+                    for (int u = 0; u < nw; ++u) row_chain(term[u] + c * kWpbDefPitch + (lane & 15), 64, accr[g]);
+                }
             }
             // the body's static harmonics in the world frame and GL (neither
-            // changes in this kernel before the spin step reads them), while
-            // wave 0 adds the first chains
-            if (W > 1 && first_pass && t0 == 0 && wv == 1 && lane == 0) {
+            // changes in this kernel before the spin step reads them)
+            if (W > 1 && first_pass && t0 == 0 && wv == W - 1 && lane == 0) {
                 Harmonics h;
                 h = harmonics_load(A, gi);
                 const ddv3 gl = A.lddv(F_GL, gi);
@@ -1251,7 +1336,15 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
             __syncthreads();
         }
         __syncthreads();
-        if (wv == 0 && lane < 13) sums[lane] = acc;        // phi, naccel: the first pass's sums, unchanged
+        if (W == 1) {
+            if (lane < 13) sums[lane] = acc;               // phi, naccel: the first pass's sums, unchanged
+        } else {
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) {
+                const int c0 = 4 * (wv + W * g), c = c0 + (lane >> 4);
+                if ((lane & 15) == 0 && c < 13 && (c0 > 0 || first_pass)) sums[c] = accr[g];
+            }
+        }
         first_pass = false;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -1430,11 +1523,9 @@ __global__ __launch_bounds__(BS) void k_main_serial(View d, const int2 *__restri
 // sequential loop: the reactions of the partners below i, the own loop over
 // every partner, the reactions of the partners above i (a tile that i splits
 // appears on both sides).  Each wavefront evaluates one tile per round, one
-// partner per lane, and leaves the non-zero terms as six-value entries
-// (daccel, dtorque) in LDS, compacted in partner and slot order as in
-// k_main_wpb; lanes 0-5 of wave 0 then add the entries of the round's tiles
-// and wave 1 the G rows of its own-loop tiles.  A reaction entry holds +0 for
-// dtorque, an exact identity in a sum that starts at +0.
+// partner per lane, and leaves the non-zero terms in a tile of LDS as in
+// k_main_wpb; wave 0 then adds the daccel entries of the round's tiles and wave
+// 1 the dtorque entries and G rows of its own-loop tiles.
 // Own-loop slots: GM dg, -LT (own spin), +LT (partner's spin), radiation,
 // -GM field_gp, -GM field_ring; reaction slots: -GM_p dg_p, +GM_p field_gp,
 // +GM_p field_ring.
@@ -1444,30 +1535,27 @@ __global__ __launch_bounds__(BS) void k_main_serial(View d, const int2 *__restri
 // 1033 us per launch one thread per body, here together with the deformation
 // and the stage update 65 us per stage (28.2 -> 1.64 ms per RK12 step); 40
 // bodies with models 7.4 -> 0.85 ms per step against the persistent workgroup.
-constexpr int kSerSlots = 6;
-constexpr int kSerEntMax = 64 * kSerSlots;           // a multiple of 16: the padding fits too
-constexpr int kSerTile = 3 * kWpbPitch + kWpbEnt * kSerEntMax;
-
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *__restrict__ work) {
     const Acc A{d.F, d.nbp};
     const int s = work[blockIdx.x].x, il = work[blockIdx.x].y;
     const SysMeta sm = d.sys[s];
     const int n = sm.n, off = sm.off, gi = off + il;
-    const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
-    __shared__ double term[W * kSerTile];
-    __shared__ int count[W];
+    using TT = TermTile<6, 4>;
+    const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    __shared__ double term[W * TT::kSize];
+    __shared__ int count[2 * W];
     __shared__ double wmax[2 * W];
-    __shared__ double gsum[3];
+    __shared__ double gsum[9];
     const IMain I = load_imain(A, gi);
     const v3 naccc = A.ldv(F_NACCC, gi);
     double mind0 = 0, maxi0 = 0;
     if (wv == 0) { mind0 = A.ld(F_MIND, gi); maxi0 = A.ld(F_MAXI, gi); }
     const int row_gp = d.san ? d.srow_gp[gi] : -1, row_ring = d.san ? d.srow_ring[gi] : -1;
     const int ring_i = d.np_ring[gi];
-    double *myg = term + wv * kSerTile, *mye = myg + 3 * kWpbPitch;
     constexpr int kGWave = W > 1 ? 1 : 0;
-    double acc = 0, gacc = 0, mind = 0, maxi = 0;
+    const int rowc = min(lane >> 4, 2), row16 = lane & 15;
+    double acc_d = 0, acc_q = 0, acc_g = 0, mind = 0, maxi = 0;
     const int tiles = (n + 63) / 64;
     const int below = (il + 63) / 64, above0 = (il + 1) / 64;
     const int own_end = below + tiles;
@@ -1477,10 +1565,11 @@ __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *
         const int kind = v < below ? 0 : v < own_end ? 1 : 2;
         const int jl = 64 * (kind == 0 ? v : kind == 1 ? v - below : above0 + v - own_end) + lane;
         const bool live = v < total_v && jl < n;
-        unsigned keep = 0;
-        v3 e[2 * kSerSlots];
+        v3 da[6], dq[4];
 #pragma unroll
-        for (int k = 0; k < 2 * kSerSlots; ++k) e[k] = v3{0, 0, 0};
+        for (int k = 0; k < 6; ++k) da[k] = v3{0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) dq[k] = v3{0, 0, 0};
         v3 G{0, 0, 0};
         if (kind == 1) {
             if (live && jl != il) {
@@ -1490,24 +1579,24 @@ __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *
                 mind = checked_max_into(mind, p.rr);
                 maxi = checked_max_into(maxi, p.tp_dg);
                 const v3 dg = (p.rr3 * p.rr2 * I.R2) * quad_field(I.C, p);
-                e[0] = T.GM * dg;
-                e[1] = T.GM * cross(p.r, dg);
+                da[0] = T.GM * dg;
+                dq[0] = T.GM * cross(p.r, dg);
                 const double rcr32 = T.GM2c * p.rr3;
                 const v3 GLb = cross(I.GL, p.b);
-                e[2] = -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r));
-                e[3] = -(rcr32 * cross(I.GL, cross(p.r, p.b)));
+                da[1] = -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r));
+                dq[1] = -(rcr32 * cross(I.GL, cross(p.r, p.b)));
                 const v3 GLj{T.GLx, T.GLy, T.GLz};
-                e[4] = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
-                e[6] = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
+                da[2] = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
+                da[3] = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
                 if (row_gp >= 0) {
                     const v3 an = san_at(d, row_gp, jl);
-                    e[8] = -(T.GM * an);
-                    e[9] = -(T.GM * cross(p.r, an));
+                    da[4] = -(T.GM * an);
+                    dq[2] = -(T.GM * cross(p.r, an));
                 }
                 if (row_ring >= 0) {
                     const v3 an = san_at(d, row_ring, jl);
-                    e[10] = -(T.GM * an);
-                    e[11] = -(T.GM * cross(p.r, an));
+                    da[5] = -(T.GM * an);
+                    dq[3] = -(T.GM * cross(p.r, an));
                 }
             }
         } else if (live && (kind == 0 ? jl < il : jl > il)) {
@@ -1524,65 +1613,42 @@ __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *
                 p.r = diff(I.r, A.lddv(F_R, gp_));
                 recip_and_root(smax(dot(p.r, p.r), A.ld(F_SR2, gp_) + I.sR2), p.rr2, p.rr);
                 p.rr3 = p.rr * p.rr2;
-                e[0] = -(GMp * ((p.rr3 * p.rr2 * R2p) * quad_field(Cp, p)));
+                da[0] = -(GMp * ((p.rr3 * p.rr2 * R2p) * quad_field(Cp, p)));
             }
-            if (rg >= 0) e[2] = GMp * san_at(d, rg, il);
-            if (rr_ >= 0) e[4] = GMp * san_at(d, rr_, il);
+            if (rg >= 0) da[1] = GMp * san_at(d, rg, il);
+            if (rr_ >= 0) da[2] = GMp * san_at(d, rr_, il);
         }
-        auto nz = [](const v3 &a) { return a.x != 0 || a.y != 0 || a.z != 0; };
-#pragma unroll
-        for (int k = 0; k < kSerSlots; ++k)
-            if (nz(e[2 * k]) || nz(e[2 * k + 1])) keep |= 1u << k;
-        myg[lane] = G.x; myg[kWpbPitch + lane] = G.y; myg[2 * kWpbPitch + lane] = G.z;
-        int pos = 0, total = 0;
-#pragma unroll
-        for (int k = 0; k < kSerSlots; ++k) {
-            const uint64_t b = __ballot((keep >> k) & 1u);
-            pos += __popcll(b & ((1ull << lane) - 1));
-            total += __popcll(b);
-        }
-#pragma unroll
-        for (int k = 0; k < kSerSlots; ++k)
-            if ((keep >> k) & 1u) {
-                double *o = mye + kWpbEnt * pos++;
-                o[0] = e[2 * k].x; o[1] = e[2 * k].y; o[2] = e[2 * k].z;
-                o[3] = e[2 * k + 1].x; o[4] = e[2 * k + 1].y; o[5] = e[2 * k + 1].z;
-            }
-        const int padded = (total + 15) & ~15;
-        if (lane < padded - total) {
-            double *o = mye + kWpbEnt * (total + lane);
-#pragma unroll
-            for (int c = 0; c < kWpbEnt; ++c) o[c] = 0.0;
-        }
-        if (lane == 0) count[wv] = padded;
+        store_terms<6, 4>(term + wv * TT::kSize, count + 2 * wv, G, da, dq, lane);
         __syncthreads();
-        if (wv == 0 && lane < 6) {
+        if (wv == 0) {
             for (int u = 0; u < W; ++u)
-                chain_add_strided<kWpbEnt>(term + u * kSerTile + 3 * kWpbPitch + lane,
-                                           __builtin_amdgcn_readfirstlane(count[u]), acc);
+                row_chain(term + u * TT::kSize + TT::kDa + rowc * TT::kDaRow + row16,
+                          __builtin_amdgcn_readfirstlane(count[2 * u]), acc_d);
         }
-        if (wv == kGWave && lane < 3) {
-            for (int u = max(0, below - v0); u < min(W, own_end - v0); ++u)
-                chain_add64(term + u * kSerTile + lane * kWpbPitch, gacc);
+        if (wv == kGWave) {
+            for (int u = 0; u < W; ++u) {
+                const double *t = term + u * TT::kSize + row16;
+                const bool own = v0 + u >= below && v0 + u < own_end;      // (reaction tiles: no G, no dtorque)
+                if (own) row_chain2(t + TT::kDq + rowc * TT::kDqRow, __builtin_amdgcn_readfirstlane(count[2 * u + 1]),
+                                    acc_q, t + rowc * 64, 64, acc_g);
+            }
         }
         __syncthreads();
     }
-    if (wv == kGWave && lane < 3) gsum[lane] = gacc;
+    if (wv == 0 && row16 == 0 && lane < 48) gsum[3 + rowc] = acc_d;
+    if (wv == kGWave && row16 == 0 && lane < 48) { gsum[rowc] = acc_g; gsum[6 + rowc] = acc_q; }
     mind = wave_checked_max(mind);
     maxi = wave_checked_max(maxi);
     if (lane == 0) { wmax[wv] = mind; wmax[W + wv] = maxi; }
     __syncthreads();
     if (wv != 0) return;
-    double v6[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) v6[k] = __shfl(acc, k, 64);
     if (lane != 0) return;
     for (int u = 0; u < W; ++u) {
         mind0 = checked_max_into(mind0, wmax[u]);
         maxi0 = checked_max_into(maxi0, wmax[W + u]);
     }
     const v3 ga{gsum[0], gsum[1], gsum[2]}, nacc = naccc * kC2;
-    v3 da{v6[0], v6[1], v6[2]}, dq{v6[3], v6[4], v6[5]};
+    v3 da{gsum[3], gsum[4], gsum[5]}, dq{gsum[6], gsum[7], gsum[8]};
     A.stv(F_GACC, gi, ga);
     A.st(F_MIND, gi, mind0);
     A.st(F_MAXI, gi, maxi0);
@@ -2240,10 +2306,13 @@ void launch_main_k4(const View &d, const int2 *blk16, int nblk, hipStream_t st) 
 // (52 KB of LDS each: three per CU): the pair terms of a 504-body system are
 // formed in two rounds instead of four (38 us instead of 44 us per launch on
 // one MI355X); the ordered sums are the same.
+int main_wpb_waves(int nwork, int max_n, int waves) {
+    if (waves) return waves;
+    return (max_n > 128 && nwork <= 1024) ? 4 : (max_n > 64 && nwork <= 1536) ? 2 : 1;
+}
 void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool fused_np, int waves, hipStream_t st) {
     if (!nwork) return;
-    int W = waves;
-    if (W == 0) W = (max_n > 128 && nwork <= 768) ? 4 : (max_n > 64 && nwork <= 1536) ? 2 : 1;
+    int W = main_wpb_waves(nwork, max_n, waves);
     if (fused_np && W == 1) W = 2;
     if (fused_np && W == 4) hipLaunchKernelGGL((k_main_wpb<true, 4>), dim3(nwork), dim3(256), 0, st, d, work);
     else if (fused_np) hipLaunchKernelGGL((k_main_wpb<true, 2>), dim3(nwork), dim3(128), 0, st, d, work);
