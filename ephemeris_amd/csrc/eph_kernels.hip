@@ -119,37 +119,87 @@ __device__ void finalize_body(const View &d, const Acc &A, int g, v3 da, v3 dq) 
     finalize_with(d, A, g, A.ldv(F_GACC, g), da, dq);
 }
 
-// Field of non-point item `row` at partner jl of its system, per unit GM of
-// the item's body (k_np_field; also run by extra workgroups of the deform
-// launches, since it needs only the stage's positions and frames).
-// Rows past the thread-pool-order items (row >= nrows) are the models of the
-// single-thread-order systems (View::sitems, written to View::san).
-__device__ __forceinline__ void np_field_one(const View &d, const Acc &A, int row, int jl, int nrows) {
-    const bool serial = row >= nrows;
-    const NPItem it = serial ? d.sitems[row - nrows] : d.items[row];
-    const SysMeta sm = d.sys[it.sys];
+__device__ __forceinline__ SysMeta sys_at(const View &d, int s) { return d.single ? d.one : d.sys[s]; }
+// the system, its data and the body of workgroup bid of a one-workgroup-per-
+// body launch
+struct BodyOf { int il; SysMeta sm; };
+__device__ __forceinline__ BodyOf body_of(const View &d, const int2 *__restrict__ work, int bid) {
+    if (d.single) return BodyOf{bid, d.one};
+    const int2 w = work[bid];
+    return BodyOf{w.y, d.sys[w.x]};
+}
+
+// Fields of the non-point items at the partners of their systems, per unit GM
+// of the item's body: one wavefront per unit, 64 partners of a geopotential,
+// or 16 partners of a ring with four lanes each that take every fourth disk (a
+// disk's transcendental chain is 5k cycles; the disks one after another were
+// the longest workgroups of the 504-body deformation launch, 41k cycles with
+// four disks).  The disks' parts are then added in order.  Units are taken
+// chunk-major, rings first, so that a row's chunks run on different CUs.
+constexpr int kRingLanes = 4, kRingPartners = 64 / kRingLanes;
+__device__ __forceinline__ void np_field_unit(const View &d, const Acc &A, int u, int max_n, int lane) {
+    const int nr = d.fring * ((max_n + kRingPartners - 1) / kRingPartners);
+    if (u < nr) {
+        const int c = u / d.fring, row = d.fgp + u - c * d.fring;
+        const NPItem it = d.fitems[row];
+        const SysMeta sm = sys_at(d, it.sys);
+        const int jl = c * kRingPartners + lane / kRingLanes, gj = sm.off + jl, part = lane % kRingLanes;
+        const bool live = jl < sm.n && gj != it.body;
+        const eph_ring &rg = d.rings[it.model];
+        const int N = (int)rg.N;
+        const double R = A.ld(F_RAD, it.body);
+        const m3 fgls = ring_frame(A.ldgl(it.body));
+        v3 r{1, 0, 0};                                     // (idle lanes: any point in the plane)
+        if (live) r = tolocal(fgls, diff(A.lddv(F_R, gj), A.lddv(F_R, it.body)));
+        const bool psign = r.z < 0;
+        if (psign) r.z = -r.z;
+        const RingGeo g = ring_geo(r);
+        v3 ret{0, 0, 0};
+        for (int i0 = 0; i0 < N; i0 += kRingLanes) {
+            v3 x{0, 0, 0};
+            if (live && i0 + part < N) x = ring_disk<DevRingTab>(rg, i0 + part, R, r, g);
+#pragma unroll
+            for (int q = 0; q < kRingLanes; ++q) {
+                const int from = (lane & ~(kRingLanes - 1)) + q;
+                const v3 y{__shfl(x.x, from, 64), __shfl(x.y, from, 64), __shfl(x.z, from, 64)};
+                if (i0 + q < N) ret += y;
+            }
+        }
+        if (psign) ret.z = -ret.z;
+        if (jl < sm.n && part == 0) {
+            const v3 an = live ? fgls * ret : v3{0, 0, 0};
+            double *o = (it.chain ? d.san : d.an) + 3 * ((int64_t)it.an_off + jl);
+            o[0] = an.x; o[1] = an.y; o[2] = an.z;
+        }
+        return;
+    }
+    u -= nr;
+    const int c = d.fgp > 0 ? u / d.fgp : 0, row = u - c * d.fgp;
+    const int jl = c * 64 + lane;
+    if (d.fgp <= 0 || c * 64 >= max_n) return;
+    const NPItem it = d.fitems[row];
+    const SysMeta sm = sys_at(d, it.sys);
     if (jl >= sm.n) return;
     const int gj = sm.off + jl;
     v3 an{0, 0, 0};
     if (gj != it.body) {
+        const m3 fmis = todbl(A.lddm(F_S, it.body));
         const v3 r = diff(A.lddv(F_R, gj), A.lddv(F_R, it.body));
-        an = nonpoint_field_inl(d, A, it.body, it.kind, it.model, r);
+        an = gp_field_world(d.gps[it.model], A.ld(F_RAD, it.body), fmis, r);
     }
-    double *o = (serial ? d.san : d.an) + 3 * ((int64_t)it.an_off + jl);
+    double *o = (it.chain ? d.san : d.an) + 3 * ((int64_t)it.an_off + jl);
     o[0] = an.x; o[1] = an.y; o[2] = an.z;
 }
 
 // Extra workgroups appended to a deform launch: each wavefront past the
-// deform workgroups covers 64 partners of one item row.  Units are taken
-// chunk-major, so the chunks of one row (a ring's are costly) run in
-// different workgroups and on different CUs.
-struct NpTail { int ndef, nrows, chunks, npool; };    // rows (npool of them thread-pool-order items), chunks of 64 partners per row
+// deform workgroups takes one unit of the item fields (which need only the
+// stage's positions and frames).
+struct NpTail { int ndef, nunits, max_n; };
 __device__ __forceinline__ bool np_tail(const View &d, const NpTail &np) {
     if ((int)blockIdx.x < np.ndef) return false;
-    if (np.nrows <= 0) return true;
-    const int u = ((int)blockIdx.x - np.ndef) * ((int)blockDim.x >> 6) + ((int)threadIdx.x >> 6);
-    const int c = u / np.nrows, row = u - c * np.nrows;
-    if (c < np.chunks) np_field_one(d, Acc{d.F, d.nbp}, row, c * 64 + ((int)threadIdx.x & 63), np.npool);
+    const int u = ((int)blockIdx.x - np.ndef) * ((int)blockDim.x >> 6) +
+                  __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (u < np.nunits) np_field_unit(d, Acc{d.F, d.nbp}, u, np.max_n, (int)threadIdx.x & 63);
     return true;
 }
 
@@ -869,8 +919,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     constexpr int kTerm = NP && kBufs * TT::kSize < kNpScratch ? kNpScratch : kBufs * TT::kSize;
     static_assert(!NP || W != 4 || kTerm >= kNpScratch4, "term tiles double as non-point scratch");
     const Acc A{d.F, d.nbp};
-    const int s = work[blockIdx.x].x, il = work[blockIdx.x].y;
-    const SysMeta sm = d.sys[s];
+    const BodyOf body = body_of(d, work, (int)blockIdx.x);
+    const int il = body.il;
+    const SysMeta sm = body.sm;
     const int n = sm.n, off = sm.off, gi = off + il;
     const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     __shared__ double term[kTerm];
@@ -1198,13 +1249,20 @@ constexpr int kWpbDefPitch = 65;
 // TAIL: the launch carries the non-point item fields in extra workgroups
 // (without them the kernel needs no scratch).  Work items with il < 0 are
 // padding of an XCD-dealt list.
-template <int W>
+template <int W, bool LISTED>
 __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__ work, int prepare, int bid,
                                                 double (*term)[13 * kWpbDefPitch]) {
     const Acc A{d.F, d.nbp};
-    const int s = work[bid].x, il = work[bid].y;
-    if (il < 0) return;
-    const SysMeta sm = d.sys[s];
+    BodyOf body;
+    if (LISTED) {                                          // not every body of the batch, with padding
+        const int2 w = work[bid];
+        if (w.y < 0) return;
+        body = BodyOf{w.y, d.sys[w.x]};
+    } else {
+        body = body_of(d, work, bid);
+    }
+    const int il = body.il;
+    const SysMeta sm = body.sm;
     const int n = sm.n, off = sm.off, gi = off + il;
     const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     __shared__ double sums[13];
@@ -1391,7 +1449,7 @@ template <int W, bool TAIL>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 3 : 1))) void k_deform_wpb(View d, const int2 *__restrict__ work, int prepare, NpTail np) {
     if (TAIL && np_tail(d, np)) return;
     __shared__ double term[W][13 * kWpbDefPitch];
-    deform_wpb_body<W>(d, work, prepare, (int)blockIdx.x, term);
+    deform_wpb_body<W, false>(d, work, prepare, (int)blockIdx.x, term);
 }
 
 // The large-batch deformation in one launch: workgroups [0, nwork) take the
@@ -1407,7 +1465,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     constexpr int kTerm = 13 * kWpbDefPitch > 64 * kDefK4Pitch ? 13 * kWpbDefPitch : 64 * kDefK4Pitch;
     __shared__ double term[kTerm];
     const int b = (int)blockIdx.x;
-    if (b < nwork) deform_wpb_body<1>(d, work, prepare, b, reinterpret_cast<double (*)[13 * kWpbDefPitch]>(term));
+    if (b < nwork) deform_wpb_body<1, true>(d, work, prepare, b, reinterpret_cast<double (*)[13 * kWpbDefPitch]>(term));
     else deform_k4_body(d, blk, prepare, b - nwork, term);
 }
 
@@ -1538,8 +1596,9 @@ __global__ __launch_bounds__(BS) void k_main_serial(View d, const int2 *__restri
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *__restrict__ work) {
     const Acc A{d.F, d.nbp};
-    const int s = work[blockIdx.x].x, il = work[blockIdx.x].y;
-    const SysMeta sm = d.sys[s];
+    const BodyOf body = body_of(d, work, (int)blockIdx.x);
+    const int il = body.il;
+    const SysMeta sm = body.sm;
     const int n = sm.n, off = sm.off, gi = off + il;
     using TT = TermTile<6, 4>;
     const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -1662,12 +1721,8 @@ __global__ __launch_bounds__(64 * W) void k_main_serial_wpb(View d, const int2 *
 // ---------------------------------------------------------------------------
 // non-point items, thread-pool order (mass.cpp:158-214, 253-307)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_np_field(View d, int nrows, int npool) {
-    // one thread per (item, partner): an = field of the item at r_j - r_p
-    const Acc A{d.F, d.nbp};
-    const int row = blockIdx.y;
-    if (row >= nrows) return;
-    np_field_one(d, A, row, blockIdx.x * blockDim.x + threadIdx.x, npool);
+__global__ __launch_bounds__(64) void k_np_field(View d, int max_n) {
+    np_field_unit(d, Acc{d.F, d.nbp}, (int)blockIdx.x, max_n, (int)threadIdx.x);
 }
 
 // one wavefront per (item, round k): the item's partial sums over the slice
@@ -2281,10 +2336,14 @@ void launch_unpack_particles(const double *in, int64_t n, int64_t npp, double *P
     hipLaunchKernelGGL(k_unpack_particles, dim3((unsigned)((npp + 255) / 256), P_COUNT), dim3(256), 0, st, in, n, npp, P);
 }
 
+// units of the item fields (np_field_unit)
+static int np_unit_count(const View &d, int max_n) {
+    return d.fring * ((max_n + kRingPartners - 1) / kRingPartners) + d.fgp * ((max_n + 63) / 64);
+}
 void launch_deform_mixed(const View &d, const int2 *work, int nwork, const int4 *blk16, int nblk, int prepare,
-                         int np_rows, int np_pool, int max_n, hipStream_t st) {
-    const NpTail np{nwork + nblk, np_rows, (max_n + 63) / 64, np_pool};
-    const int grid = nwork + nblk + np_rows * np.chunks;
+                         bool fields, int max_n, hipStream_t st) {
+    const NpTail np{nwork + nblk, fields ? np_unit_count(d, max_n) : 0, max_n};
+    const int grid = nwork + nblk + np.nunits;
     if (grid) hipLaunchKernelGGL(k_deform_mixed, dim3(grid), dim3(64), 0, st, d, work, nwork, blk16, prepare, np);
 }
 void launch_deform(const View &d, const int4 *blk_light, int n_light, const int4 *blk_damped, int n_damped,
@@ -2326,15 +2385,15 @@ void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool
 // wavefront per body).  Four, not eight, for a 504-body system: two 256-lane
 // workgroups then share each CU, one round of workgroups instead of two
 // (31 us instead of 43-58 us per launch on one MI355X).
-void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, int np_rows, int np_pool,
-                       int waves, hipStream_t st) {
-    if (!nwork && !np_rows) return;
+void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, bool fields, int waves,
+                       hipStream_t st) {
+    if (!nwork) return;
     const int chunks = (max_n + 63) / 64;
     int W = waves;
     if (W == 0) W = (chunks >= 4 && nwork <= 1280) ? 4 : (chunks >= 2 && nwork <= 2816) ? 2 : 1;
-    const NpTail np{nwork, np_rows, (max_n + 63) / 64, np_pool};
-    const dim3 grid(nwork + (np_rows * np.chunks + W - 1) / W), block(64 * W);
-    if (np_rows) {
+    const NpTail np{nwork, fields ? np_unit_count(d, max_n) : 0, max_n};
+    const dim3 grid(nwork + (np.nunits + W - 1) / W), block(64 * W);
+    if (np.nunits) {
         if (W == 4) hipLaunchKernelGGL((k_deform_wpb<4, true>), grid, block, 0, st, d, work, prepare, np);
         else if (W == 2) hipLaunchKernelGGL((k_deform_wpb<2, true>), grid, block, 0, st, d, work, prepare, np);
         else hipLaunchKernelGGL((k_deform_wpb<1, true>), grid, block, 0, st, d, work, prepare, np);
@@ -2357,13 +2416,12 @@ void launch_main_serial_wpb(const View &d, const int2 *work, int nwork, hipStrea
     else if (nwork <= 2048) hipLaunchKernelGGL(k_main_serial_wpb<2>, dim3(nwork), dim3(128), 0, st, d, work);
     else hipLaunchKernelGGL(k_main_serial_wpb<1>, dim3(nwork), dim3(64), 0, st, d, work);
 }
-void launch_np_field(const View &d, int nrows, int np_pool, int max_n, hipStream_t st) {
-    if (nrows) hipLaunchKernelGGL(k_np_field, dim3((max_n + 63) / 64, nrows), dim3(64), 0, st, d, nrows, np_pool);
+void launch_np_field(const View &d, int max_n, hipStream_t st) {
+    const int units = np_unit_count(d, max_n);
+    if (units) hipLaunchKernelGGL(k_np_field, dim3(units), dim3(64), 0, st, d, max_n);
 }
-void launch_np(const View &d, int nrows, int max_n, int maxT, const int2 *recv_blk, int nrecv, bool with_field,
-               hipStream_t st, bool with_item) {
+void launch_np(const View &d, int nrows, int maxT, const int2 *recv_blk, int nrecv, hipStream_t st, bool with_item) {
     if (!nrows) return;
-    if (with_field) launch_np_field(d, nrows, nrows, max_n, st);
     if (with_item) hipLaunchKernelGGL(k_np_item, dim3(nrows * maxT), dim3(64), 0, st, d, nrows, maxT);
     if (nrecv) hipLaunchKernelGGL(k_np_recv, dim3(nrecv), dim3(kBS), 0, st, d, recv_blk, maxT);
 }

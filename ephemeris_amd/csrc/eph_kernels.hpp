@@ -56,6 +56,14 @@ struct View {
     const int32_t *srow_gp, *srow_ring;
     double *san;
     const NPItem *sitems;        // the models behind the rows, in row order
+    // the items whose fields are formed beside the deformation, of both orders:
+    // fgp geopotentials, then fring rings
+    const NPItem *fitems;
+    int fgp, fring;
+    // a batch of one system: its data in the kernel arguments, where reading it
+    // costs no trip to memory, and every body's workgroup in index order
+    int single;
+    SysMeta one;
 };
 
 void set_rk_table(const double *tab650, hipStream_t st);
@@ -76,7 +84,7 @@ void launch_main_pool(const View &d, const int2 *blk, int nblk, hipStream_t st);
 // (system, first slot, count <= 16, 0) in the class-sorted slots) in one
 // launch, with the item fields
 void launch_deform_mixed(const View &d, const int2 *work, int nwork, const int4 *blk16, int nblk, int prepare,
-                         int np_rows, int np_pool, int max_n, hipStream_t st);
+                         bool fields, int max_n, hipStream_t st);
 // four lanes per body; blk16 = (system, first body) of every 16 bodies
 void launch_main_k4(const View &d, const int2 *blk16, int nblk, hipStream_t st);
 // the same with the items' partial sums of launch_np (rows, rounds) in extra
@@ -95,22 +103,21 @@ void launch_main_serial_wpb(const View &d, const int2 *work, int nwork, hipStrea
 // waves: wavefronts per body, 0 = chosen from the batch's shape, else 1, 2 or
 // 4 (the fused kernel has at least 2)
 void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool fused_np, int waves, hipStream_t st);
-void launch_np_field(const View &d, int nrows, int np_pool, int max_n, hipStream_t st);
+void launch_np_field(const View &d, int max_n, hipStream_t st);
 constexpr int kNpFusedMaxN_h = 512, kNpFusedMaxN4_h = 1024, kNpFusedMaxItems_h = 64;
 // wavefronts per body that launch_main_wpb takes
 int main_wpb_waves(int nwork, int max_n, int waves);
 // one workgroup of up to 4 wavefronts per body (partner chunks evaluated in
 // parallel, summed in order); max_n = largest system of the batch
-// np_rows > 0: the launch also evaluates the non-point item fields
-// (launch_np_field) in extra workgroups: np_pool thread-pool-order items, then
-// the models of the single-thread-order systems
+// fields: the launch also evaluates the non-point item fields
+// (launch_np_field) in extra workgroups
 // (waves as for launch_main_wpb)
-void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, int np_rows, int np_pool,
-                       int waves, hipStream_t st);
+void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, bool fields, int waves,
+                       hipStream_t st);
 // with_item = false: the items' partial sums were formed already
 // (launch_main_k4_items)
-void launch_np(const View &d, int nrows, int max_n, int maxT, const int2 *recv_blk, int nrecv, bool with_field,
-               hipStream_t st, bool with_item = true);
+void launch_np(const View &d, int nrows, int maxT, const int2 *recv_blk, int nrecv, hipStream_t st,
+               bool with_item = true);
 // istep: optional device step counter (graph replays); launch_step_count adds 1
 void launch_stage(const View &d, int k, double dt, double dt_k, double tadd, const int64_t *istep, hipStream_t st);
 void launch_step_count(int64_t *istep, hipStream_t st);

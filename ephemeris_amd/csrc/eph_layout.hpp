@@ -54,7 +54,7 @@ struct NPItem {
     int32_t body;      // global body index
     int32_t kind;      // 0 = geopotential, 1 = ring
     int32_t model;     // index into the geopotential or ring table
-    int32_t chain;     // chain index in the pooled non-point rounds
+    int32_t chain;     // chain index in the pooled non-point rounds (View::fitems: 1 for a single-thread-order system)
     int32_t sys;       // system
     int32_t an_off;    // offset (in bodies) of this item's row of fields
 };

@@ -27,7 +27,7 @@ constexpr size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 struct NaPlan {
     SysMeta sys;
     NPItem items[kNaMaxItems];
-    NPItem sitems[kNaMaxItems];                                   // single-thread order: each model's field rows
+    NPItem fitems[kNaMaxItems];                                   // every item or model row, geopotentials first
     int32_t srow_gp[kNaMaxBodies], srow_ring[kNaMaxBodies];
     int2 blk_main[kNaMaxBlocks], blk_recv[kNaMaxBlocks];
     int2 work[kNaMaxBodies];                                      // (system 0, body) of every body
@@ -169,6 +169,7 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
     // summation order and the non-point rounds (msystem::accel, mass.cpp:226-307)
     const int64_t n_task = std::min<int64_t>(n, (n * n + 2303) / 2304);
     const bool serial = summation == EPH_SUMMATION_SERIAL || n_task <= 1;
+    NPItem sitems[kNaMaxItems];                           // single-thread order: each model's field rows
     int n_sitems = 0;
     if (serial) {                                         // each model's field at every partner, formed first
         int32_t san_rows = 0;
@@ -177,7 +178,7 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
             for (int kind = 0; kind < 2; ++kind) {
                 const int32_t model = kind == 0 ? plan.np_gp[i] : plan.np_ring[i];
                 if (model < 0) continue;
-                plan.sitems[n_sitems++] = NPItem{(int32_t)i, kind, model, 0, 0, san_rows};
+                sitems[n_sitems++] = NPItem{(int32_t)i, kind, model, 0, 0, san_rows};
                 (kind == 0 ? plan.srow_gp : plan.srow_ring)[i] = san_rows;
                 san_rows += (int32_t)n;
             }
@@ -209,6 +210,15 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
         if (nnp)
             for (int b = 0; b < n_main; ++b) plan.blk_recv[n_recv++] = plan.blk_main[b];
     }
+    int n_f[2] = {0, 0}, nf = 0;
+    for (int kind = 0; kind < 2; ++kind)
+        for (int q = 0; q < (serial ? n_sitems : (int)nnp); ++q) {
+            NPItem it = serial ? sitems[q] : plan.items[q];
+            if (it.kind != kind) continue;
+            it.chain = serial ? 1 : 0;
+            plan.fitems[nf++] = it;
+            ++n_f[kind];
+        }
     HIP_CHECK(hipMemcpy(base + kOffPlan, &plan, sizeof plan, hipMemcpyHostToDevice));
 
     const NaPlan *dp = (const NaPlan *)(base + kOffPlan);
@@ -227,7 +237,12 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
     v.srow_gp = dp->srow_gp;
     v.srow_ring = dp->srow_ring;
     v.san = n_sitems ? (double *)(base + kOffAn) : nullptr;            // rows of at most 64 models x n partners
-    v.sitems = dp->sitems;
+    v.sitems = nullptr;                                   // (read only by the small-system kernel)
+    v.fitems = dp->fitems;
+    v.fgp = n_f[0];
+    v.fring = n_f[1];
+    v.single = 1;
+    v.one = plan.sys;
     v.an = (double *)(base + kOffAn);
     v.part = (double *)(base + kOffPart);
     v.t0 = &dp->t0;
@@ -236,13 +251,12 @@ extern "C" int eph_accel_noalloc(const eph_mass *masses, int64_t n, const eph_ge
     // the kernels of the resident path for a batch of one system: one
     // workgroup per body (the item fields in extra workgroups of the deform
     // launch), then the main force in the order asked for and the non-point pass
-    const int rows = serial ? n_sitems : (int)nnp, pool_rows = serial ? 0 : (int)nnp;
-    launch_deform_wpb(v, dp->work, (int)n, (int)n, 1, rows, pool_rows, 0, st);
+    launch_deform_wpb(v, dp->work, (int)n, (int)n, 1, nf > 0, 0, st);
     if (serial) {
         launch_main_serial_wpb(v, dp->work, (int)n, st);
     } else {
         launch_main_wpb(v, dp->work, (int)n, (int)n, false, 0, st);
-        if (nnp) launch_np(v, (int)nnp, (int)n, maxT, dp->blk_recv, n_recv, false, st);
+        if (nnp) launch_np(v, (int)nnp, maxT, dp->blk_recv, n_recv, st);
     }
     hipLaunchKernelGGL(k_na_scatter, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, v.F, v.nbp, (int)n, masses, out);
     HIP_CHECK(hipGetLastError());

@@ -279,7 +279,20 @@ int Batch::build_plan(int mode) {
         blk16 = xcd_deal(blk16, n_sys, [](int2 b) { return b.x; },
                          [&](int2 b) { return (double)sys_n[b.x]; }, make_int2(0, -1));
     }
+    // the field rows of both orders, geopotentials first
+    std::vector<NPItem> fitems;
+    pl.n_fgp = pl.n_fring = 0;
+    for (int kind = 0; kind < 2; ++kind)
+        for (const auto *list : {&items, &sitems})
+            for (NPItem it : *list) {
+                if (it.kind != kind) continue;
+                it.chain = list == &sitems ? 1 : 0;
+                fitems.push_back(it);
+                ++(kind == 0 ? pl.n_fgp : pl.n_fring);
+            }
+    pl.one = meta[0];
     int rc;
+    if ((rc = dev_upload(*this, pl.d_fitems, fitems))) return rc;
     if ((rc = dev_upload(*this, pl.d_blk16, blk16))) return rc;
     pl.n_blk16 = (int)blk16.size();
     if ((rc = dev_upload(*this, pl.d_sys, meta))) return rc;
@@ -331,6 +344,11 @@ View Batch::view(int mode) const {
     v.srow_ring = pl.d_srow_ring;
     v.san = pl.d_san;
     v.sitems = pl.d_sitems;
+    v.fitems = pl.d_fitems;
+    v.fgp = pl.n_fgp;
+    v.fring = pl.n_fring;
+    v.single = n_sys == 1 ? 1 : 0;
+    v.one = pl.one;
     v.an = pl.d_an;
     v.part = pl.d_part;
     v.t0 = d_t0;
@@ -358,14 +376,12 @@ int Batch::accel(int mode, bool prepare_only) {
     const bool wpb = use_wpb(mode);
     // the non-point item fields depend only on the stage's positions and
     // frames: they ride along in extra workgroups of the deform launch
-    // (pool items first, then the models of the single-thread-order systems)
-    const int np_rows = prepare_only ? 0 : pl.nrows + pl.n_sitems;
+    const bool fields = !prepare_only && pl.n_fgp + pl.n_fring > 0;
     bool field_done = false;
     {
         Scope sc(profiler, 1, stream);
         if (wpb) {
-            launch_deform_wpb(v, d_work_all, n_work_all, max_sys_n, prepare_only ? 0 : 1, np_rows, pl.nrows, eff_waves(),
-                              stream);
+            launch_deform_wpb(v, d_work_all, n_work_all, max_sys_n, prepare_only ? 0 : 1, fields, eff_waves(), stream);
             field_done = true;
         } else if (variant == 1) {
             launch_deform(v, d_blk_light, n_blk_light, d_blk_damped, n_blk_damped, prepare_only ? 0 : 1, stream);
@@ -374,7 +390,7 @@ int Batch::accel(int mode, bool prepare_only) {
             // one wavefront each; the rest four lanes each (that launch
             // carries the item fields)
             launch_deform_mixed(v, d_work_damped, n_work_damped, d_blk_light16, n_blk_light16,
-                                prepare_only ? 0 : 1, np_rows, pl.nrows, pl.max_n, stream);
+                                prepare_only ? 0 : 1, fields, pl.max_n, stream);
             field_done = true;
         }
     }
@@ -382,9 +398,9 @@ int Batch::accel(int mode, bool prepare_only) {
     const bool fused_np = wpb && variant != 3 &&
                           (pl.np_fusable || (pl.np_fusable4 && main_wpb_waves(pl.n_work_pool, pl.max_n, eff_waves()) == 4));
     bool items_done = false;
-    if (fused_np && pl.nrows && !field_done) {
+    if (fields && !field_done) {
         Scope sc(profiler, 4, stream);
-        launch_np_field(v, pl.nrows, pl.nrows, pl.max_n, stream);
+        launch_np_field(v, pl.max_n, stream);
     }
     if (pl.n_pool) {
         Scope sc(profiler, 2, stream);
@@ -397,18 +413,12 @@ int Batch::accel(int mode, bool prepare_only) {
     }
     if (pl.n_serial) {
         Scope sc(profiler, 3, stream);
-        if (pl.n_sitems && !field_done) {                  // the models' fields at every partner
-            View vs = v;
-            vs.items = pl.d_sitems;
-            vs.an = pl.d_san;
-            launch_np_field(vs, pl.n_sitems, pl.n_sitems, pl.max_n, stream);
-        }
         if (wpb) launch_main_serial_wpb(v, pl.d_work_serial, pl.n_work_serial, stream);
         else launch_main_serial(v, pl.d_blk_serial, pl.n_serial, stream);
     }
     if (pl.nrows && !fused_np) {
         Scope sc(profiler, 4, stream);
-        launch_np(v, pl.nrows, pl.max_n, pl.maxT, pl.d_blk_recv, pl.n_recv, !field_done, stream, !items_done);
+        launch_np(v, pl.nrows, pl.maxT, pl.d_blk_recv, pl.n_recv, stream, !items_done);
     }
     return EPH_OK;
 }

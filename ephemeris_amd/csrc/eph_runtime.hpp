@@ -60,6 +60,9 @@ struct Plan {
     int2 *d_blk16 = nullptr;         // (system, first body) of 16-body blocks, largest systems first
     int n_blk16 = 0;
     // item-field rows of the single-thread-order systems (see View::san)
+    NPItem *d_fitems = nullptr;      // every item and model row, geopotentials first (see View::fitems)
+    int n_fgp = 0, n_fring = 0;
+    SysMeta one{};                   // the first system's data
     NPItem *d_sitems = nullptr;
     int n_sitems = 0;
     int32_t *d_srow_gp = nullptr, *d_srow_ring = nullptr;

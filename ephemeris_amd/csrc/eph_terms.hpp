@@ -335,75 +335,84 @@ EPH_HD double padesum(double x, const double (&coef)[NC][2]) {
     return resn / resd;
 }
 
+// what disk i adds at offset r with r.z >= 0 (g: what every disk needs of r)
+struct RingGeo { double re2, re, rz2, r2; };
+EPH_HD RingGeo ring_geo(v3 r) {
+    RingGeo g;
+    g.re2 = r.x * r.x + r.y * r.y;
+    g.re = sqrt(g.re2);
+    g.rz2 = r.z * r.z;
+    g.r2 = g.re2 + g.rz2;
+    return g;
+}
+template <class Tab>
+EPH_HD v3 ring_disk(const eph_ring &rg, int i, double host_R, v3 r, const RingGeo &g) {
+    const double pi = kPi;
+    const double re2 = g.re2, re = g.re, rz2 = g.rz2, r2 = g.r2, rz = r.z;
+    double R = rg.R_R[i] * host_R;
+    double H = rg.H_R[i] * host_R;
+    double reR = re * R;
+    double R2 = R * R, H2, fzh = 1;
+    double k2dre = 4 / (r2 + R2 + 2 * reR);
+    if (H > 0) {
+        H2 = H * H;
+        k2dre -= H2 * (k2dre * k2dre) * (1 - k2dre * rz2) / 48;
+        fzh = (re > R ? re - R : 0);
+        fzh = 4 * (rz2 + fzh * fzh);
+        fzh = sqrt(fzh / (fzh + H2));
+    }
+    double k2 = reR * k2dre;
+    k2dre *= R2 * sqrt(k2dre);
+    double phi = atan2(rz, re - R);
+    double k = 0, lk = 0, fx;
+    bool lkh = k2 >= 0.45;
+    if (lkh) {
+        k = sqrt(k2);
+        lk = log((1 - k2) / (8 * (1 + k)));
+        fx = (Tab::xserkk(k) + lk * Tab::xserkm(k)) / (k2 * k2);
+    } else {
+        fx = Tab::xser0(k2);
+    }
+    fx *= k2dre;
+    double fz;
+    double s = sin(phi), c = cos(phi);
+    bool kh = k2 >= .5;
+    bool exphi;
+    if (kh) {
+        const double phimax = (pi / 2);
+        exphi = c > 0;
+        double ck = 1 - k2, lk2 = log(ck / 16), sk = sqrt(ck);
+        double cc = exphi ? -c : c;
+        double cphi = exphi ? pi - phi : phi;
+        fz = cphi - (s / 8) * ((lk2 * (k2 - 5) - 2 * ck) * sk + 2 * cc * (1 + lk2) * ck);
+        fz *= Tab::fz((float)((exphi ? phi : pi - phi) * (1 / phimax)), (float)(k2 * 2), 1);
+    } else {
+        const double phimax = (809. / 512);
+        exphi = phi > phimax;
+        double cr2 = exphi ? R2 + rz2 : r2;
+        double cRdr2 = (exphi ? re2 : R2) / cr2;
+        fz = (pi / 8) * (4 - 3 * cRdr2) * (rz / sqrt(cr2) * cRdr2);
+        fz *= Tab::fz((float)((exphi ? pi - phi : phi) * (1 / phimax)), (float)(k2 * 2), 0);
+    }
+    if (exphi) {
+        double ek;
+        if (lkh) ek = Tab::kserkk(k) + lk * Tab::kserkm(k);
+        else ek = Tab::kser0(k2);
+        fz = pi - 2 * sqrt(1 - k2) * ek * s - fz;
+    }
+    double Gs = rg.GsR2[i] / (host_R * host_R);
+    fx *= Gs;
+    fz *= Gs;
+    return v3{-4 * fx * r.x, -4 * fx * r.y, -2 * fz * fzh};
+}
 template <class Tab>
 EPH_HD v3 ring_sum_t(const eph_ring &rg, double host_R, v3 r) {
-    const double pi = kPi;
     bool psign = r.z < 0;
     if (psign) r.z = -r.z;
-    const double re2 = r.x * r.x + r.y * r.y;
-    const double re = sqrt(re2);
-    const double rz2 = r.z * r.z;
-    const double r2 = re2 + rz2;
-    const double rz = r.z;
+    const RingGeo g = ring_geo(r);
     v3 ret{0, 0, 0};
     const int N = (int)rg.N;
-    for (int i = 0; i < N; ++i) {
-        double R = rg.R_R[i] * host_R;
-        double H = rg.H_R[i] * host_R;
-        double reR = re * R;
-        double R2 = R * R, H2, fzh = 1;
-        double k2dre = 4 / (r2 + R2 + 2 * reR);
-        if (H > 0) {
-            H2 = H * H;
-            k2dre -= H2 * (k2dre * k2dre) * (1 - k2dre * rz2) / 48;
-            fzh = (re > R ? re - R : 0);
-            fzh = 4 * (rz2 + fzh * fzh);
-            fzh = sqrt(fzh / (fzh + H2));
-        }
-        double k2 = reR * k2dre;
-        k2dre *= R2 * sqrt(k2dre);
-        double phi = atan2(rz, re - R);
-        double k = 0, lk = 0, fx;
-        bool lkh = k2 >= 0.45;
-        if (lkh) {
-            k = sqrt(k2);
-            lk = log((1 - k2) / (8 * (1 + k)));
-            fx = (Tab::xserkk(k) + lk * Tab::xserkm(k)) / (k2 * k2);
-        } else {
-            fx = Tab::xser0(k2);
-        }
-        fx *= k2dre;
-        double fz;
-        double s = sin(phi), c = cos(phi);
-        bool kh = k2 >= .5;
-        bool exphi;
-        if (kh) {
-            const double phimax = (pi / 2);
-            exphi = c > 0;
-            double ck = 1 - k2, lk2 = log(ck / 16), sk = sqrt(ck);
-            double cc = exphi ? -c : c;
-            double cphi = exphi ? pi - phi : phi;
-            fz = cphi - (s / 8) * ((lk2 * (k2 - 5) - 2 * ck) * sk + 2 * cc * (1 + lk2) * ck);
-            fz *= Tab::fz((float)((exphi ? phi : pi - phi) * (1 / phimax)), (float)(k2 * 2), 1);
-        } else {
-            const double phimax = (809. / 512);
-            exphi = phi > phimax;
-            double cr2 = exphi ? R2 + rz2 : r2;
-            double cRdr2 = (exphi ? re2 : R2) / cr2;
-            fz = (pi / 8) * (4 - 3 * cRdr2) * (rz / sqrt(cr2) * cRdr2);
-            fz *= Tab::fz((float)((exphi ? pi - phi : phi) * (1 / phimax)), (float)(k2 * 2), 0);
-        }
-        if (exphi) {
-            double ek;
-            if (lkh) ek = Tab::kserkk(k) + lk * Tab::kserkm(k);
-            else ek = Tab::kser0(k2);
-            fz = pi - 2 * sqrt(1 - k2) * ek * s - fz;
-        }
-        double Gs = rg.GsR2[i] / (host_R * host_R);
-        fx *= Gs;
-        fz *= Gs;
-        ret += v3{-4 * fx * r.x, -4 * fx * r.y, -2 * fz * fzh};
-    }
+    for (int i = 0; i < N; ++i) ret += ring_disk<Tab>(rg, i, host_R, r, g);
     if (psign) ret.z = -ret.z;
     return ret;
 }
@@ -415,10 +424,13 @@ EPH_HD v3 gp_field_world(const eph_geopotential &gp, double R, const m3 &fmis, v
     const v3 lr = tolocal(fmis, r);
     return fmis * gp_sum(gp, R, lr);
 }
+EPH_HD m3 ring_frame(v3 migl) {
+    const v3 x = asc_node(migl), z = unit(migl);
+    return m3{x, cross(z, x), z};
+}
 template <class Tab>
 EPH_HD v3 ring_field_world(const eph_ring &rg, double R, v3 migl, v3 r) {
-    const v3 x = asc_node(migl), z = unit(migl);
-    const m3 fgls{x, cross(z, x), z};
+    const m3 fgls = ring_frame(migl);
     const v3 lr = tolocal(fgls, r);
     return fgls * ring_sum_t<Tab>(rg, R, lr);
 }
