@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace eph {
 
@@ -861,25 +862,14 @@ __device__ __forceinline__ double wave_checked_max(double x) {
     return x;
 }
 
-constexpr int kNpFusedMaxN = 512;     // systems up to this size take the fused non-point pass
-constexpr int kNpFusedMaxN4 = 1024;   // the same with four wavefronts per body
-constexpr int kNpFusedMaxItems = 64;
+constexpr int kNpFusedMaxItems = 64;   // (systems with more items take the non-point kernels)
+constexpr int kNpPreMaxN = 512;       // partners whose own-item products waves 2 and 3 form beforehand
 
 // Non-point pass of body i inside its own workgroup (mass.cpp:283-307),
 // after k_np_field has left every item's field at every partner in d.an.
 // Its inputs are gathered by spare wavefronts while wave 0 adds the last
 // tile's chains, so that only the ordered additions follow the pair loop.
 //
-// Receiver side, lane q < nitem: GM of item q's body times its field at i
-// (zero for i's own items, which the receiver sum skips).
-__device__ __forceinline__ v3 np_recv_term(const View &d, const Acc &A, const SysMeta &sm, int il, int gi, int q,
-                                           int &own_kind) {
-    const NPItem it = d.items[sm.item0 + q];
-    own_kind = it.body == gi ? it.kind : -1;
-    if (it.body == gi) return v3{0, 0, 0};
-    const double *a = d.an + 3 * ((int64_t)it.an_off + il);
-    return A.ld(F_GM, it.body) * v3{a[0], a[1], a[2]};
-}
 // FINALIZE_RELATIVITY of a body with non-point items and the inputs of its
 // RING_CORRECTION (mass.impl:133-152; finalize_with): phi and naccel are
 // final already; ring: {GM_ratio, rmGL / (rmGL + GL_R2 * R2), mGL, naccel}
@@ -899,10 +889,24 @@ __device__ __forceinline__ void np_finalize_pre(const View &d, const Acc &A, int
     }
 }
 // LDS scratch of the non-point pass (in the pair-term tiles, free by then):
-// rf, ring inputs, two own items' round sums, then per own item the
-// products of every partner (6 doubles each)
+// rf, ring inputs, two own items' round sums, then the products of an own
+// item with a block of partners (6 doubles each): all partners of up to 512
+// of both items, or blocks of 1024 with four wavefronts, of 256 and 64 below
 constexpr int kNpHead = 15 * kNpFusedMaxItems + 8;
-constexpr int kNpScratch = kNpHead + 6 * kNpFusedMaxN, kNpScratch4 = kNpHead + 6 * kNpFusedMaxN4;
+constexpr int np_block(int W) { return W == 4 ? 1024 : W == 2 ? 256 : 64; }
+
+// the larger of x and the values of the other lanes of its group of four
+__device__ __forceinline__ double quad_checked_max(double x) {
+    const int64_t a = __builtin_bit_cast(int64_t, x);
+    const int64_t a1 = __builtin_amdgcn_update_dpp(a, a, 0xb1, 0xf, 0xf, false);      // lanes 1 0 3 2
+    x = checked_max_into(x, __builtin_bit_cast(double, a1));
+    const int64_t b = __builtin_bit_cast(int64_t, x);
+    const int64_t b1 = __builtin_amdgcn_update_dpp(b, b, 0x4e, 0xf, 0xf, false);      // lanes 2 3 0 1
+    return checked_max_into(x, __builtin_bit_cast(double, b1));
+}
+
+// the terms of one pair, as they go into a tile
+struct Terms { v3 G, da[5], dq[2]; };
 
 // With four wavefronts the partners go through in chunks of four tiles: the
 // first chunk's terms come from all four wavefronts, then wave 0 adds the
@@ -916,52 +920,99 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     using TT = TermTile<5, 2>;
     constexpr bool kPipe = W == 4;
     constexpr int kBufs = kPipe ? 6 : W;
-    constexpr int kTerm = NP && kBufs * TT::kSize < kNpScratch ? kNpScratch : kBufs * TT::kSize;
-    static_assert(!NP || W != 4 || kTerm >= kNpScratch4, "term tiles double as non-point scratch");
+    constexpr int kBlock = np_block(W);
+    __shared__ double term[kBufs * TT::kSize];
+    static_assert(kBufs * TT::kSize >= kNpHead + 6 * kBlock, "term tiles double as non-point scratch");
+    static_assert(W != 4 || kBufs * TT::kSize >= kNpHead + 12 * kNpPreMaxN, "both own items' products");
     const Acc A{d.F, d.nbp};
     const BodyOf body = body_of(d, work, (int)blockIdx.x);
     const int il = body.il;
     const SysMeta sm = body.sm;
     const int n = sm.n, off = sm.off, gi = off + il;
     const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    __shared__ double term[kTerm];
     __shared__ int count[2 * kBufs];
-    __shared__ double wmax[2 * W];
+    __shared__ double mx[2][16 * W];
     __shared__ double gsum[9];
     __shared__ int own_s[2];
+    const int tid = (int)threadIdx.x;
     const IMain I = load_imain(A, gi);
+    constexpr int kMW = W > 1 ? 1 : 0;                     // the wave that ends the running maxima
     double mind0 = 0, maxi0 = 0;
-    if (wv == 0) { mind0 = A.ld(F_MIND, gi); maxi0 = A.ld(F_MAXI, gi); }
+    if (wv == kMW) { mind0 = A.ld(F_MIND, gi); maxi0 = A.ld(F_MAXI, gi); }
     const int ring_i = NP ? d.np_ring[gi] : -1;            // read early: the tail needs it last
     double acc_d = 0, acc_q = 0, acc_g = 0;                // component lane / 16 of daccel, dtorque, gaccel
     double mind = 0, maxi = 0;                             // lane-local maxima (>= +0: identities)
-    // the waves that gather the non-point inputs during the last tile's chains
+    // the waves that gather the non-point inputs
     constexpr int kHA = W > 2 ? 2 : W - 1, kHB = W > 3 ? 3 : kHA;
     const bool np = NP && sm.nitem > 0;
-    v3 rfv{0, 0, 0};
-    double ring8[8];
-    int own0 = -1, own1 = -1;
     // with four wavefronts and at most 512 partners, waves 2 and 3 also form
     // the first own item's partner products during the last chains (partners
-    // lane + 128 m of their 128 lanes; a second own item, a ring, is formed
-    // after the loop)
-    const bool pre = W == 4 && n <= kNpFusedMaxN;
-    double P0[4][6];
-    auto evaluate = [&](int jl, v3 &G, v3 (&da)[5], v3 (&dq)[2]) {
-        G = v3{0, 0, 0};
+    // lane + 128 m of their 128 lanes)
+    const bool pre = W == 4 && n <= kNpPreMaxN;
+    double P0[4][6], ring8[8];
+    int own0 = -1, own1 = -1;
+    // Receiver side, lane q < nitem of wave kHA: GM of item q's body and its
+    // field at i (i's own items are skipped by the receiver sum); read here,
+    // used after the last chain
+    double rgm = 0;
+    v3 ran{0, 0, 0};
+    if (np && (wv == kHA || wv == kHB)) {
+        int kind = -1;
+        if (lane < sm.nitem) {
+            const NPItem it = d.items[sm.item0 + lane];
+            if (it.body == gi) kind = it.kind;
+            else if (wv == kHA) {
+                const double *a = d.an + 3 * ((int64_t)it.an_off + il);
+                ran = v3{a[0], a[1], a[2]};
+                rgm = A.ld(F_GM, it.body);
+            }
+        }
+        const uint64_t k0 = __ballot(kind == 0), k1 = __ballot(kind == 1);
+        own0 = k0 ? __ffsll((unsigned long long)k0) - 1 : -1;
+        own1 = k1 ? __ffsll((unsigned long long)k1) - 1 : -1;
+    }
+    // The terms of K partners per lane, without branches, so that their chains
+    // fill each other's latency.  A lane without a partner (the self pair, past
+    // the end) takes the body itself at distance 1 with no mass and no light:
+    // all its terms are zeros.
+    auto evaluate = [&](auto count, const int (&jls)[decltype(count)::value], Terms (&o)[decltype(count)::value]) {
+        constexpr int K = decltype(count)::value;
+        JMain T[K];
+        PairGeo p[K];
+        double dist[K];
+        bool have[K], safe = true;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) da[k] = v3{0, 0, 0};
-        dq[0] = dq[1] = v3{0, 0, 0};
-        if (jl < n && jl != il) {
-            JMain T;
-            load_jmain(A, T, off + jl);
-            const PairTerms pt = pair_terms(I, T);
-            G = pt.G;
-            da[0] = pt.dg; da[1] = pt.gj; da[2] = -pt.lt1; da[3] = pt.lt3; da[4] = pt.rad;
-            dq[0] = pt.rxdg; dq[1] = -pt.lt2;
-            mind = checked_max_into(mind, pt.rr);
+        for (int k = 0; k < K; ++k) {
+            have[k] = jls[k] < n && jls[k] != il;
+            load_jmain(A, T[k], off + (have[k] ? jls[k] : il));
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (!have[k]) T[k].GM = T[k].GM2c = T[k].lum = 0.0;
+            const double d2 = pair_offset(I, T[k], p[k].r);
+            dist[k] = have[k] ? d2 : 1.0;
+            safe = safe && recip_and_root_safe(dist[k]);
+            recip_and_root_fast(dist[k], p[k].rr2, p[k].rr);
+        }
+        if (!safe) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                p[k].rr2 = 1 / dist[k];
+                p[k].rr = sqrt(p[k].rr2);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const PairTerms pt = pair_terms_from(I, T[k], p[k]);
+            o[k].G = pt.G;
+            o[k].da[0] = pt.dg; o[k].da[1] = pt.gj; o[k].da[2] = -pt.lt1; o[k].da[3] = pt.lt3; o[k].da[4] = pt.rad;
+            o[k].dq[0] = pt.rxdg; o[k].dq[1] = -pt.lt2;
+            mind = checked_max_into(mind, have[k] ? pt.rr : 0.0);
             maxi = checked_max_into(maxi, pt.tp_dg);
         }
+    };
+    auto store = [&](int b, const Terms &o) {
+        store_terms<5, 2>(term + b * TT::kSize, count + 2 * b, o.G, o.da, o.dq, lane);
     };
     int b0 = 0, b1 = 1, b2 = 2, b3 = 3, s0 = 4, s1 = 5;     // buffers of the chunk's tiles, and the spare ones
     const int rowc = min(lane >> 4, 2), row16 = lane & 15;
@@ -983,44 +1034,42 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
             }
         }
     };
-    auto evaluate_into = [&](int jl, int b) {
-        v3 G, da[5], dq[2];
-        evaluate(jl, G, da, dq);
-        store_terms<5, 2>(term + b * TT::kSize, count + 2 * b, G, da, dq, lane);
-    };
-    evaluate_into(64 * wv + lane, wv);
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    Terms o1[1];
+    {
+        const int jl[1] = {64 * wv + lane};
+        evaluate(One{}, jl, o1);
+        store(wv, o1[0]);
+    }
     __syncthreads();
     for (int t1 = 64 * W; t1 < n; t1 += 64 * W) {           // t1: the next chunk
         add_chunk();
         if constexpr (kPipe) {
-            v3 G, da[5], dq[2];
+            Terms o2[2];
             if (wv >= 2) {
-                evaluate_into(t1 + 64 * (wv - 2) + lane, wv == 2 ? s0 : s1);
-                evaluate(t1 + 64 * wv + lane, G, da, dq);
+                const int jl[2] = {t1 + 64 * (wv - 2) + lane, t1 + 64 * wv + lane};
+                evaluate(Two{}, jl, o2);
+                store(wv == 2 ? s0 : s1, o2[0]);
             }
             __syncthreads();
-            if (wv >= 2) {                                 // its first two tiles' buffers are free now
-                const int b = wv == 2 ? b0 : b1;
-                store_terms<5, 2>(term + b * TT::kSize, count + 2 * b, G, da, dq, lane);
-            }
-            const int o0 = b0, o1 = b1, o2 = b2, o3 = b3;
-            b0 = s0; b1 = s1; b2 = o0; b3 = o1; s0 = o2; s1 = o3;
+            if (wv >= 2) store(wv == 2 ? b0 : b1, o2[1]);  // its first two tiles' buffers are free now
+            const int o0 = b0, o1_ = b1, o2_ = b2, o3 = b3;
+            b0 = s0; b1 = s1; b2 = o0; b3 = o1_; s0 = o2_; s1 = o3;
         } else {
             __syncthreads();
-            evaluate_into(t1 + 64 * wv + lane, wv);
+            const int jl[1] = {t1 + 64 * wv + lane};
+            evaluate(One{}, jl, o1);
+            store(wv, o1[0]);
         }
         __syncthreads();
     }
+    {                                                      // the running maxima, reduced by another wave at the end
+        const double a = quad_checked_max(mind), b = quad_checked_max(maxi);
+        if ((lane & 3) == 0) { mx[0][16 * wv + (lane >> 2)] = a; mx[1][16 * wv + (lane >> 2)] = b; }
+    }
     add_chunk();
     if (np && (wv == kHA || (pre && wv == kHB))) {
-        int kind = -1;
-        if (lane < sm.nitem) {
-            const v3 f = np_recv_term(d, A, sm, il, gi, lane, kind);
-            if (wv == kHA) rfv = f;
-        }
-        const uint64_t k0 = __ballot(kind == 0), k1 = __ballot(kind == 1);
-        own0 = k0 ? __ffsll((unsigned long long)k0) - 1 : -1;
-        own1 = k1 ? __ffsll((unsigned long long)k1) - 1 : -1;
         if (wv == kHA && lane == 0) np_finalize_pre(d, A, gi, I.phi, ring8);
         if (W == 4 && pre && own0 >= 0) {
             const int off0 = d.items[sm.item0 + own0].an_off;
@@ -1044,11 +1093,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     }
     __syncthreads();
     // the non-point inputs into the (now free) tiles
-    double *rf = term, *ringS = rf + 3 * kNpFusedMaxItems, *partA = ringS + 8,
-           *partB = partA + 6 * kNpFusedMaxItems, *pq = term + kNpHead;
-    // both own items' products at once where they fit, else one at a time
-    const bool both = W == 4 && n <= kNpFusedMaxN;
-    static_assert(W != 4 || kTerm >= kNpHead + 12 * kNpFusedMaxN, "both items' products");
+    double *rf = term, *ringS = rf + 3 * kNpFusedMaxItems, *part = ringS + 8, *pq = term + kNpHead;
     if (W == 4 && pre && np && (wv == kHA || wv == kHB) && own0 >= 0) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -1061,7 +1106,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
         }
     }
     if (np && wv == kHA) {
-        if (lane < sm.nitem) { rf[3 * lane] = rfv.x; rf[3 * lane + 1] = rfv.y; rf[3 * lane + 2] = rfv.z; }
+        if (lane < sm.nitem) {
+            const v3 f = rgm * ran;
+            rf[3 * lane] = f.x; rf[3 * lane + 1] = f.y; rf[3 * lane + 2] = f.z;
+        }
         if (lane == 0) {
             own_s[0] = own0; own_s[1] = own1;
 #pragma unroll
@@ -1072,87 +1120,83 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
     if (wv == 0 && row16 == 0 && lane < 48) gsum[3 + rowc] = acc_d;
     if (wv == (W > 1 ? 1 : 0) && row16 == 0 && lane < 48) { gsum[rowc] = acc_g; gsum[6 + rowc] = acc_q; }
     __syncthreads();
-    double acc = wv == 0 && lane < 9 ? gsum[lane] : 0.0;
-    mind = wave_checked_max(mind);
-    maxi = wave_checked_max(maxi);
-    if (lane == 0) { wmax[wv] = mind; wmax[W + wv] = maxi; }
     // own items (mass.cpp:298-307): the products GM_j * field and
     // GM_j * (r_j - r_i) x field of every partner (+0 for the self pair), then
     // round r < T subtracts those of partner slice (chain + r) mod T in order,
     // one lane per round and component
-    if (np) {
-        const int T = sm.T;
-        const int tid = (int)threadIdx.x;
-        const int q0 = own_s[0], q1 = own_s[1];
-        for (int pass = 0; pass < (both ? 1 : 2); ++pass) {
-            const bool do0 = q0 >= 0 && (both || pass == 0), do1 = q1 >= 0 && (both || pass == 1);
-            const bool f0 = do0 && !pre;           // (formed already during the last chains)
-            if (f0 || do1) {
-                const int off0 = f0 ? d.items[sm.item0 + q0].an_off : 0;
-                const int off1 = do1 ? d.items[sm.item0 + q1].an_off : 0;
-                double *p0 = pq, *p1 = pq + (both ? 6 * kNpFusedMaxN : 0);
-                for (int jl = tid; jl < n; jl += 64 * W) {
-                    v3 a0{0, 0, 0}, t0v{0, 0, 0}, a1{0, 0, 0}, t1v{0, 0, 0};
-                    if (jl != il) {
-                        const int gj = off + jl;
-                        const double GMj = A.ld(F_GM, gj);
-                        const v3 rij = diff(A.lddv(F_R, gj), I.r);
-                        if (f0) {
-                            const double *a = d.an + 3 * ((int64_t)off0 + jl);
-                            const v3 an{a[0], a[1], a[2]};
-                            a0 = GMj * an;
-                            t0v = GMj * cross(rij, an);
-                        }
-                        if (do1) {
-                            const double *a = d.an + 3 * ((int64_t)off1 + jl);
-                            const v3 an{a[0], a[1], a[2]};
-                            a1 = GMj * an;
-                            t1v = GMj * cross(rij, an);
-                        }
-                    }
-                    if (f0) {
-                        double *o = p0 + 6 * jl;
-                        o[0] = a0.x; o[1] = a0.y; o[2] = a0.z; o[3] = t0v.x; o[4] = t0v.y; o[5] = t0v.z;
-                    }
-                    if (do1) {
-                        double *o = p1 + 6 * jl;
-                        o[0] = a1.x; o[1] = a1.y; o[2] = a1.z; o[3] = t1v.x; o[4] = t1v.y; o[5] = t1v.z;
-                    }
+    if (np && (own_s[0] >= 0 || own_s[1] >= 0)) {
+        const int T = sm.T, own[2] = {own_s[0], own_s[1]};
+        auto products = [&](int q, int base, int cnt, double *dst) {
+            const int off_q = d.items[sm.item0 + q].an_off;
+            for (int e = tid; e < cnt; e += 64 * W) {
+                const int jl = base + e;
+                v3 ta{0, 0, 0}, tt{0, 0, 0};
+                if (jl != il) {
+                    const int gj = off + jl;
+                    const double GMj = A.ld(F_GM, gj);
+                    const v3 rij = diff(A.lddv(F_R, gj), I.r);
+                    const double *a = d.an + 3 * ((int64_t)off_q + jl);
+                    const v3 an{a[0], a[1], a[2]};
+                    ta = GMj * an;
+                    tt = GMj * cross(rij, an);
                 }
+                double *o = dst + 6 * e;
+                o[0] = ta.x; o[1] = ta.y; o[2] = ta.z; o[3] = tt.x; o[4] = tt.y; o[5] = tt.z;
             }
-            __syncthreads();
-            // item 0's rounds in wave 0, item 1's in wave 1 (both in wave 0 for one item at a time)
-            const int k2 = both ? tid >> 6 : pass;
-            const int q = k2 == 0 ? q0 : q1;
-            if ((both ? k2 < 2 : tid < 64) && q >= 0 && (both || (k2 == 0 ? do0 : do1))) {
-                const double *pk = k2 == 0 ? pq : pq + (both ? 6 * kNpFusedMaxN : 0);
-                const int chain = d.items[sm.item0 + q].chain;
-                double *part = k2 == 0 ? partA : partB;
-                for (int u = tid & 63; u < 6 * T; u += 64) {
-                    const int r = u / 6, c = u - 6 * r;
-                    int kk = chain + r;
-                    if (kk >= T) kk -= T;
-                    const int j0 = kk * n / T, j1 = (kk + 1) * n / T;
-                    double x = 0;
+        };
+        // the part of round u / 6, component u % 6 within partners [base, base + cnt)
+        auto round_sum = [&](int q, int u, int base, int cnt, const double *src, double &x) {
+            const int r = u / 6, c = u - 6 * r;
+            int kk = d.items[sm.item0 + q].chain + r;
+            if (kk >= T) kk -= T;
+            const int j0 = max(kk * n / T, base), j1 = min((kk + 1) * n / T, base + cnt);
 #pragma unroll 8
-                    for (int jl = j0; jl < j1; ++jl) x -= pk[6 * jl + c];   // the self pair holds +0: an exact identity
-                    part[6 * r + c] = x;
+            for (int jl = j0; jl < j1; ++jl) x -= src[6 * (jl - base) + c];   // the self pair holds +0: an exact identity
+        };
+        if (pre) {                                         // item 0's products are there, item 1's fit beside them
+            if (own[1] >= 0) products(own[1], 0, n, pq + 6 * kNpPreMaxN);
+            __syncthreads();
+            if (wv < 2 && own[wv] >= 0)
+                for (int u = lane; u < 6 * T; u += 64) {
+                    double x = 0;
+                    round_sum(own[wv], u, 0, n, pq + 6 * kNpPreMaxN * wv, x);
+                    part[6 * kNpFusedMaxItems * wv + u] = x;
                 }
+        } else {
+            constexpr int kSums = (6 * kNpFusedMaxItems + 64 * W - 1) / (64 * W);
+            for (int k = 0; k < 2; ++k) {
+                if (own[k] < 0) continue;
+                double x[kSums];
+#pragma unroll
+                for (int m = 0; m < kSums; ++m) x[m] = 0;
+                for (int base = 0; base < n; base += kBlock) {
+                    const int cnt = min(kBlock, n - base);
+                    products(own[k], base, cnt, pq);
+                    __syncthreads();
+#pragma unroll
+                    for (int m = 0; m < kSums; ++m)
+                        if (tid + 64 * W * m < 6 * T) round_sum(own[k], tid + 64 * W * m, base, cnt, pq, x[m]);
+                    __syncthreads();
+                }
+#pragma unroll
+                for (int m = 0; m < kSums; ++m)
+                    if (tid + 64 * W * m < 6 * T) part[6 * kNpFusedMaxItems * k + tid + 64 * W * m] = x[m];
             }
-            if (!both && pass == 0) __syncthreads();      // the products of item 1 overwrite item 0's
+        }
+        __syncthreads();
+    }
+    if (wv == kMW) {
+        double a = lane < 16 * W ? mx[0][lane] : 0.0, b = lane < 16 * W ? mx[1][lane] : 0.0;
+        a = wave_checked_max(a);
+        b = wave_checked_max(b);
+        if (lane == 0) {
+            A.st(F_MIND, gi, checked_max_into(mind0, a));
+            A.st(F_MAXI, gi, checked_max_into(maxi0, b));
         }
     }
-    __syncthreads();
     if (wv != 0) return;
-    for (int u = 1; u < W; ++u) {
-        mind = checked_max_into(mind, wmax[u]);
-        maxi = checked_max_into(maxi, wmax[W + u]);
-    }
-    mind = checked_max_into(mind0, mind);
-    maxi = checked_max_into(maxi0, maxi);
+    double acc = lane < 9 ? gsum[lane] : 0.0;
     if (lane < 3) A.st(F_GACC + lane, gi, acc);
-    else if (lane == 9) A.st(F_MIND, gi, mind);
-    else if (lane == 10) A.st(F_MAXI, gi, maxi);
     if (np) {
         const int nit = sm.nitem, T = sm.T;
         const int o0 = own_s[0], o1 = own_s[1];
@@ -1172,11 +1216,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ?
         // (b) own items: geopotential (idaccel) first, then ring (jdaccel), mass.cpp:298-307
         for (int kind = 0; kind < 2; ++kind) {
             if ((kind == 0 ? o0 : o1) < 0) continue;
-            const double *part = kind == 0 ? partA : partB;
+            const double *sums = part + 6 * kNpFusedMaxItems * kind;
             if (lane >= 3 && lane < 9) {
                 const int col = lane - 3;                  // 0-2 acceleration, 3-5 torque
                 double sum = 0;
-                for (int k = 0; k < T; ++k) sum += part[6 * k + col];
+                for (int k = 0; k < T; ++k) sum += sums[6 * k + col];
                 const int f = (kind == 0 ? (col < 3 ? F_IDACC : F_IDTQ - 3) : (col < 3 ? F_JDACC : F_JDTQ - 3)) + col;
                 A.st(f, gi, sum);
                 acc += sum;
@@ -2371,10 +2415,10 @@ int main_wpb_waves(int nwork, int max_n, int waves) {
 }
 void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool fused_np, int waves, hipStream_t st) {
     if (!nwork) return;
-    int W = main_wpb_waves(nwork, max_n, waves);
-    if (fused_np && W == 1) W = 2;
+    const int W = main_wpb_waves(nwork, max_n, waves);
     if (fused_np && W == 4) hipLaunchKernelGGL((k_main_wpb<true, 4>), dim3(nwork), dim3(256), 0, st, d, work);
-    else if (fused_np) hipLaunchKernelGGL((k_main_wpb<true, 2>), dim3(nwork), dim3(128), 0, st, d, work);
+    else if (fused_np && W == 2) hipLaunchKernelGGL((k_main_wpb<true, 2>), dim3(nwork), dim3(128), 0, st, d, work);
+    else if (fused_np) hipLaunchKernelGGL((k_main_wpb<true, 1>), dim3(nwork), dim3(64), 0, st, d, work);
     else if (W == 4) hipLaunchKernelGGL((k_main_wpb<false, 4>), dim3(nwork), dim3(256), 0, st, d, work);
     else if (W == 2) hipLaunchKernelGGL((k_main_wpb<false, 2>), dim3(nwork), dim3(128), 0, st, d, work);
     else hipLaunchKernelGGL((k_main_wpb<false, 1>), dim3(nwork), dim3(64), 0, st, d, work);

@@ -98,13 +98,11 @@ void launch_main_serial_wpb(const View &d, const int2 *work, int nwork, hipStrea
 // fused_np: the receiver and own-item sums of the non-point pass run inside
 // each body's workgroup, after the item fields are formed (launch_np_field or
 // the extra workgroups of a deform launch; every thread-pool-order system
-// has at most 512 bodies -- 1024 with four wavefronts -- and 64 non-point
-// items)
-// waves: wavefronts per body, 0 = chosen from the batch's shape, else 1, 2 or
-// 4 (the fused kernel has at least 2)
+// has at most 64 non-point items)
+// waves: wavefronts per body, 0 = chosen from the batch's shape, else 1, 2 or 4
 void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool fused_np, int waves, hipStream_t st);
 void launch_np_field(const View &d, int max_n, hipStream_t st);
-constexpr int kNpFusedMaxN_h = 512, kNpFusedMaxN4_h = 1024, kNpFusedMaxItems_h = 64;
+constexpr int kNpFusedMaxItems_h = 64;
 // wavefronts per body that launch_main_wpb takes
 int main_wpb_waves(int nwork, int max_n, int waves);
 // one workgroup of up to 4 wavefronts per body (partner chunks evaluated in

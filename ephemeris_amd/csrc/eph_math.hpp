@@ -70,24 +70,36 @@ EPH_HD bool finite(dd a) { return !((0 * a.hi) != 0 || (0 * a.lo) != 0); }
 // of all ones, the one case where the last step of a reciprocal can round the
 // wrong way -- is checked in the two words of d; anything else (0, infinities
 // and NaN too) takes the language's operations.
-EPH_HD void recip_and_root(double d, double &q, double &s) {
+EPH_HD bool recip_and_root_safe(double d) {
 #ifdef __HIP_DEVICE_COMPILE__
-    const uint32_t hi = (uint32_t)__double2hiint(d);
-    if (hi - 0x20000000u < 0x40000000u && (uint32_t)__double2loint(d) != 0xffffffffu) {
-        const double y0 = __builtin_amdgcn_rsq(d);
-        const double r = fma(-(d * y0), y0, 1.0);
-        const double y = fma(y0 * r, fma(0.375, r, 0.5), y0);
-        double p = y * y;
-        p = fma(p, fma(-d, p, 1.0), p);
-        p = fma(p, fma(-d, p, 1.0), p);
-        const double h = 0.5 * (d * y);
-        double g = fma(fma(-y, y, p), h, y);
-        g = fma(fma(-g, g, p), h, g);
-        q = p;
-        s = g;
+    return (uint32_t)__double2hiint(d) - 0x20000000u < 0x40000000u && (uint32_t)__double2loint(d) != 0xffffffffu;
+#else
+    (void)d;
+    return false;
+#endif
+}
+EPH_HD void recip_and_root_fast(double d, double &q, double &s) {      // without the check
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y0 = __builtin_amdgcn_rsq(d);
+    const double r = fma(-(d * y0), y0, 1.0);
+    const double y = fma(y0 * r, fma(0.375, r, 0.5), y0);
+    double p = y * y;
+    p = fma(p, fma(-d, p, 1.0), p);
+    p = fma(p, fma(-d, p, 1.0), p);
+    const double h = 0.5 * (d * y);
+    const double g = fma(fma(-y, y, p), h, y);
+    q = p;
+    s = fma(fma(-g, g, p), h, g);
+#else
+    q = 1 / d;
+    s = sqrt(q);
+#endif
+}
+EPH_HD void recip_and_root(double d, double &q, double &s) {
+    if (recip_and_root_safe(d)) {
+        recip_and_root_fast(d, q, s);
         return;
     }
-#endif
     q = 1 / d;
     s = sqrt(q);
 }

@@ -203,7 +203,7 @@ int Batch::build_plan(int mode) {
     int64_t san_rows = 0;
     pl.maxT = 1;
     pl.max_n = 1;
-    pl.np_fusable = pl.np_fusable4 = true;
+    pl.np_fusable = true;
     for (int64_t s = 0; s < n_sys; ++s) {
         SysMeta &m = meta[s];
         const int64_t n = sys_n[s];
@@ -259,8 +259,7 @@ int Batch::build_plan(int mode) {
         }
         m.nitem = (int32_t)nnp;
         m.T = (int32_t)T;
-        if (n > kNpFusedMaxN_h || nnp > kNpFusedMaxItems_h) pl.np_fusable = false;
-        if (n > kNpFusedMaxN4_h || nnp > kNpFusedMaxItems_h) pl.np_fusable4 = false;
+        if (nnp > kNpFusedMaxItems_h) pl.np_fusable = false;
         pl.maxT = std::max<int>(pl.maxT, (int)T);
         items.insert(items.end(), sys_items.begin(), sys_items.end());
         append_blocks(blk_pool, (int)s, (int)n);
@@ -395,8 +394,7 @@ int Batch::accel(int mode, bool prepare_only) {
         }
     }
     if (prepare_only) return EPH_OK;
-    const bool fused_np = wpb && variant != 3 &&
-                          (pl.np_fusable || (pl.np_fusable4 && main_wpb_waves(pl.n_work_pool, pl.max_n, eff_waves()) == 4));
+    const bool fused_np = wpb && variant != 3 && pl.np_fusable;
     bool items_done = false;
     if (fields && !field_done) {
         Scope sc(profiler, 4, stream);

@@ -54,9 +54,7 @@ struct Plan {
     int n_work_pool = 0;
     int2 *d_work_serial = nullptr;   // the same of the single-thread-order systems
     int n_work_serial = 0;
-    // every pool system fits the fused non-point pass, at any number of
-    // wavefronts and with four
-    bool np_fusable = true, np_fusable4 = true;
+    bool np_fusable = true;          // every pool system fits the fused non-point pass
     int2 *d_blk16 = nullptr;         // (system, first body) of 16-body blocks, largest systems first
     int n_blk16 = 0;
     // item-field rows of the single-thread-order systems (see View::san)

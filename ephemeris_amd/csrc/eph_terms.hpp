@@ -30,11 +30,14 @@ struct IMain {
 struct PairGeo { v3 r, b, G; double rr2, rr, rr3, tp_dg; };
 
 // RELATIVITY (mass.impl:82-97)
-EPH_HD PairGeo relativity(const IMain &I, const JMain &T, v3 &gaccel) {
-    PairGeo p;
+// offset of the partner and squared distance, softened
+EPH_HD double pair_offset(const IMain &I, const JMain &T, v3 &r) {
     const ddv3 rj{dd{T.rxh, T.rxl}, dd{T.ryh, T.ryl}, dd{T.rzh, T.rzl}};
-    p.r = diff(rj, I.r);
-    recip_and_root(smax(dot(p.r, p.r), I.sR2 + T.sR2), p.rr2, p.rr);
+    r = diff(rj, I.r);
+    return smax(dot(r, r), I.sR2 + T.sR2);
+}
+// the rest, from p.r, p.rr2 and p.rr
+EPH_HD void relativity_from(const IMain &I, const JMain &T, PairGeo &p, v3 &gaccel) {
     p.rr3 = p.rr * p.rr2;
     const double tp_dphi = p.rr * T.GM;
     p.tp_dg = p.rr2 * tp_dphi;
@@ -47,6 +50,11 @@ EPH_HD PairGeo relativity(const IMain &I, const JMain &T, v3 &gaccel) {
     p.b = bj - I.beta;
     p.G = ((7 * tp_dphi / 2) * nj + (p.tp_dg * delta1) * p.r) + (p.tp_dg * (rbj - dot(p.r, p.b) * 4)) * p.b;
     gaccel += p.G;
+}
+EPH_HD PairGeo relativity(const IMain &I, const JMain &T, v3 &gaccel) {
+    PairGeo p;
+    recip_and_root(pair_offset(I, T, p.r), p.rr2, p.rr);
+    relativity_from(I, T, p, gaccel);
     return p;
 }
 
@@ -71,10 +79,10 @@ EPH_HD void lt_rad(const IMain &I, const JMain &T, const PairGeo &p, v3 &da, v3 
 // (RELATIVITY, ROTATIONAL_TIDAL_DEFORMATION_NANTI_FORCE, LENSE_THIRRING,
 // RADIATION_PRESSURE; mass.impl:82-125, mass.cpp:147-155).
 struct PairTerms { v3 G, dg, rxdg, gj, lt1, lt2, lt3, rad; double rr, tp_dg; };
-EPH_HD PairTerms pair_terms(const IMain &I, const JMain &T) {
+EPH_HD PairTerms pair_terms_from(const IMain &I, const JMain &T, PairGeo p) {   // p: r, rr2, rr
     PairTerms o;
     v3 unused{0, 0, 0};
-    const PairGeo p = relativity(I, T, unused);
+    relativity_from(I, T, p, unused);
     o.G = p.G;
     o.rr = p.rr;
     o.tp_dg = p.tp_dg;
@@ -90,6 +98,11 @@ EPH_HD PairTerms pair_terms(const IMain &I, const JMain &T) {
     o.lt3 = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
     o.rad = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
     return o;
+}
+EPH_HD PairTerms pair_terms(const IMain &I, const JMain &T) {
+    PairGeo p;
+    recip_and_root(pair_offset(I, T, p.r), p.rr2, p.rr);
+    return pair_terms_from(I, T, p);
 }
 
 // Add one pair's terms in the reference order.
