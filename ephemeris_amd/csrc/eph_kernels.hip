@@ -49,6 +49,16 @@ struct DevSin {
 // ---------------------------------------------------------------------------
 // field access
 // ---------------------------------------------------------------------------
+// What a body presents to its partners in the four-lane main force, as one
+// record: a wavefront copies the next sixteen partners to LDS in three loads,
+// where reading their rows took 25 for every four partners (81% of that
+// kernel's time on the vector memory path)
+struct __attribute__((aligned(16))) KRec {
+    double rxh, rxl, ryh, ryl, rzh, rzl, GM, sR2, phi, beta2, bx, by, bz, nx, ny, nz, GLx, GLy, GLz, lum, GM2c;
+    double quad;                 // R2 if C_potential has a non-zero entry, else 0
+};
+static_assert(sizeof(KRec) == 22 * 8 && F_KREC % 2 == 0, "16-byte records");
+
 struct Acc {
     double *F;
     int64_t P;
@@ -66,6 +76,7 @@ struct Acc {
     __device__ void stddm(int f, int g, const ddm3 &a) const { stddv(f, g, a.x); stddv(f + 6, g, a.y); stddv(f + 12, g, a.z); }
     __device__ v3 ldgl(int g) const { return todbl(lddv(F_GL, g)); }          // GL rounded to double
     __device__ double ldgm2c(int g) const { return 2 * ld(F_GM, g) / kC; }
+    __device__ KRec *krec(int g) const { return reinterpret_cast<KRec *>(F + (int64_t)F_KREC * P) + g; }
 };
 
 // ---------------------------------------------------------------------------
@@ -272,7 +283,8 @@ __device__ __forceinline__ void load_jdeform(const Acc &A, JDeform &T, int gj) {
     T.GM = A.ld(F_GM, gj); T.sR2 = A.ld(F_SR2, gj); T.tdf = A.ld(F_TDF, gj);
 }
 
-template <class Access>
+// REC: also the body's record of the four-lane main force
+template <bool REC, class Access>
 __device__ __forceinline__ void deform_write(const Access &A, int g, int prepare, const ddv3 &vi, double phi, v3 nacc,
                                              const m3 &C, const m3 &GI, v3 w) {
     A.stm(F_CPOT, g, C);
@@ -284,6 +296,15 @@ __device__ __forceinline__ void deform_write(const Access &A, int g, int prepare
         A.st(F_BETA2, g, dot(beta, beta));
         A.st(F_PHIC, g, phi / kC2);
         A.stv(F_NACCC, g, nacc / kC2);
+        if constexpr (REC) {
+            const v3 n = nacc / kC2, gl = A.ldgl(g);
+            const ddv3 r = A.lddv(F_R, g);
+            const bool quad = C.x.x != 0 || C.x.y != 0 || C.x.z != 0 || C.y.x != 0 || C.y.y != 0 || C.y.z != 0 ||
+                              C.z.x != 0 || C.z.y != 0 || C.z.z != 0;
+            *A.krec(g) = KRec{r.x.hi, r.x.lo, r.y.hi, r.y.lo, r.z.hi, r.z.lo, A.ld(F_GM, g), A.ld(F_SR2, g),
+                              phi / kC2, dot(beta, beta), beta.x, beta.y, beta.z, n.x, n.y, n.z,
+                              gl.x, gl.y, gl.z, A.ld(F_LUM, g), A.ldgm2c(g), quad ? A.ld(F_R2, g) : 0.0};
+        }
     } else {                                               // plain msystem::deform()
         A.st(F_PHI, g, phi);
         A.stv(F_NACC, g, nacc);
@@ -345,7 +366,7 @@ __global__ __launch_bounds__(BS) void k_deform_light(View d, const int4 *__restr
         H.apply(Csum, w, C, GI);
         if (!prepare || update_spin(A, gi, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
     }
-    deform_write(A, gi, prepare, A.lddv(F_V, gi), phi, nacc, C, GI, w);
+    deform_write<false>(A, gi, prepare, A.lddv(F_V, gi), phi, nacc, C, GI, w);
 }
 
 // The same for large batches with four lanes per body (16 bodies per
@@ -457,7 +478,7 @@ __device__ __forceinline__ void deform_k4_body(View d, const int4 *__restrict__ 
         H.apply(Csum, w, C, GI);
         if (!prepare || update_spin(A, gi, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
     }
-    deform_write(A, gi, prepare, A.lddv(F_V, gi), phi, nacc, C, GI, w);
+    deform_write<true>(A, gi, prepare, A.lddv(F_V, gi), phi, nacc, C, GI, w);
 }
 
 // Bodies with constant-time-lag tides (k2 != 0, tide_delay != 0): the tidal
@@ -531,7 +552,7 @@ __global__ __launch_bounds__(BS) void k_deform_damped(View d, const int4 *__rest
         if (!__syncthreads_or(again)) break;
     }
     if (!valid) return;
-    deform_write(A, gi, prepare, vi, phi, nacc, C, GI, w);
+    deform_write<false>(A, gi, prepare, vi, phi, nacc, C, GI, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -616,51 +637,66 @@ __global__ __launch_bounds__(BS) void k_main_pool(View d, const int2 *__restrict
 // sums start at +0 and never hold -0); the running maxima are order-free.
 // Four times as many wavefronts as one thread per body keep every SIMD busy
 // and balanced across systems of different sizes.
+//
+// What bounds it (256 systems of 64-504 bodies, 24.8 million pairs a launch):
+// with the partners read from their rows, 25 loads for every four partners,
+// the vector memory path was busy 81% of 404 us.  Partners now come as
+// records through an LDS tile, and only the rows of terms that some pair of
+// the group has are written and added (12 to 18 of 24): 284 us, the LDS busy
+// 76% and the FP64 units 68% of it.  Four wavefronts per SIMD in place of three
+// (128 registers, reached before the tile was there) did not help: 359 us
+// against 347 at that point.
 // ---------------------------------------------------------------------------
-constexpr int kK4Pitch = 25;
+constexpr int kK4Pitch = 19, kK4Tile = 16;
 
-// pair_terms for the four-lane kernel, which only adds the terms to sums that
-// start at +0: a term that is exactly zero for finite inputs -- the own or
-// the partner's quadrupole when there is none, the partner-spin LT term of a
-// partner without spin, the radiation of a dark partner -- is left at +0
-// without being formed (adding a zero of either sign to such a sum is an
-// exact identity).  The branches are uniform whenever the wavefront's 16
-// bodies or 4 partners agree, which they mostly do.
-__device__ __forceinline__ PairTerms pair_terms_k4(const IMain &I, bool own_quad, const JMain &T) {
-    PairTerms o;
-    v3 unused{0, 0, 0};
-    const PairGeo p = relativity(I, T, unused);
-    o.G = p.G;
-    o.rr = p.rr;
-    o.tp_dg = p.tp_dg;
-    o.dg = v3{0, 0, 0};
-    o.rxdg = v3{0, 0, 0};
-    if (own_quad) {
-        o.dg = (T.GM * p.rr3 * p.rr2 * I.R2) * quad_field(I.C, p);
-        o.rxdg = cross(p.r, o.dg);
-    }
-    o.gj = v3{0, 0, 0};
-    bool cj = false;
-#pragma unroll
-    for (int q = 0; q < 9; ++q) cj = cj || T.C[q] != 0;
-    if (cj && T.R2 != 0) {
-        const m3 Cj{v3{T.C[0], T.C[1], T.C[2]}, v3{T.C[3], T.C[4], T.C[5]}, v3{T.C[6], T.C[7], T.C[8]}};
-        o.gj = (T.GM * p.rr3 * p.rr2 * T.R2) * quad_field(Cj, p);
-    }
-    const double rcr32 = T.GM2c * p.rr3;
-    const v3 GLb = cross(I.GL, p.b);
-    o.lt1 = rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r);
-    o.lt2 = rcr32 * cross(I.GL, cross(p.r, p.b));
-    const v3 GLj{T.GLx, T.GLy, T.GLz};
-    o.lt3 = v3{0, 0, 0};
-    if (GLj.x != 0 || GLj.y != 0 || GLj.z != 0) o.lt3 = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
-    o.rad = v3{0, 0, 0};
-    if (T.lum != 0) o.rad = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
-    return o;
+// own body and partner without the quadrupoles' matrices, which few have and
+// which are loaded where they are needed
+__device__ __forceinline__ JMain jmain_k4(const KRec &q) {
+    JMain T;
+    T.rxh = q.rxh; T.rxl = q.rxl; T.ryh = q.ryh; T.ryl = q.ryl; T.rzh = q.rzh; T.rzl = q.rzl;
+    T.GM = q.GM; T.sR2 = q.sR2; T.phi = q.phi; T.beta2 = q.beta2;
+    T.bx = q.bx; T.by = q.by; T.bz = q.bz; T.nx = q.nx; T.ny = q.ny; T.nz = q.nz;
+    T.GLx = q.GLx; T.GLy = q.GLy; T.GLz = q.GLz; T.lum = q.lum; T.GM2c = q.GM2c; T.R2 = q.quad;
+    return T;
+}
+__device__ __forceinline__ IMain imain_k4(const Acc &A, int gi) {
+    const KRec q = *A.krec(gi);
+    IMain I;
+    I.r = ddv3{dd{q.rxh, q.rxl}, dd{q.ryh, q.ryl}, dd{q.rzh, q.rzl}};
+    I.sR2 = q.sR2; I.phi = q.phi; I.beta2 = q.beta2; I.R2 = q.quad; I.GM = q.GM; I.rR2G4c = A.ld(F_RR2G4C, gi);
+    I.beta = v3{q.bx, q.by, q.bz};
+    I.GL = v3{q.GLx, q.GLy, q.GLz};
+    return I;
 }
 
-// block `bid` of the list; term holds 64 x kK4Pitch doubles
-__device__ __forceinline__ void main_k4_body(View d, const int2 *__restrict__ blk, int bid, double *term) {
+// LDS rows of a pair: the terms every pair has, then two that only an own
+// quadrupole (X its force, Y its torque), or a partner's quadrupole (X) or
+// luminosity (Y), brings.  A group that has both kinds adds gaccel and
+// dtorque first; the partners' terms then take the rows of those.
+enum K4Row : int { K4_LT1 = 0, K4_LT3 = 3, K4_G = 6, K4_LT2 = 9, K4_X = 12, K4_Y = 15, K4_GJ2 = K4_G, K4_RAD2 = K4_LT2 };
+
+// adds the R rows of a group's four partners to a sum, in partner and row order
+template <int R>
+__device__ __forceinline__ void add_rows_k4(const double *grp, const int (&row)[R], double &a) {
+    double t[4][R];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < R; ++r) t[u][r] = grp[u * kK4Pitch + row[r]];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < R; ++r) a += t[u][r];
+}
+
+// block `bid` of the list; term holds 64 x kK4Pitch doubles.  A term that is
+// exactly zero for finite inputs -- the own or the partner's quadrupole when
+// there is none, the partner-spin LT term of a partner without spin, the
+// radiation of a dark partner -- is left at +0 without being formed, and where
+// no pair of the wavefront's group has it, its rows are neither written nor
+// added (the sums start at +0 and never hold -0: adding a zero of either sign
+// is an exact identity).
+__device__ __forceinline__ void main_k4_body(View d, const int2 *__restrict__ blk, int bid, double *term, KRec *tile) {
     const Acc A{d.F, d.nbp};
     const int s = blk[bid].x, i0 = blk[bid].y;             // bodies i0 .. i0 + 15
     if (i0 < 0) return;                                    // padding of an XCD-dealt list
@@ -670,55 +706,77 @@ __device__ __forceinline__ void main_k4_body(View d, const int2 *__restrict__ bl
     const int il = i0 + b;
     const bool valid = il < n;
     const int gi = off + (valid ? il : 0);
-    const IMain I = load_imain(A, gi);
-    bool own_quad = false;
-    {
-        const double *ci = &I.C.x.x;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) own_quad = own_quad || ci[q] != 0;
-        own_quad = own_quad && I.R2 != 0;
-    }
+    const IMain I = imain_k4(A, gi);
+    const bool own_quad = valid && I.R2 != 0;
+    const bool ow = __any(own_quad);
     const int c = k < 3 ? k : 0;
     double a_d = 0, a_g = 0, a_q = 0;                      // daccel, gaccel, dtorque component c
     double mind = 0, maxi = 0;
-    const double *grp = term + (b * 4) * kK4Pitch;
+    double *mine = term + lane * kK4Pitch;
+    const double *grp = term + (b * 4) * kK4Pitch + c;
+    const auto put = [&](int row, const v3 &v) { mine[row] = v.x; mine[row + 1] = v.y; mine[row + 2] = v.z; };
     for (int q0 = 0; q0 < n; q0 += 4) {
-        const int jl = q0 + k;
-        double t[24];
-        if (valid && jl < n && jl != il) {
-            JMain T;
-            load_jmain(A, T, off + jl);
-            const PairTerms pt = pair_terms_k4(I, own_quad, T);
-            const double v[24] = {pt.G.x, pt.G.y, pt.G.z, pt.dg.x, pt.dg.y, pt.dg.z, pt.gj.x, pt.gj.y, pt.gj.z,
-                                  -pt.lt1.x, -pt.lt1.y, -pt.lt1.z, pt.lt3.x, pt.lt3.y, pt.lt3.z,
-                                  pt.rad.x, pt.rad.y, pt.rad.z, pt.rxdg.x, pt.rxdg.y, pt.rxdg.z,
-                                  -pt.lt2.x, -pt.lt2.y, -pt.lt2.z};
+        if ((q0 & (kK4Tile - 1)) == 0) {                   // the next sixteen partners
+            const double2 *src = reinterpret_cast<const double2 *>(A.krec(off + q0));
+            const int cnt = min(kK4Tile, n - q0) * (int)(sizeof(KRec) / 16);
 #pragma unroll
-            for (int r = 0; r < 24; ++r) t[r] = v[r];
-            mind = checked_max_into(mind, pt.rr);
-            maxi = checked_max_into(maxi, pt.tp_dg);
+            for (int u = 0; u < 3; ++u) {
+                const int e = lane + 64 * u;
+                if (e < cnt) reinterpret_cast<double2 *>(tile)[e] = src[e];
+            }
+            __syncthreads();
+        }
+        const int jl = q0 + k;
+        const bool live = valid && jl < n && jl != il;
+        v3 gj{0, 0, 0}, rad{0, 0, 0};
+        bool jx = false;
+        if (live) {
+            const JMain T = jmain_k4(tile[(q0 & (kK4Tile - 1)) + k]);
+            v3 unused{0, 0, 0};
+            const PairGeo p = relativity(I, T, unused);
+            put(K4_G, p.G);
+            mind = checked_max_into(mind, p.rr);
+            maxi = checked_max_into(maxi, p.tp_dg);
+            const double rcr32 = T.GM2c * p.rr3;
+            const v3 GLb = cross(I.GL, p.b);
+            put(K4_LT1, -(rcr32 * (GLb - (3 * dot(GLb, p.r) * p.rr2) * p.r)));
+            put(K4_LT2, -(rcr32 * cross(I.GL, cross(p.r, p.b))));
+            const v3 GLj{T.GLx, T.GLy, T.GLz};
+            v3 lt3{0, 0, 0};
+            if (GLj.x != 0 || GLj.y != 0 || GLj.z != 0) lt3 = cross(rcr32 * (GLj - (3 * dot(GLj, p.r) * p.rr2) * p.r), p.b);
+            put(K4_LT3, lt3);
+            if (ow) {
+                v3 dg{0, 0, 0};
+                if (own_quad) dg = (T.GM * p.rr3 * p.rr2 * I.R2) * quad_field(A.ldm(F_CPOT, gi), p);
+                put(K4_X, dg);
+                put(K4_Y, own_quad ? cross(p.r, dg) : dg);
+            }
+            jx = T.R2 != 0 || T.lum != 0;
+            if (T.R2 != 0) gj = (T.GM * p.rr3 * p.rr2 * T.R2) * quad_field(A.ldm(F_CPOT, off + jl), p);
+            if (T.lum != 0) rad = (T.lum * I.rR2G4c * p.rr3 / I.GM) * p.r;
         } else {
 #pragma unroll
-            for (int r = 0; r < 24; ++r) t[r] = 0.0;
+            for (int r = 0; r < K4_Y + 3; ++r) mine[r] = 0.0;
         }
-#pragma unroll
-        for (int r = 0; r < 24; ++r) term[lane * kK4Pitch + r] = t[r];
+        const bool jxs = __any(jx);
+        if (jxs && !ow) { put(K4_X, gj); put(K4_Y, rad); }
         __syncthreads();
         if (k < 3) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const double *tr = grp + u * kK4Pitch;
-                a_d += tr[3 + c];
-                a_d += tr[6 + c];
-                a_d += tr[9 + c];
-                a_d += tr[12 + c];
-                a_d += tr[15 + c];
-                a_g += tr[c];
-                a_q += tr[18 + c];
-                a_q += tr[21 + c];
-            }
+            if (!ow && !jxs) add_rows_k4<2>(grp, {K4_LT1, K4_LT3}, a_d);
+            else if (!ow) add_rows_k4<4>(grp, {K4_X, K4_LT1, K4_LT3, K4_Y}, a_d);
+            else if (!jxs) add_rows_k4<3>(grp, {K4_X, K4_LT1, K4_LT3}, a_d);
+            add_rows_k4<1>(grp, {K4_G}, a_g);
+            if (ow) add_rows_k4<2>(grp, {K4_Y, K4_LT2}, a_q);
+            else add_rows_k4<1>(grp, {K4_LT2}, a_q);
         }
         __syncthreads();
+        if (ow && jxs) {
+            put(K4_GJ2, gj);
+            put(K4_RAD2, rad);
+            __syncthreads();
+            if (k < 3) add_rows_k4<5>(grp, {K4_X, K4_GJ2, K4_LT1, K4_LT3, K4_RAD2}, a_d);
+            __syncthreads();
+        }
     }
     mind = checked_max_into(mind, __shfl_xor(mind, 1, 64));
     mind = checked_max_into(mind, __shfl_xor(mind, 2, 64));
@@ -741,7 +799,8 @@ __device__ __forceinline__ void main_k4_body(View d, const int2 *__restrict__ bl
 
 __global__ __launch_bounds__(64) void k_main_k4(View d, const int2 *__restrict__ blk) {
     __shared__ double term[64 * kK4Pitch];
-    main_k4_body(d, blk, (int)blockIdx.x, term);
+    __shared__ KRec tile[kK4Tile];
+    main_k4_body(d, blk, (int)blockIdx.x, term, tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -1478,7 +1537,7 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
                 brk = true;
             }
             again_s = brk ? 0 : 1;
-            if (brk) deform_write(A, gi, prepare, vi, sums[0], v3{sums[1], sums[2], sums[3]}, C, GI, w);
+            if (brk) deform_write<LISTED>(A, gi, prepare, vi, sums[0], v3{sums[1], sums[2], sums[3]}, C, GI, w);
             else A.stv(F_W, gi, w);
             wsh[0] = w.x; wsh[1] = w.y; wsh[2] = w.z;
         }
@@ -1828,8 +1887,9 @@ __global__ __launch_bounds__(64) void k_np_item(View d, int nrows, int maxT) {
 static_assert(kK4Pitch >= 7, "the item sums use 7 doubles per lane of the term buffer");
 __global__ __launch_bounds__(64) void k_main_k4_items(View d, const int2 *__restrict__ blk, int nblk, int nrows, int maxT) {
     __shared__ double term[64 * kK4Pitch];
+    __shared__ KRec tile[kK4Tile];
     const int b = (int)blockIdx.x;
-    if (b < nblk) main_k4_body(d, blk, b, term);
+    if (b < nblk) main_k4_body(d, blk, b, term, tile);
     else np_item_body(d, nrows, maxT, b - nblk, term);
 }
 
@@ -1865,7 +1925,7 @@ __global__ __launch_bounds__(kBS) void k_np_recv(View d, const int2 *__restrict_
     // the ordered additions.
     const int sj = ((jl + 1) * T - 1) / n;
     int q = (sj + 1) * nit / T - 1;
-#pragma unroll 4
+#pragma unroll 8
     for (int m = 0; m < nit; ++m) {
         int body, an_off;
         double gm;
@@ -1880,28 +1940,28 @@ __global__ __launch_bounds__(kBS) void k_np_recv(View d, const int2 *__restrict_
         if (body != gj) da += gm * an;
         q = q == 0 ? nit - 1 : q - 1;
     }
-    // own items: idaccel (geopotential) then jdaccel (ring), mass.cpp:298-307
+    // own items: idaccel (geopotential) then jdaccel (ring), mass.cpp:298-307.
+    // Each body finds its item first, so that the workgroup's items are added
+    // at the same time; one after another they took half of this kernel.
     for (int kind = 0; kind < 2; ++kind) {
+        int own = -1;
         for (int q = 0; q < nit; ++q) {
-            int body, knd;
-            if (staged) {
-                body = s_body[q]; knd = s_kind[q];
-            } else {
-                const NPItem it = d.items[sm.item0 + q];
-                body = it.body; knd = it.kind;
-            }
-            if (body != gj || knd != kind) continue;
-            v3 sa{0, 0, 0}, sq{0, 0, 0};
-            for (int k = 0; k < T; ++k) {
-                const double *p = d.part + 6 * ((int64_t)(sm.item0 + q) * maxT + k);
-                sa += v3{p[0], p[1], p[2]};
-                sq += v3{p[3], p[4], p[5]};
-            }
-            A.stv(kind == 0 ? F_IDACC : F_JDACC, gj, sa);
-            A.stv(kind == 0 ? F_IDTQ : F_JDTQ, gj, sq);
-            da += sa;
-            dq += sq;
+            const int body = staged ? s_body[q] : d.items[sm.item0 + q].body;
+            const int knd = staged ? s_kind[q] : d.items[sm.item0 + q].kind;
+            if (body == gj && knd == kind) own = q;
         }
+        if (own < 0) continue;
+        v3 sa{0, 0, 0}, sq{0, 0, 0};
+        const double *p = d.part + 6 * (int64_t)(sm.item0 + own) * maxT;
+#pragma unroll 8
+        for (int k = 0; k < T; ++k, p += 6) {
+            sa += v3{p[0], p[1], p[2]};
+            sq += v3{p[3], p[4], p[5]};
+        }
+        A.stv(kind == 0 ? F_IDACC : F_JDACC, gj, sa);
+        A.stv(kind == 0 ? F_IDTQ : F_JDTQ, gj, sq);
+        da += sa;
+        dq += sq;
     }
     finalize_body(d, A, gj, da, dq);
 }

@@ -45,7 +45,9 @@ enum Field : int {
     F_X0S = 139,        // 18
     F_X0W = 157,        // 3
     F_STAGE = 160,      // 25 stages x 15: v(6 dd), a(3), w(3), dtorque(3)
-    F_COUNT = 160 + 25 * 15
+    // partner records of the four-lane main force (KRec), body by body
+    F_KREC = 536,
+    F_COUNT = 536 + 22
 };
 constexpr int kStageFields = 15;
 
