@@ -256,6 +256,34 @@ struct PartnerBlock {
 struct JDeform { double rxh, rxl, ryh, ryl, rzh, rzl, vxh, vxl, vyh, vyl, vzh, vzl, GM, sR2, tdf, pad; };
 
 // Per-body constants of UPDATE_HARMONICS (mass.impl:48-61) from the state
+// A workgroup's own body: its rows 0 .. F_CST + 8 in one load, a row a lane,
+// read from there as wavefront constants.  (A load per row by every lane took
+// half of a lone 504-body deformation launch's first phase, 9.7k -> 7.5k
+// cycles, and held 40 registers.)
+static_assert(F_CST + 9 <= 64, "a lane per row");
+struct OwnRows {
+    double raw;
+    __device__ __forceinline__ OwnRows(const Acc &A, int g, int lane) : raw(0) {
+        if (lane < F_CST + 9) raw = A.ld(lane, g);
+    }
+    __device__ __forceinline__ double ld(int f) const {
+        const int64_t x = __builtin_bit_cast(int64_t, raw);
+        const uint32_t lo = __builtin_amdgcn_readlane((int)x, f), hi = __builtin_amdgcn_readlane((int)(x >> 32), f);
+        return __builtin_bit_cast(double, (int64_t)((uint64_t)hi << 32 | lo));
+    }
+    __device__ __forceinline__ ddv3 lddv(int f) const {
+        return ddv3{dd{ld(f), ld(f + 1)}, dd{ld(f + 2), ld(f + 3)}, dd{ld(f + 4), ld(f + 5)}};
+    }
+};
+// the same rows left in LDS (a row a lane), with the names of Acc
+struct RowAcc {
+    const double *L;
+    __device__ double ld(int f, int) const { return L[f]; }
+    __device__ v3 ldv(int f, int) const { return v3{L[f], L[f + 1], L[f + 2]}; }
+    __device__ m3 ldm(int f, int g) const { return m3{ldv(f, g), ldv(f + 3, g), ldv(f + 6, g)}; }
+    __device__ ddv3 lddv(int f, int) const { return ddv3{dd{L[f], L[f + 1]}, dd{L[f + 2], L[f + 3]}, dd{L[f + 4], L[f + 5]}}; }
+    __device__ ddm3 lddm(int f, int g) const { return ddm3{lddv(f, g), lddv(f + 6, g), lddv(f + 12, g)}; }
+};
 template <class Access>
 __device__ __forceinline__ Harmonics harmonics_load(const Access &Ac, int g) {
     Harmonics h;
@@ -1346,15 +1374,86 @@ __device__ __forceinline__ void chain_add64(const double *row, double &acc) {
 // contributes +0, as in k_main_wpb.
 constexpr int kWpbDefPitch = 65;
 
-// W waves per body: in each round wave w evaluates partner chunk
-// (round * W + w); then the W chunks are added in partner order, with several
-// waves four chains on each (row_chain), with one thirteen lanes a chain each.
-// TAIL: the launch carries the non-point item fields in extra workgroups
-// (without them the kernel needs no scratch).  Work items with il < 0 are
-// padding of an XCD-dealt list.
-template <int W, bool LISTED>
-__device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__ work, int prepare, int bid,
-                                                double (*term)[13 * kWpbDefPitch]) {
+// the spin-independent part of a pair of the deformation
+struct DefGeo { v3 r, v; double rr2, dphi, dg, tdf; };
+
+struct DefPartner { ddv3 r, v; double sR2, GM, tdf; };
+__device__ __forceinline__ DefPartner def_partner(const Acc &A, int gj) {
+    return DefPartner{A.lddv(F_R, gj), A.lddv(F_V, gj), A.ld(F_SR2, gj), A.ld(F_GM, gj), A.ld(F_TDF, gj)};
+}
+// H pairs side by side: 1 / d and its root as in recip_and_root; the wavefront
+// takes the language's operations where one of its lanes fails the check
+template <int H>
+__device__ __forceinline__ void def_geo(const DefPartner *q, const DefPartner &own, const bool *live, DefGeo *p) {
+    double d[H];
+    bool ok = true;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        p[h].r = diff(q[h].r, own.r);
+        d[h] = smax(dot(p[h].r, p[h].r), own.sR2 + q[h].sR2);
+        ok = ok && (recip_and_root_safe(d[h]) || !live[h]);
+    }
+    double rr[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) recip_and_root_fast(d[h], p[h].rr2, rr[h]);
+    if (__any(!ok)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) recip_and_root(d[h], p[h].rr2, rr[h]);
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        p[h].dphi = rr[h] * q[h].GM;
+        p[h].dg = p[h].rr2 * p[h].dphi;
+        p[h].v = diff(q[h].v, own.v);
+        p[h].tdf = q[h].tdf;
+    }
+}
+
+// tidal matrix terms of a partner, negated: without delay, or with the
+// damped tide's axis dw (unit) and angle dwt (DAMPED_TIDAL_DEFORMATION_MATRIX,
+// mass.impl:1-23)
+__device__ __forceinline__ m3 plain_matrix(const DefGeo &p, double k2) {
+    const double fmj = -3 * p.dg;
+    return (fmj * k2) * subdiag(outer(p.rr2 * p.r, p.r), 1.0 / 3);
+}
+__device__ __forceinline__ m3 damped_matrix(const DefGeo &p, double k2, v3 dw, double dwt) {
+    const double fmj = -3 * p.dg;
+    const double ecwt2 = 1 + 4 * dwt * dwt,
+                 secwt2 = sqrt(ecwt2),
+                 x0 = sqrt((1 + secwt2) / (2 * ecwt2)),
+                 y0 = dwt * sqrt(2 / (ecwt2 * (1 + secwt2))),
+                 z02 = dwt * dwt * (2 / (ecwt2 + secwt2));
+    const v3 dr = x0 * p.r + y0 * cross(dw, p.r);
+    const m3 tm = outer(p.rr2 * dr, dr) - outer(z02 * dw, dw);
+    return (fmj * k2) * adddiag(tm, z02 - 1.0 / 3);
+}
+template <int H>
+__device__ __forceinline__ void damped_matrices(const DefGeo *p, const bool *live, double k2, double td, v3 w, m3 *tm) {
+    v3 dw[H];
+    double len[H], q[H];
+    bool ok = true;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        dw[h] = p[h].rr2 * cross(p[h].r, cross(w, p[h].r) - p[h].v);
+        const bool safe = root_and_recip_fast(dot(dw[h], dw[h]), len[h], q[h]);
+        ok = ok && (safe || !live[h]);
+    }
+    if (__any(!ok)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            len[h] = normalize(dw[h]);
+            q[h] = 1;
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) tm[h] = damped_matrix(p[h], k2, v3{dw[h].x * q[h], dw[h].y * q[h], dw[h].z * q[h]}, len[h] * (td * p[h].tdf));
+}
+
+// One wavefront per body: partners in chunks of 64, thirteen lanes a chain
+// each.  LISTED: the bodies of a work list that may hold padding (il < 0), as
+// part of the large-batch launch, whose main force reads records (KRec).
+template <bool LISTED>
+__device__ __forceinline__ void deform_wave_body(View d, const int2 *__restrict__ work, int prepare, int bid, double *term) {
     const Acc A{d.F, d.nbp};
     BodyOf body;
     if (LISTED) {                                          // not every body of the batch, with padding
@@ -1367,162 +1466,64 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
     const int il = body.il;
     const SysMeta sm = body.sm;
     const int n = sm.n, off = sm.off, gi = off + il;
-    const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lane = (int)threadIdx.x;
     __shared__ double sums[13];
     __shared__ int again_s;
     __shared__ double wsh[3];
-    __shared__ double hsh[19];                             // harmonics and GL, gathered by wave 1
-    // constant-time-lag bodies repeat the pair loop for each spin pass: with
-    // four wavefronts the spin-independent part of every pair is kept here
-    constexpr int kGeo = 10, kGeoN = 512;
-    __shared__ double geo[W == 4 ? kGeo * kGeoN : 1];
     const ddv3 ri = A.lddv(F_R, gi), vi = A.lddv(F_V, gi);
     const double sR2 = A.ld(F_SR2, gi), k2 = A.ld(F_K2, gi), td = A.ld(F_TD, gi);
     const bool damped = k2 != 0 && td != 0, ndelay = k2 != 0 && td == 0;
     const int nacc_chains = (k2 != 0) ? 13 : 4;
-    constexpr int kGroups = W == 1 ? 1 : (4 + W - 1) / W;  // groups of four chains per wavefront
     v3 w = A.ldv(F_W, gi);
     Harmonics H;
     m3 C, GI;
     int iters_left = 4;
-    // the spin-independent part of a pair; when every partner has its own
-    // lane (one round), it is formed once and kept across spin passes
-    const bool one_round = W > 1 && n <= 64 * W;           // (one wavefront: keep registers for occupancy)
-    v3 pr{0, 0, 0}, pv{0, 0, 0};
-    double prr2 = 0, ptp_dphi = 0, ptp_dg = 0, ptdf = 0;
-    auto pair_geo = [&](int jl) {
-        const int gj = off + jl;
-        pr = diff(A.lddv(F_R, gj), ri);
-        double rr;
-        recip_and_root(smax(dot(pr, pr), sR2 + A.ld(F_SR2, gj)), prr2, rr);
-        ptp_dphi = rr * A.ld(F_GM, gj);
-        ptp_dg = prr2 * ptp_dphi;
-        if (damped) {
-            pv = diff(A.lddv(F_V, gj), vi);
-            ptdf = A.ld(F_TDF, gj);
-        }
-    };
-    if (one_round) {
-        const int jl = 64 * wv + lane;
-        if (jl < n && jl != il) pair_geo(jl);
-    }
     bool first_pass = true;
     for (;;) {
-        double acc = (wv == 0 && lane < 4 && !first_pass) ? sums[lane] : 0.0;      // (one wavefront)
-        double accr[kGroups];                              // component 4 (wv + W g) + lane / 16 (several)
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g) accr[g] = 0.0;
-        for (int t0 = 0; t0 < n; t0 += 64 * W) {
-            const int jl = t0 + 64 * wv + lane;
+        double acc = (lane < 4 && !first_pass) ? sums[lane] : 0.0;
+        for (int t0 = 0; t0 < n; t0 += 64) {
+            const int jl = t0 + lane;
             double t[13];
 #pragma unroll
             for (int q = 0; q < 13; ++q) t[q] = 0.0;
             if (jl < n && jl != il) {
-                if (!one_round) {
-                    if (W == 4 && damped && n <= kGeoN && !first_pass) {
-                        pr = v3{geo[jl], geo[kGeoN + jl], geo[2 * kGeoN + jl]};
-                        prr2 = geo[3 * kGeoN + jl]; ptp_dphi = geo[4 * kGeoN + jl]; ptp_dg = geo[5 * kGeoN + jl];
-                        pv = v3{geo[6 * kGeoN + jl], geo[7 * kGeoN + jl], geo[8 * kGeoN + jl]};
-                        ptdf = geo[9 * kGeoN + jl];
-                    } else {
-                        pair_geo(jl);
-                        if (W == 4 && damped && n <= kGeoN) {
-                            geo[jl] = pr.x; geo[kGeoN + jl] = pr.y; geo[2 * kGeoN + jl] = pr.z;
-                            geo[3 * kGeoN + jl] = prr2; geo[4 * kGeoN + jl] = ptp_dphi; geo[5 * kGeoN + jl] = ptp_dg;
-                            geo[6 * kGeoN + jl] = pv.x; geo[7 * kGeoN + jl] = pv.y; geo[8 * kGeoN + jl] = pv.z;
-                            geo[9 * kGeoN + jl] = ptdf;
-                        }
-                    }
-                }
-                const v3 r = pr;
-                const double rr2 = prr2, tp_dphi = ptp_dphi, tp_dg = ptp_dg;
-                const v3 na = tp_dg * r;
-                t[0] = -tp_dphi;
+                const int gj = off + jl;
+                DefGeo p;
+                p.r = diff(A.lddv(F_R, gj), ri);
+                double rr;
+                recip_and_root(smax(dot(p.r, p.r), sR2 + A.ld(F_SR2, gj)), p.rr2, rr);
+                p.dphi = rr * A.ld(F_GM, gj);
+                p.dg = p.rr2 * p.dphi;
+                const v3 na = p.dg * p.r;
+                t[0] = -p.dphi;
                 t[1] = na.x; t[2] = na.y; t[3] = na.z;
-                if (ndelay) {
-                    const double fmj = -3 * tp_dg;
-                    const m3 tm = (fmj * k2) * subdiag(outer(rr2 * r, r), 1.0 / 3);
-                    const double *tp = &tm.x.x;
-#pragma unroll
-                    for (int q = 0; q < 9; ++q) t[4 + q] = -tp[q];
-                } else if (damped) {
-                    const v3 v = pv;
-                    const double fmj = -3 * tp_dg;
-                    v3 dw = rr2 * cross(r, cross(w, r) - v);
-                    double dwt = normalize(dw);
-                    dwt *= td * ptdf;
-                    const double ecwt2 = 1 + 4 * dwt * dwt,
-                                 secwt2 = sqrt(ecwt2),
-                                 x0 = sqrt((1 + secwt2) / (2 * ecwt2)),
-                                 y0 = dwt * sqrt(2 / (ecwt2 * (1 + secwt2))),
-                                 z02 = dwt * dwt * (2 / (ecwt2 + secwt2));
-                    const v3 dr = x0 * r + y0 * cross(dw, r);
-                    m3 tm = outer(rr2 * dr, dr) - outer(z02 * dw, dw);
-                    tm = (fmj * k2) * adddiag(tm, z02 - 1.0 / 3);
+                if (ndelay || damped) {
+                    m3 tm;
+                    if (ndelay) {
+                        tm = plain_matrix(p, k2);
+                    } else {
+                        v3 dw = p.rr2 * cross(p.r, cross(w, p.r) - diff(A.lddv(F_V, gj), vi));
+                        const double len = normalize(dw);
+                        tm = damped_matrix(p, k2, dw, len * (td * A.ld(F_TDF, gj)));
+                    }
                     const double *tp = &tm.x.x;
 #pragma unroll
                     for (int q = 0; q < 9; ++q) t[4 + q] = -tp[q];
                 }
             }
-            if (t0 + 64 * wv < n) {
 #pragma unroll
-                for (int q = 0; q < 13; ++q) term[wv][q * kWpbDefPitch + lane] = t[q];
-            }
+            for (int q = 0; q < 13; ++q) term[q * kWpbDefPitch + lane] = t[q];
             __syncthreads();
-            const int nw = min(W, (n - t0 + 63) / 64);
-            if (W == 1) {
-                if (lane < nacc_chains && (first_pass || lane >= 4)) chain_add64(term[0] + lane * kWpbDefPitch, acc);
-            } else {
-#pragma unroll
-                for (int g = 0; g < kGroups; ++g) {
-                    const int c0 = 4 * (wv + W * g);       // components c0 .. c0 + 3 on the four rows of sixteen lanes
-                    if (c0 >= nacc_chains || (c0 == 0 && !first_pass)) continue;
-                    const int c = min(c0 + (lane >> 4), 12);
-                    for (int u = 0; u < nw; ++u) row_chain(term[u] + c * kWpbDefPitch + (lane & 15), 64, accr[g]);
-                }
-            }
-            // the body's static harmonics in the world frame and GL (neither
-            // changes in this kernel before the spin step reads them)
-            if (W > 1 && first_pass && t0 == 0 && wv == W - 1 && lane == 0) {
-                Harmonics h;
-                h = harmonics_load(A, gi);
-                const ddv3 gl = A.lddv(F_GL, gi);
-                hsh[0] = h.k2r; hsh[1] = h.scale; hsh[2] = h.R2; hsh[3] = h.A;
-                const double *c = &h.Cw.x.x;
-#pragma unroll
-                for (int q = 0; q < 9; ++q) hsh[4 + q] = c[q];
-                hsh[13] = gl.x.hi; hsh[14] = gl.x.lo; hsh[15] = gl.y.hi; hsh[16] = gl.y.lo;
-                hsh[17] = gl.z.hi; hsh[18] = gl.z.lo;
-            }
+            if (lane < nacc_chains && (first_pass || lane >= 4)) chain_add64(term + lane * kWpbDefPitch, acc);
             __syncthreads();
         }
-        __syncthreads();
-        if (W == 1) {
-            if (lane < 13) sums[lane] = acc;               // phi, naccel: the first pass's sums, unchanged
-        } else {
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-                const int c0 = 4 * (wv + W * g), c = c0 + (lane >> 4);
-                if ((lane & 15) == 0 && c < 13 && (c0 > 0 || first_pass)) sums[c] = accr[g];
-            }
-        }
+        if (lane < 13) sums[lane] = acc;                   // phi, naccel: the first pass's sums, unchanged
         first_pass = false;
         __syncthreads();
-        if (threadIdx.x == 0) {
+        if (lane == 0) {
             const m3 Csum{v3{sums[4], sums[5], sums[6]}, v3{sums[7], sums[8], sums[9]}, v3{sums[10], sums[11], sums[12]}};
-            ddv3 GL;
-            if (W > 1) {
-                if (iters_left == 4) {
-                    H.k2r = hsh[0]; H.scale = hsh[1]; H.R2 = hsh[2]; H.A = hsh[3];
-                    double *c = &H.Cw.x.x;
-#pragma unroll
-                    for (int q = 0; q < 9; ++q) c[q] = hsh[4 + q];
-                }
-                GL = ddv3{dd{hsh[13], hsh[14]}, dd{hsh[15], hsh[16]}, dd{hsh[17], hsh[18]}};
-            } else {
-                if (iters_left == 4) H = harmonics_load(A, gi);
-                GL = A.lddv(F_GL, gi);
-            }
+            if (iters_left == 4) H = harmonics_load(A, gi);
+            const ddv3 GL = A.lddv(F_GL, gi);
             bool brk;
             if (damped) {
                 H.apply(Csum, w, C, GI);
@@ -1548,11 +1549,175 @@ __device__ __forceinline__ void deform_wpb_body(View d, const int2 *__restrict__
     }
 }
 
+// W wavefronts per body: in each round every lane evaluates two partners side
+// by side (one chain of a reciprocal, three square roots and three divisions
+// each, for a constant-time-lag body), 128 W in all, then the terms are added
+// in partner order, four chains on each wavefront.  A body with a time lag
+// repeats this for each of up to four spin passes and is what the launch waits
+// for; up to 128 W bodies it keeps the spin-independent part of its pairs in
+// registers.
+//
+// What bounds it (504 bodies, four wavefronts, two workgroups per CU): a body
+// with a time lag that needs three passes, 43k cycles -- 7.5k until the first
+// partners are there, then per pass 4k of terms, 5k of chains (504 dependent
+// additions at 9.5) and 2.4k of spin step on one lane.  One partner at a time
+// in rounds of 256, with the harmonics loaded by one lane between two
+// barriers, it was 53k: 21.3 -> 18.9 us per launch; 804 bodies 38.2 -> 32.4
+// (the geometry is formed again in each pass), 16 systems of 64-504 bodies
+// (two wavefronts) 68 -> 60.5.  Two chains side by side on one wavefront take
+// twice the time of one: the additions of a row are issue-bound.
+template <int W>
+constexpr int kDefSpan = 128 * W;
+template <int W>
+constexpr int kDefPitch = 128 * W + 8;                     // (the four rows of a group on different banks)
+template <int W>
+__device__ __forceinline__ void deform_waves_body(View d, const int2 *__restrict__ work, int prepare, int bid, double *term) {
+    const Acc A{d.F, d.nbp};
+    const BodyOf body = body_of(d, work, bid);
+    const int il = body.il;
+    const SysMeta sm = body.sm;
+    const int n = sm.n, off = sm.off, gi = off + il;
+    const int lane = (int)threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    static_assert(W == 2 || W == 4, "chain groups");
+    constexpr int kSpan = kDefSpan<W>, kPitch = kDefPitch<W>;
+    __shared__ double sums[13];
+    __shared__ int again_s;
+    __shared__ double wsh[3];
+    __shared__ double state[64], hsh[13];                  // the body's state; its harmonics, formed by the last wave
+    const bool kept = n <= kSpan;                          // one round: the pairs stay in registers
+    bool live[2], first_pass = true;
+    const auto fetch = [&](int t0, DefPartner *part) {     // this wavefront's two chunks of 64 partners
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = t0 + 64 * (W * h + wv), jl = c + lane;
+            live[h] = jl < n && jl != il;
+            if (c < n) part[h] = def_partner(A, off + min(jl, n - 1));
+        }
+    };
+    const OwnRows rows(A, gi, lane);                       // in flight with the first partners
+    DefPartner first[2];
+    if (kept) fetch(0, first);
+    const DefPartner own{rows.lddv(F_R), rows.lddv(F_V), rows.ld(F_SR2), 0, 0};
+    const double k2 = rows.ld(F_K2), td = rows.ld(F_TD);
+    const bool tide = k2 != 0, damped = tide && td != 0;
+    v3 w{rows.ld(F_W), rows.ld(F_W + 1), rows.ld(F_W + 2)};
+    int iters_left = 4;
+    DefGeo p[2];
+    const auto geo = [&](const DefPartner *part, bool two) {
+        if (two) def_geo<2>(part, own, live, p);
+        else def_geo<1>(part, own, live, p);
+    };
+    if (kept && 64 * wv < n) geo(first, 64 * (W + wv) < n);
+    for (;;) {
+        // the chains: components 4 g .. 4 g + 3 on the four rows of sixteen lanes
+        const int g0 = first_pass || wv > 0 ? wv : 4, g1 = W == 4 ? 4 : wv + 2;
+        double acc0 = 0, acc1 = 0;
+        for (int t0 = 0; t0 < n; t0 += kSpan) {
+            const int b0 = t0 + 64 * wv, b1 = b0 + 64 * W; // this wavefront's two chunks of 64 partners
+            if (b0 < n) {
+                const bool two = b1 < n;
+                if (!kept) {
+                    DefPartner part[2];
+                    fetch(t0, part);
+                    geo(part, two);
+                }
+                const auto put = [&](int h, const m3 &tm) {
+                    double *row = term + (h ? b1 : b0) - t0 + lane;
+                    const bool lv = live[h];
+                    if (first_pass) {
+                        const v3 na = p[h].dg * p[h].r;
+                        row[0] = lv ? -p[h].dphi : 0.0;
+                        row[kPitch] = lv ? na.x : 0.0; row[2 * kPitch] = lv ? na.y : 0.0; row[3 * kPitch] = lv ? na.z : 0.0;
+                    }
+                    if (tide) {
+                        const double *tp = &tm.x.x;
+#pragma unroll
+                        for (int q = 0; q < 9; ++q) row[(4 + q) * kPitch] = lv ? -tp[q] : 0.0;
+                    }
+                };
+                m3 tm[2];
+                if (damped) {
+                    if (two) damped_matrices<2>(p, live, k2, td, w, tm);
+                    else damped_matrices<1>(p, live, k2, td, w, tm);
+                } else if (tide) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) tm[h] = plain_matrix(p[h], k2);
+                }
+                put(0, tm[0]);
+                if (two) put(1, tm[1]);
+            }
+            if (first_pass && t0 == 0 && wv == W - 1) state[lane] = rows.raw;
+            __syncthreads();
+            const int cnt = (min(kSpan, n - t0) + 15) & ~15;
+            // the body's static harmonics in the world frame
+            if (first_pass && t0 == 0 && wv == W - 1 && lane == 0) {
+                const Harmonics h = harmonics_load(RowAcc{state}, 0);
+                hsh[0] = h.k2r; hsh[1] = h.scale; hsh[2] = h.R2; hsh[3] = h.A;
+                const double *c = &h.Cw.x.x;
+#pragma unroll
+                for (int q = 0; q < 9; ++q) hsh[4 + q] = c[q];
+            }
+            const auto row_of = [&](int g) { return term + min(4 * g + (lane >> 4), 12) * kPitch + (lane & 15); };
+            const int lim = tide ? 4 : 1;
+            if (g0 < lim && g1 < lim) {
+                row_chain2(row_of(g0), cnt, acc0, row_of(g1), cnt, acc1);
+            } else {
+                if (g0 < lim) row_chain(row_of(g0), cnt, acc0);
+                if (g1 < lim) row_chain(row_of(g1), cnt, acc1);
+            }
+            if (!kept) __syncthreads();
+        }
+        if ((lane & 15) == 0) {
+            const int c0 = 4 * g0 + (lane >> 4), c1 = 4 * g1 + (lane >> 4);
+            if (c0 < 13) sums[c0] = acc0;
+            if (c1 < 13) sums[c1] = acc1;
+        }
+        first_pass = false;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const m3 Csum{v3{sums[4], sums[5], sums[6]}, v3{sums[7], sums[8], sums[9]}, v3{sums[10], sums[11], sums[12]}};
+            Harmonics H;
+            m3 C, GI;
+            H.k2r = hsh[0]; H.scale = hsh[1]; H.R2 = hsh[2]; H.A = hsh[3];
+            double *c = &H.Cw.x.x;
+#pragma unroll
+            for (int q = 0; q < 9; ++q) c[q] = hsh[4 + q];
+            const ddv3 GL = RowAcc{state}.lddv(F_GL, 0);
+            bool brk;
+            if (damped) {
+                H.apply(Csum, w, C, GI);
+                brk = !prepare || update_spin(A, gi, GI, w, GL);
+                brk = brk || --iters_left == 0;
+            } else {
+                int iters = 4;
+                for (;;) {
+                    H.apply(Csum, w, C, GI);
+                    if (!prepare || update_spin(A, gi, GI, w, GL) || H.k2r == 0 || --iters == 0) break;
+                }
+                brk = true;
+            }
+            again_s = brk ? 0 : 1;
+            if (brk) deform_write<false>(A, gi, prepare, RowAcc{state}.lddv(F_V, 0), sums[0], v3{sums[1], sums[2], sums[3]}, C, GI, w);
+            else A.stv(F_W, gi, w);
+            wsh[0] = w.x; wsh[1] = w.y; wsh[2] = w.z;
+        }
+        __syncthreads();
+        if (!again_s) break;
+        w = v3{wsh[0], wsh[1], wsh[2]};
+    }
+}
+
+// TAIL: the launch carries the non-point item fields in extra workgroups
 template <int W, bool TAIL>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 3 : 1))) void k_deform_wpb(View d, const int2 *__restrict__ work, int prepare, NpTail np) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 3 : 2))) void k_deform_wpb(View d, const int2 *__restrict__ work, int prepare, NpTail np) {
     if (TAIL && np_tail(d, np)) return;
-    __shared__ double term[W][13 * kWpbDefPitch];
-    deform_wpb_body<W, false>(d, work, prepare, (int)blockIdx.x, term);
+    if constexpr (W == 1) {
+        __shared__ double term[13 * kWpbDefPitch];
+        deform_wave_body<false>(d, work, prepare, (int)blockIdx.x, term);
+    } else {
+        __shared__ double term[13 * kDefPitch<W>];
+        deform_waves_body<W>(d, work, prepare, (int)blockIdx.x, term);
+    }
 }
 
 // The large-batch deformation in one launch: workgroups [0, nwork) take the
@@ -1568,7 +1733,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     constexpr int kTerm = 13 * kWpbDefPitch > 64 * kDefK4Pitch ? 13 * kWpbDefPitch : 64 * kDefK4Pitch;
     __shared__ double term[kTerm];
     const int b = (int)blockIdx.x;
-    if (b < nwork) deform_wpb_body<1, true>(d, work, prepare, b, reinterpret_cast<double (*)[13 * kWpbDefPitch]>(term));
+    if (b < nwork) deform_wave_body<true>(d, work, prepare, b, term);
     else deform_k4_body(d, blk, prepare, b - nwork, term);
 }
 
@@ -2483,18 +2648,18 @@ void launch_main_wpb(const View &d, const int2 *work, int nwork, int max_n, bool
     else if (W == 2) hipLaunchKernelGGL((k_main_wpb<false, 2>), dim3(nwork), dim3(128), 0, st, d, work);
     else hipLaunchKernelGGL((k_main_wpb<false, 1>), dim3(nwork), dim3(64), 0, st, d, work);
 }
-// Wavefronts per body: several while every body's workgroup still fits on
-// the GPU at once (the ordered sums are serial, so extra wavefronts only pay
-// while CUs would otherwise be idle; a large batch is faster with one
-// wavefront per body).  Four, not eight, for a 504-body system: two 256-lane
-// workgroups then share each CU, one round of workgroups instead of two
-// (31 us instead of 43-58 us per launch on one MI355X).
+// Wavefronts per body: several while CUs would otherwise be idle (the ordered
+// sums are serial; a large batch is faster with one).  Per stage of variant 2
+// with one / two / four: 40 bodies 30.3 / 27.1 / 26.6 us, 10 systems of 50
+// 38.0 / 34.2 / 33.3, 20 of 50 40.8 / 37.2 / 45.7, 60 of 50 61.6 / 57.8 / 71.0, 24
+// of 100 73.8 / 61.8 / 71.8, one of 800 140 / 107 / 91; 9400 bodies in 32
+// systems 264 / 289 / 428.
 void launch_deform_wpb(const View &d, const int2 *work, int nwork, int max_n, int prepare, bool fields, int waves,
                        hipStream_t st) {
     if (!nwork) return;
     const int chunks = (max_n + 63) / 64;
     int W = waves;
-    if (W == 0) W = (chunks >= 4 && nwork <= 1280) ? 4 : (chunks >= 2 && nwork <= 2816) ? 2 : 1;
+    if (W == 0) W = nwork <= 512 || (chunks >= 4 && nwork <= 1280) ? 4 : nwork <= 4096 ? 2 : 1;
     const NpTail np{nwork, fields ? np_unit_count(d, max_n) : 0, max_n};
     const dim3 grid(nwork + (np.nunits + W - 1) / W), block(64 * W);
     if (np.nunits) {

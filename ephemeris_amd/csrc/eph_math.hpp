@@ -122,26 +122,27 @@ EPH_HD v3 &operator-=(v3 &a, v3 b) { a = a - b; return a; }
 // s = sqrt(r) and q = 1 / s, both correctly rounded: recip_and_root's steps
 // the other way round, with the same checks (on r, and on s for the final
 // reciprocal step) and the language's operations where they fail.
-EPH_HD void root_and_recip(double r, double &s, double &q) {
+EPH_HD bool root_and_recip_fast(double r, double &s, double &q) {      // false: the check failed
 #ifdef __HIP_DEVICE_COMPILE__
-    const uint32_t hi = (uint32_t)__double2hiint(r);
-    if (hi - 0x20000000u < 0x40000000u) {
-        const double y0 = __builtin_amdgcn_rsq(r);
-        const double d = fma(-(r * y0), y0, 1.0);
-        double y = fma(y0 * d, fma(0.375, d, 0.5), y0);
-        const double h = 0.5 * y;
-        double g = r * y;
-        g = fma(fma(-g, g, r), h, g);
-        g = fma(fma(-g, g, r), h, g);
-        if ((uint32_t)__double2loint(g) != 0xffffffffu) {
-            y = fma(y, fma(-g, y, 1.0), y);
-            y = fma(y, fma(-g, y, 1.0), y);
-            s = g;
-            q = y;
-            return;
-        }
-    }
+    const double y0 = __builtin_amdgcn_rsq(r);
+    const double d = fma(-(r * y0), y0, 1.0);
+    double y = fma(y0 * d, fma(0.375, d, 0.5), y0);
+    const double h = 0.5 * y;
+    double g = r * y;
+    g = fma(fma(-g, g, r), h, g);
+    g = fma(fma(-g, g, r), h, g);
+    y = fma(y, fma(-g, y, 1.0), y);
+    y = fma(y, fma(-g, y, 1.0), y);
+    s = g;
+    q = y;
+    return (uint32_t)__double2hiint(r) - 0x20000000u < 0x40000000u && (uint32_t)__double2loint(g) != 0xffffffffu;
+#else
+    (void)r; (void)s; (void)q;
+    return false;
 #endif
+}
+EPH_HD void root_and_recip(double r, double &s, double &q) {
+    if (root_and_recip_fast(r, s, q)) return;
     s = sqrt(r);
     q = 1 / s;
 }
