@@ -2289,26 +2289,89 @@ __global__ void k_extrema(View d, int invert) {
 // reference: the particle is one more body, after the field bodies, of a
 // system with N <= 48, so the single-thread summation order applies)
 // ---------------------------------------------------------------------------
+// A launch's field records do not change while it runs, and every lane reads
+// the same one, so they come through scalar loads (25 vector loads per partner
+// and lane before).
+typedef const __attribute__((address_space(4))) JMain cst_jmain;
+typedef const __attribute__((address_space(4))) uint64_t cst_u64;
+
+// Offsets, reciprocals and roots of H partners from T on: the reciprocals side
+// by side, one branch for all their checks.
+template <int H>
+__device__ __forceinline__ void particle_pairs(cst_jmain *T, const ddv3 &r, double sR2, v3 *d, double *rr2, double *rr) {
+    double dist[H];
+    bool safe = true;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        const ddv3 rj{dd{T[h].rxh, T[h].rxl}, dd{T[h].ryh, T[h].ryl}, dd{T[h].rzh, T[h].rzl}};
+        d[h] = diff(rj, r);
+        dist[h] = smax(dot(d[h], d[h]), sR2 + T[h].sR2);
+        safe = safe && recip_and_root_safe(dist[h]);
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) recip_and_root_fast(dist[h], rr2[h], rr[h]);
+    if (!safe) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) recip_and_root(dist[h], rr2[h], rr[h]);
+    }
+}
+// what one field body adds to the 1PN and Lense-Thirring sums of a particle
+__device__ __forceinline__ void particle_partner(cst_jmain *T, const IMain &I, v3 d, double rr2, double rr, v3 &ga, v3 &da,
+                                                 double &mind, double &maxi) {
+    JMain q;
+    q.GM = T->GM; q.phi = T->phi; q.beta2 = T->beta2;
+    q.bx = T->bx; q.by = T->by; q.bz = T->bz;
+    q.nx = T->nx; q.ny = T->ny; q.nz = T->nz;
+    PairGeo g;
+    g.r = d; g.rr2 = rr2; g.rr = rr;
+    relativity_from(I, q, g, ga);
+    mind = checked_max_into(mind, g.rr);
+    maxi = checked_max_into(maxi, g.tp_dg);
+    cst_u64 *gl = (cst_u64 *)&T->GLx;
+    if ((gl[0] | gl[1] | gl[2]) << 1) {                     // LENSE_THIRRING, the partner's spin, when it is not zero
+        const double rcr32 = T->GM2c * g.rr3;
+        const v3 GLj{T->GLx, T->GLy, T->GLz};
+        da += cross(rcr32 * (GLj - (3 * dot(GLj, g.r) * g.rr2) * g.r), g.b);
+    }
+}
+
 // Acceleration of one particle at state (r, v) from the field records T[0..nf)
 // (mass.cpp:311-374 for body index nf of an (nf+1)-body system).  The field
 // bodies' own sums are unaffected by the particle: its terms sit far below
 // their last ulp.  Terms that are exactly zero for a body without spin,
 // deformation or receptance (own tidal torque/force, own Lense-Thirring,
 // radiation received) are skipped: adding +-0 never changes a sum that
-// starts at +0 in round-to-nearest.
-__device__ __forceinline__ v3 particle_accel(const JMain *__restrict__ T, int nf, const ddv3 &r, const ddv3 &v,
+// starts at +0 in round-to-nearest.  Both passes over the partners need the
+// same offsets, reciprocals and roots: those of the first kPartKept partners,
+// in batches of kPartBatch, stay in registers (54 of 193 operations per
+// partner), the rest are formed again.  Nine is what the registers of two
+// wavefronts per SIMD hold.
+constexpr int kPartBatch = 3, kPartKept = 9;
+__device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, const ddv3 &r, const ddv3 &v,
                                              double sR2, double &mind, double &maxi) {
     double phi = 0;
     v3 nacc{0, 0, 0};
-    for (int j = 0; j < nf; ++j) {                          // deform_by, _NK2 class
-        const ddv3 rj{dd{T[j].rxh, T[j].rxl}, dd{T[j].ryh, T[j].ryl}, dd{T[j].rzh, T[j].rzl}};
-        const v3 d = diff(rj, r);
-        double rr2, rr;
-        recip_and_root(smax(dot(d, d), sR2 + T[j].sR2), rr2, rr);
-        const double tp_dphi = rr * T[j].GM;
+    auto newton = [&](cst_jmain *Tj, v3 d, double rr2, double rr) {   // deform_by, _NK2 class
+        const double tp_dphi = rr * Tj->GM;
         const double tp_dg = rr2 * tp_dphi;
         phi -= tp_dphi;
         nacc += tp_dg * d;
+    };
+    v3 d[kPartKept];
+    double rr2[kPartKept], rr[kPartKept];
+#pragma unroll
+    for (int j = 0; j < kPartKept; j += kPartBatch) {
+        if (j + kPartBatch > nf) continue;
+        particle_pairs<kPartBatch>(T + j, r, sR2, d + j, rr2 + j, rr + j);
+#pragma unroll
+        for (int h = j; h < j + kPartBatch; ++h) newton(T + h, d[h], rr2[h], rr[h]);
+    }
+    const int kept = min(nf / kPartBatch * kPartBatch, kPartKept);
+    for (int j = kept; j < nf; ++j) {
+        v3 dj;
+        double qj, sj;
+        particle_pairs<1>(T + j, r, sR2, &dj, &qj, &sj);
+        newton(T + j, dj, qj, sj);
     }
     IMain I;
     I.r = r;
@@ -2319,11 +2382,9 @@ __device__ __forceinline__ v3 particle_accel(const JMain *__restrict__ T, int nf
     const v3 naccc = nacc / kC2;
     v3 da{0, 0, 0}, ga{0, 0, 0};
     for (int p = 0; p < nf; ++p) {                          // reactions of earlier bodies' quadrupoles
-        const JMain &Tp = T[p];
-        bool quad = false;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) quad |= Tp.C[q] != 0;
-        if (!quad) continue;
+        cst_jmain &Tp = T[p];
+        cst_u64 *c = (cst_u64 *)Tp.C;
+        if (!((c[0] | c[1] | c[2] | c[3] | c[4] | c[5] | c[6] | c[7] | c[8]) << 1)) continue;   // all +-0
         const ddv3 rp{dd{Tp.rxh, Tp.rxl}, dd{Tp.ryh, Tp.ryl}, dd{Tp.rzh, Tp.rzl}};
         PairGeo g;
         g.r = diff(r, rp);
@@ -2332,129 +2393,172 @@ __device__ __forceinline__ v3 particle_accel(const JMain *__restrict__ T, int nf
         const m3 Cp{v3{Tp.C[0], Tp.C[1], Tp.C[2]}, v3{Tp.C[3], Tp.C[4], Tp.C[5]}, v3{Tp.C[6], Tp.C[7], Tp.C[8]}};
         da -= Tp.GM * ((g.rr3 * g.rr2 * Tp.R2) * quad_field(Cp, g));
     }
-    for (int j = 0; j < nf; ++j) {                          // own partner loop
-        const JMain &Tj = T[j];
-        const PairGeo g = relativity(I, Tj, ga);
-        mind = checked_max_into(mind, g.rr);
-        maxi = checked_max_into(maxi, g.tp_dg);
-        if (Tj.GLx != 0 || Tj.GLy != 0 || Tj.GLz != 0) {    // LENSE_THIRRING, the partner's spin
-            const double rcr32 = Tj.GM2c * g.rr3;
-            const v3 GLj{Tj.GLx, Tj.GLy, Tj.GLz};
-            da += cross(rcr32 * (GLj - (3 * dot(GLj, g.r) * g.rr2) * g.r), g.b);
-        }
+#pragma unroll
+    for (int j = 0; j < kPartKept; j += kPartBatch) {       // own partner loop
+        if (j + kPartBatch > nf) continue;
+#pragma unroll
+        for (int h = j; h < j + kPartBatch; ++h) particle_partner(T + h, I, d[h], rr2[h], rr[h], ga, da, mind, maxi);
+    }
+    for (int j = kept; j < nf; ++j) {
+        v3 dj;
+        double qj, sj;
+        particle_pairs<1>(T + j, r, sR2, &dj, &qj, &sj);
+        particle_partner(T + j, I, dj, qj, sj, ga, da, mind, maxi);
     }
     return (ga + da) + naccc * kC2;                          // gaccel + daccel + naccel
 }
 
 // Particle fields (stride pv.npp): r (6), v (6), last acceleration (3),
-// min_distance, max_influence; then, per lane of the launch, the derivatives
-// of stages kPartLdsStages..24 of the step in progress (3 rows each) and the
-// stage sums of stages 1..24 (3 rows each).
+// min_distance, max_influence; then, per lane of the launch, the stage sum and
+// the derivative (3 rows each) of stages 1..kPartStages of the step in progress.
 enum PField : int { P_R = 0, P_V = 6, P_A = 12, P_MIND = 15, P_MAXI = 16, P_COUNT = 17, P_STAGE = 17 };
-// Stage derivatives 0..7 of a step live in LDS (192 B per particle: three
-// 256-particle workgroups per CU), 8..24 in the particle's scratch rows;
-// every access names its address space, so no access goes through a
-// generic pointer.
-static_assert(kPartLdsStages == 8, "the LDS share and the occupancy hint of k_particles go together");
+
+// One column of a group of kPartRows consecutive rows of the tableau, left of
+// the group: its coefficients {hi, lo, hi + lo} in the rows whose bit is set.
+struct alignas(16) PGather {
+    int j, mask;
+    double c[kPartRows][3];
+};
+constexpr int kPartGroups = 25 / kPartRows;
+constexpr int kPartGather = kPartRows * kPartGroups * (kPartGroups - 1) / 2 + kPartGroups;   // columns 0..K-1 of each K = 1 + g rows
+__constant__ PGather c_pg[kPartGather];
+__constant__ int c_pg0[kPartGroups + 1];
+__constant__ int c_pin[26];       // column k in the rows of its own group: bit i of row K + i
+__constant__ int c_pkeep;         // bit k: stage k is a column of a later group
+
+struct PAcc { ddv3 v; v3 a; };
+__device__ __forceinline__ void padd(PAcc &s, dd c, double fc, const ddv3 &vj, v3 aj) {
+    s.v = add(s.v, scale(c, vj));
+    s.a += fc * aj;
+}
 
 // n_steps > 0: advance; n_steps < 0: compute the first acceleration from
 // the records; 0: leave the workgroup's particles alone.
-// Three wavefronts per SIMD (168 registers; a few values spill to scratch).
-__global__ __launch_bounds__(kPartBS) __attribute__((amdgpu_waves_per_eu(3))) void k_particles(PView pv, int n_steps, double dt, DtK dtk,
+//
+// x_k = x0 + dt * sum_j a_kj f_j (RungeKutta.impl:148-170); the velocity of
+// stage j is v0 + dt * (sum_l a_jl a_l), that sum as stage j formed it (the
+// same operations, so the same bits).  The rows are taken in groups of
+// kPartRows: one pass over the stages before the group reads each stage's sum
+// and derivative once and forms its velocity once for all rows of the group
+// (row by row it was 277 reads of a stage vector per step from beyond L1 and
+// 191 velocities, now 82 and 45); what is still to come of the later rows
+// waits in LDS, where each stage of the group adds its own column when it is
+// known.  Every sum keeps its order, ascending columns.  288 B of LDS per
+// particle and up to 256 registers: two wavefronts per SIMD.  1e6 particles
+// about 4.0 -> 2.95 ms per step, 8 steps of 20k particles and a download 3.97
+// -> 3.12 ms.
+__global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_particles(PView pv, int n_steps, double dt, DtK dtk,
                                                        const PBlock *__restrict__ blocks) {
-    const int p = blockIdx.x * kPartBS + (int)threadIdx.x;
+    const int lane = (int)threadIdx.x;
+    const int w0 = (int)blockIdx.x * kPartLanes;           // the wavefront's first particle
     int64_t entry0 = 0;
     int n_valid = kPartBS;
     if (blocks) {                                           // per-workgroup job offset and length
-        entry0 = blocks[blockIdx.x].rec_entry0;
-        n_steps = blocks[blockIdx.x].n_steps;
-        n_valid = blocks[blockIdx.x].n_valid;
+        const int b = w0 / kPartBS;
+        entry0 = blocks[b].rec_entry0;
+        n_steps = blocks[b].n_steps;
+        n_valid = blocks[b].n_valid;
     }
-    if (n_steps == 0) return;
+    const int left = min(pv.np - w0, n_valid - w0 % kPartBS);   // particles from w0 on
+    if (n_steps == 0 || left <= 0) return;
     const bool init = n_steps < 0;
-    // lanes past the last particle replay the workgroup's first one and store nothing
-    const bool valid = p < pv.np && (int)threadIdx.x < n_valid;
-    const int q = valid ? p : blockIdx.x * kPartBS;
-    double *P = pv.P;
+    // lanes past the last particle replay the wavefront's first one and store nothing
+    const bool valid = lane < left;
     const int64_t S = pv.npp;
+    glb_f64 *P = (glb_f64 *)pv.P + w0;
+    const int q = valid ? lane : 0;
     auto ld = [&](int f) { return P[f * S + q]; };
     ddv3 r{dd{ld(P_R + 0), ld(P_R + 1)}, dd{ld(P_R + 2), ld(P_R + 3)}, dd{ld(P_R + 4), ld(P_R + 5)}};
     ddv3 v{dd{ld(P_V + 0), ld(P_V + 1)}, dd{ld(P_V + 2), ld(P_V + 3)}, dd{ld(P_V + 4), ld(P_V + 5)}};
     double mind = ld(P_MIND), maxi = ld(P_MAXI);
+    cst_jmain *rec = (cst_jmain *)pv.rec;
     if (init) {
-        const v3 a = particle_accel(pv.rec + entry0 * pv.nrec_sys * kSmallMax, pv.nf, r, v, pv.sR2, mind, maxi);
+        const v3 a = particle_accel(rec + entry0 * pv.nrec_sys * kSmallMax, pv.nf, r, v, pv.sR2, mind, maxi);
         if (valid) {
             P[(P_A + 0) * S + q] = a.x; P[(P_A + 1) * S + q] = a.y; P[(P_A + 2) * S + q] = a.z;
             P[P_MIND * S + q] = mind; P[P_MAXI * S + q] = maxi;
         }
         return;
     }
-    // stage derivatives a_j (j = 0..24) of this step, per particle
-    __shared__ double fa[kPartLdsStages * 3 * kPartBS];
-    lds_f64 *fl = (lds_f64 *)fa + threadIdx.x;
-    glb_f64 *fg = (glb_f64 *)(P + (int64_t)P_STAGE * S + p);   // this lane's own column (p < npp)
-    auto get_l = [&](int j) { return v3{fl[(j * 3 + 0) * kPartBS], fl[(j * 3 + 1) * kPartBS], fl[(j * 3 + 2) * kPartBS]}; };
-    auto get_g = [&](int j) {
-        const int64_t r = (int64_t)(j - kPartLdsStages) * 3;
-        return v3{fg[(r + 0) * S], fg[(r + 1) * S], fg[(r + 2) * S]};
+    // the sums of the group's later rows so far
+    __shared__ double pend[(kPartRows - 1) * 9 * kPartLanes];
+    lds_f64 *pl = (lds_f64 *)pend + lane;
+    auto get_p = [&](int i) {                               // of row K + i, i >= 1
+        lds_f64 *o = pl + (i - 1) * 9 * kPartLanes;
+        return PAcc{ddv3{dd{o[0], o[1 * kPartLanes]}, dd{o[2 * kPartLanes], o[3 * kPartLanes]},
+                         dd{o[4 * kPartLanes], o[5 * kPartLanes]}},
+                    v3{o[6 * kPartLanes], o[7 * kPartLanes], o[8 * kPartLanes]}};
     };
-    auto put = [&](int j, v3 a) {
-        if (j < kPartLdsStages) {
-            fl[(j * 3 + 0) * kPartBS] = a.x; fl[(j * 3 + 1) * kPartBS] = a.y; fl[(j * 3 + 2) * kPartBS] = a.z;
-        } else {
-            const int64_t r = (int64_t)(j - kPartLdsStages) * 3;
-            fg[(r + 0) * S] = a.x; fg[(r + 1) * S] = a.y; fg[(r + 2) * S] = a.z;
-        }
+    auto put_p = [&](int i, const PAcc &s) {
+        lds_f64 *o = pl + (i - 1) * 9 * kPartLanes;
+        o[0] = s.v.x.hi; o[1 * kPartLanes] = s.v.x.lo; o[2 * kPartLanes] = s.v.y.hi; o[3 * kPartLanes] = s.v.y.lo;
+        o[4 * kPartLanes] = s.v.z.hi; o[5 * kPartLanes] = s.v.z.lo;
+        o[6 * kPartLanes] = s.a.x; o[7 * kPartLanes] = s.a.y; o[8 * kPartLanes] = s.a.z;
     };
-    // stage sums sum_l (a_jl) * a_l of stages j = 1..24, kept from stage j
-    // (the velocity of stage j is v0 + dt * that sum)
-    glb_f64 *fs = fg + (int64_t)kPartStageRows * S;
-    auto get_s = [&](int j) {
-        const int64_t r = (int64_t)(j - 1) * 3;
-        return v3{fs[(r + 0) * S], fs[(r + 1) * S], fs[(r + 2) * S]};
+    // stage sum and derivative of stage j (1..kPartStages); this lane's own column (w0 + lane < npp)
+    glb_f64 *fg = P + (int64_t)P_STAGE * S;
+    auto get_g = [&](int j, v3 &s, v3 &a) {
+        glb_f64 *o = fg + (int64_t)(j - 1) * 6 * S;
+        s = v3{o[lane], (o + S)[lane], (o + 2 * S)[lane]};
+        a = v3{(o + 3 * S)[lane], (o + 4 * S)[lane], (o + 5 * S)[lane]};
     };
-    auto put_s = [&](int j, v3 c) {
-        const int64_t r = (int64_t)(j - 1) * 3;
-        fs[(r + 0) * S] = c.x; fs[(r + 1) * S] = c.y; fs[(r + 2) * S] = c.z;
+    auto put_g = [&](int j, v3 s, v3 a) {
+        glb_f64 *o = fg + (int64_t)(j - 1) * 6 * S;
+        o[lane] = s.x; (o + S)[lane] = s.y; (o + 2 * S)[lane] = s.z;
+        (o + 3 * S)[lane] = a.x; (o + 4 * S)[lane] = a.y; (o + 5 * S)[lane] = a.z;
     };
     v3 a{ld(P_A + 0), ld(P_A + 1), ld(P_A + 2)};
     for (int step = 0; step < n_steps; ++step) {
         const ddv3 r0 = r, v0 = v;
-        put(0, a);
-        for (int k = 1; k <= 25; ++k) {
-            // x_k = x0 + dt * sum_j a_kj f_j (RungeKutta.impl:148-170); the
-            // velocity of stage j is v0 + dt * (sum_l a_jl a_l), that sum as
-            // stage j formed it (the same operations, so the same bits)
-            ddv3 cv = mkddv(v3{0, 0, 0});
-            v3 ca{0, 0, 0};
-            const int base = k * (k - 1) / 2;
-            const int e1 = c_row0[k + 1];
-            int e = c_row0[k];
-            for (; e < e1 && c_nzj[e] < kPartLdsStages; ++e) {   // non-zero columns, ascending
-                const int j = c_nzj[e];
-                const double2 c = c_rk[base + j];
-                const dd ckj{c.x, c.y};
-                const double fc = c.x + c.y;
-                ddv3 vj = v0;
-                if (j > 0) vj = add(v0, mkddv(dt * get_s(j)));
-                cv = add(cv, scale(ckj, vj));
-                ca += fc * get_l(j);
+        const v3 a0 = a;
+        cst_jmain *T = rec + ((entry0 + 25 * (int64_t)step) * pv.nrec_sys) * kSmallMax;
+        for (int g = 0; g < kPartGroups; ++g) {
+            PAcc s[kPartRows];
+#pragma unroll
+            for (int i = 0; i < kPartRows; ++i) s[i] = PAcc{mkddv(v3{0, 0, 0}), v3{0, 0, 0}};
+            auto column = [&](int e, const ddv3 &vj, v3 aj) {
+                const int mask = c_pg[e].mask;
+#pragma unroll
+                for (int i = 0; i < kPartRows; ++i)
+                    if (mask >> i & 1) padd(s[i], dd{c_pg[e].c[i][0], c_pg[e].c[i][1]}, c_pg[e].c[i][2], vj, aj);
+            };
+            int e = c_pg0[g];
+            const int e1 = c_pg0[g + 1];
+            v3 sn{0, 0, 0}, an{0, 0, 0};                    // of the next column
+            if (e + 1 < e1) get_g(c_pg[e + 1].j, sn, an);
+            column(e, v0, a0);
+            for (++e; e < e1; ++e) {
+                const v3 sj = sn, aj = an;
+                if (e + 1 < e1) get_g(c_pg[e + 1].j, sn, an);
+                column(e, add(v0, mkddv(dt * sj)), aj);
             }
-            for (; e < e1; ++e) {
-                const int j = c_nzj[e];
-                const double2 c = c_rk[base + j];
-                const dd ckj{c.x, c.y};
-                const double fc = c.x + c.y;
-                const ddv3 vj = add(v0, mkddv(dt * get_s(j)));
-                cv = add(cv, scale(ckj, vj));
-                ca += fc * get_g(j);
+#pragma unroll
+            for (int i = 1; i < kPartRows; ++i) put_p(i, s[i]);
+            PAcc cur = s[0];
+#pragma unroll 1
+            for (int i = 0; i < kPartRows; ++i) {
+                const int k = g * kPartRows + 1 + i;
+                r = add(r0, scale(mkdd(dt), cur.v));
+                v = add(v0, mkddv(dt * cur.a));
+                a = particle_accel(T, pv.nf, r, v, pv.sR2, mind, maxi);
+                T += pv.nrec_sys * kSmallMax;
+                if (c_pkeep >> k & 1) put_g(k, cur.a, a);
+                if (i + 1 == kPartRows) break;
+                const int mask = c_pin[k];
+                for (int i2 = i + 2; i2 < kPartRows; ++i2) {
+                    if (!(mask >> i2 & 1)) continue;
+                    const int k2 = g * kPartRows + 1 + i2;
+                    const double2 c = c_rk[k2 * (k2 - 1) / 2 + k];
+                    PAcc o = get_p(i2);
+                    padd(o, dd{c.x, c.y}, c.x + c.y, v, a);
+                    put_p(i2, o);
+                }
+                cur = get_p(i + 1);
+                if (mask >> (i + 1) & 1) {
+                    const double2 c = c_rk[(k + 1) * k / 2 + k];
+                    padd(cur, dd{c.x, c.y}, c.x + c.y, v, a);
+                }
             }
-            if (k < 25) put_s(k, ca);
-            r = add(r0, scale(mkdd(dt), cv));
-            v = add(v0, mkddv(dt * ca));
-            const JMain *T = pv.rec + ((entry0 + 25 * (int64_t)step + (k - 1)) * pv.nrec_sys) * kSmallMax;
-            a = particle_accel(T, pv.nf, r, v, pv.sR2, mind, maxi);
-            if (k < 25) put(k, a);
         }
     }
     if (!valid) return;
@@ -2465,7 +2569,7 @@ __global__ __launch_bounds__(kPartBS) __attribute__((amdgpu_waves_per_eu(3))) vo
 }
 
 void launch_particles(const PView &pv, int n_steps, double dt, const DtK &dtk, hipStream_t st, const PBlock *blocks) {
-    if (pv.np) hipLaunchKernelGGL(k_particles, dim3((pv.np + kPartBS - 1) / kPartBS), dim3(kPartBS), 0, st, pv,
+    if (pv.np) hipLaunchKernelGGL(k_particles, dim3((pv.np + kPartLanes - 1) / kPartLanes), dim3(kPartLanes), 0, st, pv,
                                   n_steps, dt, dtk, blocks);
 }
 
@@ -2558,6 +2662,8 @@ void set_rk_table(const double *tab650, hipStream_t st) {
     struct Tables {
         int nzj[325] = {}, row0[27] = {}, padj[kPadCols] = {}, pad0[27] = {};
         double padc[2 * kPadCols] = {};
+        PGather pg[kPartGather] = {};
+        int pg0[kPartGroups + 1] = {}, pin[26] = {}, pkeep = 0;
     };
     static const Tables t = [&] {
         Tables t;
@@ -2577,6 +2683,27 @@ void set_rk_table(const double *tab650, hipStream_t st) {
         }
         t.row0[26] = e;
         t.pad0[26] = p;
+        int n = 0;
+        for (int g = 0; g < kPartGroups; ++g) {
+            const int K = g * kPartRows + 1;
+            t.pg0[g] = n;
+            for (int j = 0; j < K + kPartRows - 1; ++j) {
+                PGather q{};
+                q.j = j;
+                for (int i = std::max(0, j + 1 - K); i < kPartRows; ++i) {
+                    const double *c = tab650 + 2 * ((K + i) * (K + i - 1) / 2 + j);
+                    if (c[0] == 0) continue;
+                    q.mask |= 1 << i;
+                    q.c[i][0] = c[0]; q.c[i][1] = c[1]; q.c[i][2] = c[0] + c[1];
+                }
+                if (j >= K) t.pin[j] = q.mask;
+                else if (j == 0 || q.mask) {                // column 0, the step's start, always comes first
+                    t.pg[n++] = q;
+                    t.pkeep |= j > 0 ? 1 << j : 0;
+                }
+            }
+        }
+        t.pg0[kPartGroups] = n;
         return t;
     }();
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_nzj), t.nzj, sizeof(t.nzj), 0, hipMemcpyHostToDevice, st);
@@ -2584,6 +2711,10 @@ void set_rk_table(const double *tab650, hipStream_t st) {
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_padj), t.padj, sizeof(t.padj), 0, hipMemcpyHostToDevice, st);
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_padc), t.padc, sizeof(t.padc), 0, hipMemcpyHostToDevice, st);
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pad0), t.pad0, sizeof(t.pad0), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pg), t.pg, sizeof(t.pg), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pg0), t.pg0, sizeof(t.pg0), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pin), t.pin, sizeof(t.pin), 0, hipMemcpyHostToDevice, st);
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_pkeep), &t.pkeep, sizeof(t.pkeep), 0, hipMemcpyHostToDevice, st);
 }
 
 void set_mass_fields(const int *field_of_slot, hipStream_t st) {

@@ -16,13 +16,16 @@ constexpr int kSmallMax = 64;    // largest system integrated by one workgroup
 struct DtK { double v[26]; };
 
 constexpr int kPartBS = 256;     // particles per workgroup
-// A particle's stage derivatives 0..kPartLdsStages-1 of the step in progress
-// live in LDS (24 B each per particle), the rest and the stage sums of
-// stages 1..24 in per-particle scratch rows after the particle's state:
-// kPartScratchRows rows, which every particle pool allocates.
-constexpr int kPartLdsStages = 8;
-constexpr int kPartStageRows = 3 * (25 - kPartLdsStages);        // derivatives kPartLdsStages..24
-constexpr int kPartScratchRows = kPartStageRows + 3 * 24;          // and the stage sums 1..24
+constexpr int kPartLanes = 64;   // particles per wavefront: a launch's workgroups, so that few particles spread over more CUs
+// k_particles forms the stage combinations of kPartRows rows of the tableau at
+// a time; the stages that a later group reads, 1..kPartStages at most, keep
+// their sum and derivative (3 rows each) in per-particle scratch rows after
+// the particle's state: kPartScratchRows rows, which every particle pool
+// allocates.
+constexpr int kPartRows = 5;
+constexpr int kPartStages = 25 - kPartRows;
+constexpr int kPartScratchRows = 6 * kPartStages;
+static_assert(25 % kPartRows == 0 && kPartBS % kPartLanes == 0, "whole groups of rows, whole wavefronts");
 
 // test particles in the recorded field of one small system
 struct PView {
