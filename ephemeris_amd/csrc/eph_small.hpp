@@ -287,6 +287,15 @@ __global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sy
         const int f = e / NB, b = e % NB;
         if (b < n && small_kept(f)) S.st(f, b, A.ld(f, off + b));
     }
+    auto record = [&](int step, int k) {
+        if (rec && tid >= NT - NB && tid - (NT - NB) < n) {
+            JMain T;
+            const int b = tid - (NT - NB);
+            load_jmain(S, T, b);
+            const int64_t e = 25 * (int64_t)step + (k - 1);
+            rec[(e * nrec_sys + blockIdx.x) * kSmallMax + b] = T;
+        }
+    };
     const int m = n - 1;                                   // pairs per body
     const int pair_i = m > 0 ? tid / m : 0, pair_q = tid - pair_i * m;     // this thread's pair of a round
     // thread roles: (component, body) of the stage sums, (rotation, body) of the
@@ -483,6 +492,7 @@ __global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sy
                 S.stv(F_DACC, 0, v3{0, 0, 0});
                 S.stv(F_DTQ, 0, v3{0, 0, 0});
             }
+            if (m == 0) record(step, k);
             for (int b0 = 0; m > 0 && b0 < n; b0 += bpr_m) {
                 const int nbr = min(bpr_m, n - b0);
                 if (tid < nbr * m) {
@@ -516,13 +526,7 @@ __global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sy
                         S.st(F_MIND + c, i, x);
                     }
                 }
-                if (rec && b0 == 0 && tid >= NT - NB && tid - (NT - NB) < n) {
-                    JMain T;
-                    const int b = tid - (NT - NB);
-                    load_jmain(S, T, b);
-                    const int64_t e = 25 * (int64_t)step + (k - 1);
-                    rec[(e * nrec_sys + blockIdx.x) * kSmallMax + b] = T;
-                }
+                if (b0 == 0) record(step, k);
                 __syncthreads();
             }
             if (NP) {                                      // RING_CORRECTION of a ring host
