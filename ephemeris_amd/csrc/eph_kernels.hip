@@ -2291,23 +2291,47 @@ __global__ void k_extrema(View d, int invert) {
 // ---------------------------------------------------------------------------
 // A launch's field records do not change while it runs, and every lane reads
 // the same one, so they come through scalar loads (25 vector loads per partner
-// and lane before).
+// and lane before).  A scalar load that misses its cache takes about a
+// thousand cycles, and two wavefronts per SIMD do not hide that (the wavefronts
+// waited 48% of their cycles, 2.95 ms per step of 1e6 particles, while each
+// partner was loaded where it is used and its quadrupole and spin were looked
+// at): what a partner needs is loaded while the partners before it are
+// evaluated, and one pair of masks says which have a quadrupole or a spin:
+// 2.33 ms.  Only what fits the scalar registers goes ahead: with GM and the
+// soft radius too, 450 of 2,100 instructions of a stage moved scalars to and
+// from vector registers.
 typedef const __attribute__((address_space(4))) JMain cst_jmain;
 typedef const __attribute__((address_space(4))) uint64_t cst_u64;
 
-// Offsets, reciprocals and roots of H partners from T on: the reciprocals side
-// by side, one branch for all their checks.
+// a partner's position, the start of its record ...
+__device__ __forceinline__ ddv3 part_near(cst_jmain *T) {
+    return ddv3{dd{T->rxh, T->rxl}, dd{T->ryh, T->ryl}, dd{T->rzh, T->rzl}};
+}
+// ... and what its 1PN term needs
+__device__ __forceinline__ JMain part_rel(cst_jmain *T) {
+    JMain q;
+    q.GM = T->GM; q.phi = T->phi; q.beta2 = T->beta2;
+    q.bx = T->bx; q.by = T->by; q.bz = T->bz;
+    q.nx = T->nx; q.ny = T->ny; q.nz = T->nz;
+    return q;
+}
+constexpr int kPartBatch = 3, kPartKept = 9;
+
+// Offsets, reciprocals and roots of the H partners from T on, at the positions
+// p: the reciprocals side by side, one branch for all their checks; p becomes
+// the positions of the H partners after them.
 template <int H>
-__device__ __forceinline__ void particle_pairs(cst_jmain *T, const ddv3 &r, double sR2, v3 *d, double *rr2, double *rr) {
+__device__ __forceinline__ void particle_pairs(ddv3 *p, cst_jmain *T, const ddv3 &r, double sR2, v3 *d, double *rr2, double *rr) {
     double dist[H];
     bool safe = true;
 #pragma unroll
     for (int h = 0; h < H; ++h) {
-        const ddv3 rj{dd{T[h].rxh, T[h].rxl}, dd{T[h].ryh, T[h].ryl}, dd{T[h].rzh, T[h].rzl}};
-        d[h] = diff(rj, r);
+        d[h] = diff(p[h], r);
         dist[h] = smax(dot(d[h], d[h]), sR2 + T[h].sR2);
         safe = safe && recip_and_root_safe(dist[h]);
     }
+#pragma unroll
+    for (int h = 0; h < H; ++h) p[h] = part_near(T + H + h);
 #pragma unroll
     for (int h = 0; h < H; ++h) recip_and_root_fast(dist[h], rr2[h], rr[h]);
     if (!safe) {
@@ -2315,20 +2339,15 @@ __device__ __forceinline__ void particle_pairs(cst_jmain *T, const ddv3 &r, doub
         for (int h = 0; h < H; ++h) recip_and_root(dist[h], rr2[h], rr[h]);
     }
 }
-// what one field body adds to the 1PN and Lense-Thirring sums of a particle
-__device__ __forceinline__ void particle_partner(cst_jmain *T, const IMain &I, v3 d, double rr2, double rr, v3 &ga, v3 &da,
-                                                 double &mind, double &maxi) {
-    JMain q;
-    q.GM = T->GM; q.phi = T->phi; q.beta2 = T->beta2;
-    q.bx = T->bx; q.by = T->by; q.bz = T->bz;
-    q.nx = T->nx; q.ny = T->ny; q.nz = T->nz;
+// what one field body adds to the 1PN and (with a spin) Lense-Thirring sums of a particle
+__device__ __forceinline__ void particle_partner(const JMain &q, cst_jmain *T, bool spin, const IMain &I, v3 d, double rr2,
+                                                 double rr, v3 &ga, v3 &da, double &mind, double &maxi) {
     PairGeo g;
     g.r = d; g.rr2 = rr2; g.rr = rr;
     relativity_from(I, q, g, ga);
     mind = checked_max_into(mind, g.rr);
     maxi = checked_max_into(maxi, g.tp_dg);
-    cst_u64 *gl = (cst_u64 *)&T->GLx;
-    if ((gl[0] | gl[1] | gl[2]) << 1) {                     // LENSE_THIRRING, the partner's spin, when it is not zero
+    if (spin) {                                             // LENSE_THIRRING, the partner's spin
         const double rcr32 = T->GM2c * g.rr3;
         const v3 GLj{T->GLx, T->GLy, T->GLz};
         da += cross(rcr32 * (GLj - (3 * dot(GLj, g.r) * g.rr2) * g.r), g.b);
@@ -2336,23 +2355,27 @@ __device__ __forceinline__ void particle_partner(cst_jmain *T, const IMain &I, v
 }
 
 // Acceleration of one particle at state (r, v) from the field records T[0..nf)
-// (mass.cpp:311-374 for body index nf of an (nf+1)-body system).  The field
-// bodies' own sums are unaffected by the particle: its terms sit far below
-// their last ulp.  Terms that are exactly zero for a body without spin,
-// deformation or receptance (own tidal torque/force, own Lense-Thirring,
-// radiation received) are skipped: adding +-0 never changes a sum that
-// starts at +0 in round-to-nearest.  Both passes over the partners need the
-// same offsets, reciprocals and roots: those of the first kPartKept partners,
-// in batches of kPartBatch, stay in registers (54 of 193 operations per
-// partner), the rest are formed again.  Nine is what the registers of two
-// wavefronts per SIMD hold.
-constexpr int kPartBatch = 3, kPartKept = 9;
-__device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, const ddv3 &r, const ddv3 &v,
+// (mass.cpp:311-374 for body index nf of an (nf+1)-body system); p: the positions of
+// the first kPartBatch of them.  The field bodies' own sums are unaffected by the
+// particle: its terms sit far below their last ulp.  Terms that are exactly
+// zero for a body without spin, deformation or receptance (own tidal
+// torque/force, own Lense-Thirring, radiation received) or for a partner
+// without quadrupole or spin (part_masks) are skipped: adding +-0 never
+// changes a sum that starts at +0 in round-to-nearest.  Both passes over the
+// partners need the same offsets, reciprocals and roots: those of the first
+// kPartKept partners, in batches of kPartBatch, stay in registers (54 of 193
+// operations per partner), the rest are formed again.  Nine is what the
+// registers of two wavefronts per SIMD hold.  Records past the field's last
+// (all kSmallMax of an entry are allocated) are loaded ahead but not used.
+static_assert(kSmallBodies + kPartBatch < kPartMasks, "records loaded ahead stay below the masks");
+__device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, ddv3 *p, const ddv3 &r, const ddv3 &v,
                                              double sR2, double &mind, double &maxi) {
+    cst_u64 *masks = (cst_u64 *)(T + kPartMasks);
+    const uint64_t quad = masks[0], spin = masks[1];
     double phi = 0;
     v3 nacc{0, 0, 0};
-    auto newton = [&](cst_jmain *Tj, v3 d, double rr2, double rr) {   // deform_by, _NK2 class
-        const double tp_dphi = rr * Tj->GM;
+    auto newton = [&](double GM, v3 d, double rr2, double rr) {   // deform_by, _NK2 class
+        const double tp_dphi = rr * GM;
         const double tp_dg = rr2 * tp_dphi;
         phi -= tp_dphi;
         nacc += tp_dg * d;
@@ -2362,17 +2385,18 @@ __device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, const ddv3 &r
 #pragma unroll
     for (int j = 0; j < kPartKept; j += kPartBatch) {
         if (j + kPartBatch > nf) continue;
-        particle_pairs<kPartBatch>(T + j, r, sR2, d + j, rr2 + j, rr + j);
+        particle_pairs<kPartBatch>(p, T + j, r, sR2, d + j, rr2 + j, rr + j);
 #pragma unroll
-        for (int h = j; h < j + kPartBatch; ++h) newton(T + h, d[h], rr2[h], rr[h]);
+        for (int h = 0; h < kPartBatch; ++h) newton(T[j + h].GM, d[j + h], rr2[j + h], rr[j + h]);
     }
     const int kept = min(nf / kPartBatch * kPartBatch, kPartKept);
     for (int j = kept; j < nf; ++j) {
         v3 dj;
         double qj, sj;
-        particle_pairs<1>(T + j, r, sR2, &dj, &qj, &sj);
-        newton(T + j, dj, qj, sj);
+        particle_pairs<1>(p, T + j, r, sR2, &dj, &qj, &sj);
+        newton(T[j].GM, dj, qj, sj);
     }
+    JMain q = part_rel(T);
     IMain I;
     I.r = r;
     I.sR2 = sR2;
@@ -2381,10 +2405,8 @@ __device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, const ddv3 &r
     I.phi = phi / kC2;
     const v3 naccc = nacc / kC2;
     v3 da{0, 0, 0}, ga{0, 0, 0};
-    for (int p = 0; p < nf; ++p) {                          // reactions of earlier bodies' quadrupoles
-        cst_jmain &Tp = T[p];
-        cst_u64 *c = (cst_u64 *)Tp.C;
-        if (!((c[0] | c[1] | c[2] | c[3] | c[4] | c[5] | c[6] | c[7] | c[8]) << 1)) continue;   // all +-0
+    for (uint64_t m = quad; m; m &= m - 1) {                // reactions of earlier bodies' quadrupoles
+        cst_jmain &Tp = T[__builtin_ctzll(m)];
         const ddv3 rp{dd{Tp.rxh, Tp.rxl}, dd{Tp.ryh, Tp.ryl}, dd{Tp.rzh, Tp.rzl}};
         PairGeo g;
         g.r = diff(r, rp);
@@ -2397,13 +2419,20 @@ __device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, const ddv3 &r
     for (int j = 0; j < kPartKept; j += kPartBatch) {       // own partner loop
         if (j + kPartBatch > nf) continue;
 #pragma unroll
-        for (int h = j; h < j + kPartBatch; ++h) particle_partner(T + h, I, d[h], rr2[h], rr[h], ga, da, mind, maxi);
+        for (int h = j; h < j + kPartBatch; ++h) {
+            const JMain qn = part_rel(T + h + 1);
+            particle_partner(q, T + h, spin >> h & 1, I, d[h], rr2[h], rr[h], ga, da, mind, maxi);
+            q = qn;
+        }
     }
+    if (kept < nf) p[0] = part_near(T + kept);
     for (int j = kept; j < nf; ++j) {
         v3 dj;
         double qj, sj;
-        particle_pairs<1>(T + j, r, sR2, &dj, &qj, &sj);
-        particle_partner(T + j, I, dj, qj, sj, ga, da, mind, maxi);
+        const JMain qn = part_rel(T + j + 1);
+        particle_pairs<1>(p, T + j, r, sR2, &dj, &qj, &sj);
+        particle_partner(q, T + j, spin >> j & 1, I, dj, qj, sj, ga, da, mind, maxi);
+        q = qn;
     }
     return (ga + da) + naccc * kC2;                          // gaccel + daccel + naccel
 }
@@ -2414,22 +2443,22 @@ __device__ __forceinline__ v3 particle_accel(cst_jmain *T, int nf, const ddv3 &r
 enum PField : int { P_R = 0, P_V = 6, P_A = 12, P_MIND = 15, P_MAXI = 16, P_COUNT = 17, P_STAGE = 17 };
 
 // One column of a group of kPartRows consecutive rows of the tableau, left of
-// the group: its coefficients {hi, lo, hi + lo} in the rows whose bit is set.
+// the group: its coefficients {hi, lo} in the rows whose bit is set.
 struct alignas(16) PGather {
     int j, mask;
-    double c[kPartRows][3];
+    double c[kPartRows][2];
 };
 constexpr int kPartGroups = 25 / kPartRows;
 constexpr int kPartGather = kPartRows * kPartGroups * (kPartGroups - 1) / 2 + kPartGroups;   // columns 0..K-1 of each K = 1 + g rows
-__constant__ PGather c_pg[kPartGather];
+__constant__ PGather c_pg[kPartGather + 1];
 __constant__ int c_pg0[kPartGroups + 1];
 __constant__ int c_pin[26];       // column k in the rows of its own group: bit i of row K + i
 __constant__ int c_pkeep;         // bit k: stage k is a column of a later group
 
 struct PAcc { ddv3 v; v3 a; };
-__device__ __forceinline__ void padd(PAcc &s, dd c, double fc, const ddv3 &vj, v3 aj) {
+__device__ __forceinline__ void padd(PAcc &s, dd c, const ddv3 &vj, v3 aj) {
     s.v = add(s.v, scale(c, vj));
-    s.a += fc * aj;
+    s.a += todbl(c) * aj;
 }
 
 // n_steps > 0: advance; n_steps < 0: compute the first acceleration from
@@ -2446,7 +2475,7 @@ __device__ __forceinline__ void padd(PAcc &s, dd c, double fc, const ddv3 &vj, v
 // known.  Every sum keeps its order, ascending columns.  288 B of LDS per
 // particle and up to 256 registers: two wavefronts per SIMD.  1e6 particles
 // about 4.0 -> 2.95 ms per step, 8 steps of 20k particles and a download 3.97
-// -> 3.12 ms.
+// -> 3.12 ms; with the records and coefficients loaded ahead 2.33 and 2.69 ms.
 __global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_particles(PView pv, int n_steps, double dt, DtK dtk,
                                                        const PBlock *__restrict__ blocks) {
     const int lane = (int)threadIdx.x;
@@ -2472,8 +2501,15 @@ __global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2
     ddv3 v{dd{ld(P_V + 0), ld(P_V + 1)}, dd{ld(P_V + 2), ld(P_V + 3)}, dd{ld(P_V + 4), ld(P_V + 5)}};
     double mind = ld(P_MIND), maxi = ld(P_MAXI);
     cst_jmain *rec = (cst_jmain *)pv.rec;
+    ddv3 near[kPartBatch];                                  // positions of the next evaluation's first partners
+    auto load_near = [&](cst_jmain *T) {
+#pragma unroll
+        for (int h = 0; h < kPartBatch; ++h) near[h] = part_near(T + h);
+    };
     if (init) {
-        const v3 a = particle_accel(rec + entry0 * pv.nrec_sys * kSmallMax, pv.nf, r, v, pv.sR2, mind, maxi);
+        cst_jmain *T = rec + entry0 * pv.nrec_sys * kSmallMax;
+        load_near(T);
+        const v3 a = particle_accel(T, pv.nf, near, r, v, pv.sR2, mind, maxi);
         if (valid) {
             P[(P_A + 0) * S + q] = a.x; P[(P_A + 1) * S + q] = a.y; P[(P_A + 2) * S + q] = a.z;
             P[P_MIND * S + q] = mind; P[P_MAXI * S + q] = maxi;
@@ -2516,21 +2552,23 @@ __global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2
             PAcc s[kPartRows];
 #pragma unroll
             for (int i = 0; i < kPartRows; ++i) s[i] = PAcc{mkddv(v3{0, 0, 0}), v3{0, 0, 0}};
-            auto column = [&](int e, const ddv3 &vj, v3 aj) {
-                const int mask = c_pg[e].mask;
+            auto column = [&](const PGather &q, const ddv3 &vj, v3 aj) {
 #pragma unroll
                 for (int i = 0; i < kPartRows; ++i)
-                    if (mask >> i & 1) padd(s[i], dd{c_pg[e].c[i][0], c_pg[e].c[i][1]}, c_pg[e].c[i][2], vj, aj);
+                    if (q.mask >> i & 1) padd(s[i], dd{q.c[i][0], q.c[i][1]}, vj, aj);
             };
             int e = c_pg0[g];
             const int e1 = c_pg0[g + 1];
+            PGather q = c_pg[e], qn = c_pg[e + 1];          // the column's coefficients, and the next one's (one more past the last)
             v3 sn{0, 0, 0}, an{0, 0, 0};                    // of the next column
-            if (e + 1 < e1) get_g(c_pg[e + 1].j, sn, an);
-            column(e, v0, a0);
+            if (e + 1 < e1) get_g(qn.j, sn, an);
+            column(q, v0, a0);
             for (++e; e < e1; ++e) {
                 const v3 sj = sn, aj = an;
-                if (e + 1 < e1) get_g(c_pg[e + 1].j, sn, an);
-                column(e, add(v0, mkddv(dt * sj)), aj);
+                q = qn;
+                qn = c_pg[e + 1];
+                if (e + 1 < e1) get_g(qn.j, sn, an);
+                column(q, add(v0, mkddv(dt * sj)), aj);
             }
 #pragma unroll
             for (int i = 1; i < kPartRows; ++i) put_p(i, s[i]);
@@ -2538,9 +2576,10 @@ __global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll 1
             for (int i = 0; i < kPartRows; ++i) {
                 const int k = g * kPartRows + 1 + i;
+                load_near(T);
                 r = add(r0, scale(mkdd(dt), cur.v));
                 v = add(v0, mkddv(dt * cur.a));
-                a = particle_accel(T, pv.nf, r, v, pv.sR2, mind, maxi);
+                a = particle_accel(T, pv.nf, near, r, v, pv.sR2, mind, maxi);
                 T += pv.nrec_sys * kSmallMax;
                 if (c_pkeep >> k & 1) put_g(k, cur.a, a);
                 if (i + 1 == kPartRows) break;
@@ -2550,13 +2589,13 @@ __global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2
                     const int k2 = g * kPartRows + 1 + i2;
                     const double2 c = c_rk[k2 * (k2 - 1) / 2 + k];
                     PAcc o = get_p(i2);
-                    padd(o, dd{c.x, c.y}, c.x + c.y, v, a);
+                    padd(o, dd{c.x, c.y}, v, a);
                     put_p(i2, o);
                 }
                 cur = get_p(i + 1);
                 if (mask >> (i + 1) & 1) {
                     const double2 c = c_rk[(k + 1) * k / 2 + k];
-                    padd(cur, dd{c.x, c.y}, c.x + c.y, v, a);
+                    padd(cur, dd{c.x, c.y}, v, a);
                 }
             }
         }
@@ -2662,7 +2701,7 @@ void set_rk_table(const double *tab650, hipStream_t st) {
     struct Tables {
         int nzj[325] = {}, row0[27] = {}, padj[kPadCols] = {}, pad0[27] = {};
         double padc[2 * kPadCols] = {};
-        PGather pg[kPartGather] = {};
+        PGather pg[kPartGather + 1] = {};
         int pg0[kPartGroups + 1] = {}, pin[26] = {}, pkeep = 0;
     };
     static const Tables t = [&] {
@@ -2694,7 +2733,7 @@ void set_rk_table(const double *tab650, hipStream_t st) {
                     const double *c = tab650 + 2 * ((K + i) * (K + i - 1) / 2 + j);
                     if (c[0] == 0) continue;
                     q.mask |= 1 << i;
-                    q.c[i][0] = c[0]; q.c[i][1] = c[1]; q.c[i][2] = c[0] + c[1];
+                    q.c[i][0] = c[0]; q.c[i][1] = c[1];
                 }
                 if (j >= K) t.pin[j] = q.mask;
                 else if (j == 0 || q.mask) {                // column 0, the step's start, always comes first

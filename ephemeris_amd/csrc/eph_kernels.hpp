@@ -16,6 +16,9 @@ constexpr int kSmallMax = 64;    // largest system integrated by one workgroup
 struct DtK { double v[26]; };
 
 constexpr int kPartBS = 256;     // particles per workgroup
+// slot of a stage's field records that holds, in its first two words, which
+// bodies have a quadrupole and which a spin (bit j: body j)
+constexpr int kPartMasks = kSmallMax - 1;
 constexpr int kPartLanes = 64;   // particles per wavefront: a launch's workgroups, so that few particles spread over more CUs
 // k_particles forms the stage combinations of kPartRows rows of the tableau at
 // a time; the stages that a later group reads, 1..kPartStages at most, keep

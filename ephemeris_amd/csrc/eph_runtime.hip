@@ -964,6 +964,13 @@ int field_epoch_record(Batch *field, JMain *dst) {
         t0[j].phi = pc[j];
         t0[j].nx = nc[j]; t0[j].ny = nc[field->nb + j]; t0[j].nz = nc[2 * field->nb + j];
     }
+    uint64_t masks[2] = {0, 0};
+    for (int64_t j = 0; j < field->nb; ++j) {
+        const JMain &T = t0[j];
+        for (int q = 0; q < 9; ++q) masks[0] |= (uint64_t)(T.C[q] != 0) << j;
+        masks[1] |= (uint64_t)(T.GLx != 0 || T.GLy != 0 || T.GLz != 0) << j;
+    }
+    memcpy(&t0[kPartMasks], masks, sizeof masks);
     HIP_CHECK(hipMemcpy(dst, t0.data(), sizeof(JMain) * kSmallMax, hipMemcpyHostToDevice));
     return EPH_OK;
 }

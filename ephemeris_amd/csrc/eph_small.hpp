@@ -29,6 +29,7 @@
 
 // single-thread-order systems have at most 48 bodies (min(N, ceil(N^2 / 2304)) = 1)
 constexpr int kSmallBodies = 48;
+static_assert(kSmallBodies <= kPartMasks, "the masks come after the last body's record");
 
 // fields of the LDS state, after those of the state that are kept
 enum SmallField : int {
@@ -267,7 +268,8 @@ __device__ __forceinline__ bool small_kept(int f) {
 // rings.  LDS: S_COUNT rows of NB, the stage records where NB == 16, then
 // `pairs` pairs of terms.  With `rec`, the partner data (JMain) of every body
 // after each stage's deform is recorded: entry e = 25*step + (k-1) of the
-// launch, workgroup b, body t at rec[(e*nrec_sys + b)*kSmallMax + t].
+// launch, workgroup b, body t at rec[(e*nrec_sys + b)*kSmallMax + t], and which
+// bodies have a quadrupole or a spin in entry kPartMasks.
 template <int NB, int NT, bool NP>
 __global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sys_ids, int n_steps, double dt, DtK dtk,
                                               int64_t i_step0, JMain *rec, int nrec_sys, int pairs) {
@@ -293,7 +295,19 @@ __global__ __launch_bounds__(NT) void k_small(View d, const int *__restrict__ sy
             const int b = tid - (NT - NB);
             load_jmain(S, T, b);
             const int64_t e = 25 * (int64_t)step + (k - 1);
-            rec[(e * nrec_sys + blockIdx.x) * kSmallMax + b] = T;
+            JMain *entry = rec + (e * nrec_sys + blockIdx.x) * kSmallMax;
+            entry[b] = T;
+            // bodies with a quadrupole and with a spin (the lanes are the last NB of a wavefront)
+            bool quad = false;
+#pragma unroll
+            for (int q = 0; q < 9; ++q) quad |= T.C[q] != 0;
+            const uint64_t quads = __ballot(quad) >> (64 - NB);
+            const uint64_t spins = __ballot(T.GLx != 0 || T.GLy != 0 || T.GLz != 0) >> (64 - NB);
+            if (b == 0) {
+                uint64_t *masks = (uint64_t *)(entry + kPartMasks);
+                masks[0] = quads;
+                masks[1] = spins;
+            }
         }
     };
     const int m = n - 1;                                   // pairs per body
