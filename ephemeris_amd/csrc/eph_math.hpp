@@ -104,6 +104,36 @@ EPH_HD void recip_and_root(double d, double &q, double &s) {
     s = sqrt(q);
 }
 
+// a / b and sqrt(x), correctly rounded, for operands whose exponents are so
+// moderate that the language's operations would scale nothing: the same steps
+// (two of Newton's on the reciprocal and a residual; Goldschmidt's on the root
+// and two residuals) without their scaling, 8 for 11 and 10 for 18
+// instructions.  The caller has checked the operands.
+EPH_HD double div_moderate(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(y, fma(-b, y, 1.0), y);
+    y = fma(y, fma(-b, y, 1.0), y);
+    const double q = a * y;
+    return fma(fma(-b, q, a), y, q);
+#else
+    return a / b;
+#endif
+}
+EPH_HD double sqrt_moderate(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+#else
+    return sqrt(x);
+#endif
+}
+
 // ---- vectors ----------------------------------------------------------------
 EPH_HD v3 mkv(double x, double y, double z) { return v3{x, y, z}; }
 EPH_HD v3 operator+(v3 a, v3 b) { return v3{a.x + b.x, a.y + b.y, a.z + b.z}; }
