@@ -670,8 +670,8 @@ __global__ __launch_bounds__(BS) void k_main_pool(View d, const int2 *__restrict
 // with the partners read from their rows, 25 loads for every four partners,
 // the vector memory path was busy 81% of 404 us.  Partners now come as
 // records through an LDS tile, and only the rows of terms that some pair of
-// the group has are written and added (12 to 18 of 24): 284 us, the LDS busy
-// 76% and the FP64 units 68% of it.  Four wavefronts per SIMD in place of three
+// the group has are written and added (12 to 18 of 24): 284 us, vector issue
+// on 64% and the LDS busy on 47% of the cycles.  Four wavefronts per SIMD in place of three
 // (128 registers, reached before the tile was there) did not help: 359 us
 // against 347 at that point.
 // ---------------------------------------------------------------------------
