@@ -2499,7 +2499,7 @@ __device__ __forceinline__ void padd(PAcc &s, dd c, const ddv3 &vj, v3 aj) {
 // known.  Every sum keeps its order, ascending columns.  288 B of LDS per
 // particle and up to 256 registers: two wavefronts per SIMD.  1e6 particles
 // about 4.0 -> 2.95 ms per step, 8 steps of 20k particles and a download 3.97
-// -> 3.12 ms; with the records and coefficients loaded ahead 2.17 and 2.39 ms.
+// -> 3.12 ms; with the records and coefficients loaded ahead 2.17 and 2.01 ms.
 __global__ __launch_bounds__(kPartLanes) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_particles(PView pv, int n_steps, double dt, DtK dtk,
                                                        const PBlock *__restrict__ blocks) {
     const int lane = (int)threadIdx.x;
